@@ -1204,7 +1204,8 @@ __global__ __launch_bounds__(kBlock) void k_normals(const DevScene* __restrict__
     const Chunk c = C[blockIdx.x];
     const DevScene& S = T[c.scene];
     const int i = c.begin + threadIdx.x;
-    if (i >= S.n) return;
+    // a batch may hold scenes without surface tension, which have no normals
+    if (i >= S.n || !(S.flags & F_ST)) return;
     const KCoefD k = S.kd;
     const float4 xi = ld4(S.x, i);
     const double xx = xi.x, xy = xi.y, xz = xi.z;
