@@ -581,9 +581,11 @@ int batch_one_step(sphg_ctx* ctx, Batch& B, uint32_t& syncs) {
     hipStream_t st = ctx->stream;
     const int method = B.scenes[0]->desc.method;
     const int ns = (int)B.scenes.size();
+    int sameFlags = B.scenes[0]->view[0].flags;   // -1: they differ
     int anyFlags = 0, anySt = 0, anyCube = 0, anyEmit = 0, anyPb = 0;
     for (auto* s : B.scenes) {
         anyFlags |= s->view[0].flags;
+        if (s->view[0].flags != sameFlags) sameFlags = -1;
         anySt |= (s->view[0].flags & F_ST);
         anyCube |= s->view[0].cubeOn;
         anyEmit |= s->view[0].nEmit;
@@ -602,7 +604,7 @@ int batch_one_step(sphg_ctx* ctx, Batch& B, uint32_t& syncs) {
             if (anyFlags) {
                 if (anySt) { Scope s(P, st, K_NORMALS); launch_normals(st, T, B.dP, B.nP); }
                 Scope s(P, st, K_FORCES);
-                launch_forces(st, DFSPH, T, B.dP, B.nP);
+                launch_forces(st, DFSPH, sameFlags, T, B.dP, B.nP);
             }
             { Scope s(P, st, K_DT); launch_dt(st, T, B.dP, B.nP); }
             finalize(ctx, B, T, 0);
@@ -664,7 +666,7 @@ int batch_one_step(sphg_ctx* ctx, Batch& B, uint32_t& syncs) {
             // (src/SPHSolver.cpp:123-135, src/WCSPHSolver.cpp:116-128)
             if (anyPb) { Scope s(P, st, K_PB); pbDensity(T2, 0, 0); }
             if (anySt) { Scope s(P, st, K_NORMALS); launch_normals(st, T2, B.dP, B.nP); }
-            { Scope s(P, st, K_FORCES); launch_forces(st, WCSPH, T2, B.dP, B.nP); }
+            { Scope s(P, st, K_FORCES); launch_forces(st, WCSPH, sameFlags, T2, B.dP, B.nP); }
             // cube boundary after the integration (src/WCSPHSolver.cpp:51-60),
             // or the PCISPH boundary projection (:62-73), then the emitters
             // (:75), then time += dt (:77)
@@ -687,7 +689,7 @@ int batch_one_step(sphg_ctx* ctx, Batch& B, uint32_t& syncs) {
             grid_sort(ctx, B, T);
             { Scope s(P, st, K_BUILD); launch_build(st, PCISPH, T2, B.dP, B.nP); }
             if (anySt) { Scope s(P, st, K_NORMALS); launch_normals(st, T2, B.dP, B.nP); }
-            { Scope s(P, st, K_FORCES); launch_forces(st, PCISPH, T2, B.dP, B.nP); }
+            { Scope s(P, st, K_FORCES); launch_forces(st, PCISPH, sameFlags, T2, B.dP, B.nP); }
         });
         if (rc) return rc;
         int seen = 0;

@@ -1260,7 +1260,13 @@ __device__ inline bool time_in_last_kernel(const DevScene& S) { return !(S.cubeO
 // written by k_build) because it updates x and v in place.  M = PCISPH also
 // predicts v*, x* for the first pressure iteration (pacc = 0,
 // src/PCISPHSolver.cpp:139-146).
-template <int M>
+// FL: the forces (Flags, F_ADH aside) every scene of the launch has, known at
+// compile time, or -1.  The kernel is bound by its FP64 pair math, and by how
+// many wavefronts hide its gathers: with every force compiled in it holds 166
+// to 190 registers, 2 wavefronts a SIMD, with one of XSPH and cohesion 90 to
+// 118, with both 124 to 146.  XSPH alone, WCSPH, 599,169 particles: 99.8 ->
+// 78.4 us; XSPH and cohesion, DFSPH, 35,805 particles: 30.4 -> 15 us.
+template <int M, int FL>
 __global__ __launch_bounds__(kBlock) void k_forces(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
     const Chunk c = C[blockIdx.x];
     const DevScene& S = T[c.scene];
@@ -1269,8 +1275,9 @@ __global__ __launch_bounds__(kBlock) void k_forces(const DevScene* __restrict__ 
     if (i >= S.n) return;
     const KCoefD k = S.kd;
     const double dt = S.ss->dt;
-    const bool xs = (S.flags & F_XSPH) != 0, st = (S.flags & F_ST) != 0;
-    const bool vstd = (S.flags & F_VSTD) != 0, vart = (S.flags & F_VART) != 0;
+    const int fl = FL >= 0 ? FL : S.flags;
+    const bool xs = (fl & F_XSPH) != 0, st = (fl & F_ST) != 0;
+    const bool vstd = (fl & F_VSTD) != 0, vart = (fl & F_VART) != 0;
     const bool vel = xs || vstd || vart;
     const float4 xi = (M == WCSPH) ? ld4(S.xk, i) : ld4(S.x, i);
     const float4 vi = (M == WCSPH) ? ld4(S.aux, i) : ld4(S.v, i);
@@ -2362,11 +2369,24 @@ void launch_build(hipStream_t st, int method, const DevScene* T, const Chunk* C,
     else LAUNCH(k_build<PCISPH>, n, st, T, C);
 }
 void launch_normals(hipStream_t st, const DevScene* T, const Chunk* C, int n) { if (n) LAUNCH(k_normals, n, st, T, C); }
-void launch_forces(hipStream_t st, int method, const DevScene* T, const Chunk* C, int n) {
+// The combinations of XSPH and cohesion get a kernel of their own; the two
+// viscosity forces that read rho_j as well, and batches whose scenes differ,
+// take the general one.
+template <int M>
+void launch_forces_m(hipStream_t st, int flags, const DevScene* T, const Chunk* C, int n) {
+    switch (flags < 0 ? -1 : flags & ~F_ADH) {
+        case 0: LAUNCH((k_forces<M, 0>), n, st, T, C); break;
+        case F_XSPH: LAUNCH((k_forces<M, F_XSPH>), n, st, T, C); break;
+        case F_ST: LAUNCH((k_forces<M, F_ST>), n, st, T, C); break;
+        case F_XSPH | F_ST: LAUNCH((k_forces<M, F_XSPH | F_ST>), n, st, T, C); break;
+        default: LAUNCH((k_forces<M, -1>), n, st, T, C);
+    }
+}
+void launch_forces(hipStream_t st, int method, int flags, const DevScene* T, const Chunk* C, int n) {
     if (!n) return;
-    if (method == DFSPH) LAUNCH(k_forces<DFSPH>, n, st, T, C);
-    else if (method == WCSPH) LAUNCH(k_forces<WCSPH>, n, st, T, C);
-    else LAUNCH(k_forces<PCISPH>, n, st, T, C);
+    if (method == DFSPH) launch_forces_m<DFSPH>(st, flags, T, C, n);
+    else if (method == WCSPH) launch_forces_m<WCSPH>(st, flags, T, C, n);
+    else launch_forces_m<PCISPH>(st, flags, T, C, n);
 }
 void launch_dt(hipStream_t st, const DevScene* T, const Chunk* C, int n) { if (n) LAUNCH(k_dt, n, st, T, C); }
 void launch_df_predict(hipStream_t st, const DevScene* T, const Chunk* C, int n) { if (n) LAUNCH(k_df_predict, n, st, T, C); }
@@ -2380,7 +2400,6 @@ void launch_df_err(hipStream_t st, int mode, const DevScene* T, const Chunk* C, 
     if (!n) return;
     if (mode == 0) LAUNCH(k_df_err<0>, n, st, T, C);
     else if (mode == 1) LAUNCH(k_df_err<1>, n, st, T, C);
-    else if (mode == 2) LAUNCH(k_df_err<2>, n, st, T, C);
     else LAUNCH(k_df_err<3>, n, st, T, C);
 }
 void launch_finalize(hipStream_t st, int kind, const DevScene* T, int nscenes, int* active) {
