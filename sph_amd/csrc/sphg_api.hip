@@ -4,8 +4,10 @@
 //   WCSPH  src/WCSPHSolver.cpp:14-78
 //   PCISPH src/PCISPHSolver.cpp:21-81 (loop :360-387)
 //   DFSPH  src/DFSPHSolver.cpp:38-112 (loops :311-406, :494-590)
-// The iteration loops are driven from the host here, reading one int (the
-// number of scenes still iterating) per iteration.
+// The iteration loops are driven from the host here.  A batch reads one int
+// (the number of scenes still iterating) per iteration past its prediction; a
+// lone scene's iterations are launched ahead and its steps follow each other
+// without a wait (run_lone).
 
 #include "../../include/sphg.h"
 #include "sphg_internal.h"
@@ -21,6 +23,7 @@
 #include <mutex>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 using namespace sphg;
@@ -160,6 +163,8 @@ struct Scope {
 
 }  // namespace
 
+constexpr uint32_t kRecs = 4;   // records in flight at most: a step that runs, one behind it, a check
+
 struct sphg_ctx {
     int device = 0;
     unsigned char* scratch = nullptr;   // this device's address of `scratch`
@@ -169,7 +174,9 @@ struct sphg_ctx {
     hipStream_t copyStream = nullptr;
     bool graphs = false;                // replay captured step segments (persistent batches)
     int* dActive = nullptr;   // [0] scenes still iterating, [1] largest iteration count reached
-    int* hActive = nullptr;   // pinned copy
+    // what the host waits for in a step, written by its kernels (pinned)
+    StepRec* recs = nullptr;
+    uint32_t recSeq = 0;      // number of the last record asked for
     Profiler prof;
     // the context's scenes; creating and destroying a scene that no running
     // call uses may happen on another thread than the one running the
@@ -469,23 +476,53 @@ int upload_batch_tables(sphg_ctx* ctx, Batch& B) {
     return SPHG_OK;
 }
 
+// The chunk tables of B's launches; a batch of one scene needs none.
+const Chunk* particle_chunks(const Batch& B) { return B.scenes.size() == 1 ? nullptr : B.dP; }
+const Chunk* cell_chunks(const Batch& B) { return B.scenes.size() == 1 ? nullptr : B.dC; }
+
 // Counting sort of the fluid into (cell, id) order; tables T (before) and
 // T2 (after: the other half of each double buffer is current).  Keys and
 // histogram are formed by the caller (k_keys or k_df_positions).
-void grid_sort(sphg_ctx* ctx, Batch& B, const DevScene* T) {
+void grid_sort(sphg_ctx* ctx, Batch& B, const DevScene* T, Tables tables = Tables{}, int fused = 0) {
     Profiler* P = &ctx->prof;
     hipStream_t st = ctx->stream;
     const int ns = (int)B.scenes.size();
-    { Scope s(P, st, K_SCAN); launch_scan(st, T, B.dC, B.nC, ns, B.maxCellChunks); }
-    { Scope s(P, st, K_SCATTER); launch_scatter(st, T, B.dP, B.nP); }
-    { Scope s(P, st, K_REORDER); launch_rank_reorder(st, T, B.dP, B.nP); }
+    { Scope s(P, st, K_SCAN); launch_scan(st, T, cell_chunks(B), B.nC, ns, B.maxCellChunks, tables, fused); }
+    { Scope s(P, st, K_SCATTER); launch_scatter(st, T, particle_chunks(B), B.nP); }
+    { Scope s(P, st, K_REORDER); launch_rank_reorder(st, T, particle_chunks(B), B.nP); }
+}
+
+// Waits for record `seq`.  The host polls the pinned memory (9 us from a
+// kernel's end, against 16 for a copy and a stream synchronisation), and asks
+// the stream now and then, so that a failed launch ends the wait.
+int wait_rec(sphg_ctx* ctx, uint32_t seq, StepRec& out) {
+    const StepRec* r = ctx->recs + seq % kRecs;
+    for (uint32_t spin = 1;; ++spin) {
+        if (__atomic_load_n(&r->seq, __ATOMIC_ACQUIRE) == seq) {
+            out = *r;
+            return SPHG_OK;
+        }
+        if (spin % 4096 == 0) {
+            const hipError_t q = hipStreamQuery(ctx->stream);
+            if (q == hipErrorNotReady) {
+                std::this_thread::yield();
+                continue;
+            }
+            if (q != hipSuccess) return fail(SPHG_EHIP, std::string("step: ") + hipGetErrorString(q));
+            // the stream has drained: the record is there now or never
+            if (__atomic_load_n(&r->seq, __ATOMIC_ACQUIRE) != seq) return fail(SPHG_EHIP, "a step left no outcome");
+        }
+    }
 }
 
 int read_active(sphg_ctx* ctx, int& v, int& maxIt, uint32_t& syncs) {
-    HIP_TRY(hipMemcpyAsync(ctx->hActive, ctx->dActive, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
-    v = ctx->hActive[0];
-    maxIt = ctx->hActive[1];
+    const uint32_t q = ++ctx->recSeq;
+    launch_tell_active(ctx->stream, ctx->dActive, ctx->recs + q % kRecs, q);
+    StepRec r;
+    const int rc = wait_rec(ctx, q, r);
+    if (rc) return rc;
+    v = r.done;
+    maxIt = r.it;
     ++syncs;
     return SPHG_OK;
 }
@@ -602,16 +639,16 @@ int batch_one_step(sphg_ctx* ctx, Batch& B, uint32_t& syncs) {
         const DevScene* T = B.dT[0];
         rc = run_segment(ctx, B, 0, [&] {
             if (anyFlags) {
-                if (anySt) { Scope s(P, st, K_NORMALS); launch_normals(st, T, B.dP, B.nP); }
+                if (anySt) { Scope s(P, st, K_NORMALS); launch_normals(st, T, particle_chunks(B), B.nP); }
                 Scope s(P, st, K_FORCES);
-                launch_forces(st, DFSPH, sameFlags, T, B.dP, B.nP);
+                launch_forces(st, DFSPH, sameFlags, T, particle_chunks(B), B.nP);
             }
-            { Scope s(P, st, K_DT); launch_dt(st, T, B.dP, B.nP); }
+            { Scope s(P, st, K_DT); launch_dt(st, T, particle_chunks(B), B.nP); }
             finalize(ctx, B, T, 0);
-            { Scope s(P, st, K_DFPREDICT); launch_df_predict(st, T, B.dP, B.nP); }
-            { Scope s(P, st, K_DFVEL_WARM); launch_df_vel(st, 0, T, B.dP, B.nP); }
+            { Scope s(P, st, K_DFPREDICT); launch_df_predict(st, T, particle_chunks(B), B.nP, 0); }
+            { Scope s(P, st, K_DFVEL_WARM); launch_df_vel(st, 0, T, particle_chunks(B), B.nP, 0, 0); }
             // the loop counters were cleared by the dt finalize
-            { Scope s(P, st, K_DFERR_DENS); launch_df_err(st, 0, T, B.dP, B.nP); }
+            { Scope s(P, st, K_DFERR_DENS); launch_df_err(st, 0, T, particle_chunks(B), B.nP, 0); }
             finalize(ctx, B, T, 1);
         });
         if (rc) return rc;
@@ -619,17 +656,17 @@ int batch_one_step(sphg_ctx* ctx, Batch& B, uint32_t& syncs) {
         for (int it = 0; it < B.maxIt; ++it) {
             if ((rc = loop_more(ctx, it, density_ahead(B), more, seen, syncs))) return rc;
             if (!more) break;
-            { Scope s(P, st, K_DFVEL_DENS); launch_df_vel(st, 1, T, B.dP, B.nP); }
-            { Scope s(P, st, K_DFERR_DENS); launch_df_err(st, 1, T, B.dP, B.nP); }
+            { Scope s(P, st, K_DFVEL_DENS); launch_df_vel(st, 1, T, particle_chunks(B), B.nP, it, 0); }
+            { Scope s(P, st, K_DFERR_DENS); launch_df_err(st, 1, T, particle_chunks(B), B.nP, 0); }
             finalize(ctx, B, T, 2);
         }
         B.lastIt = seen;
         const DevScene* T2 = B.dT[1];
         rc = run_segment(ctx, B, 1, [&] {
-            { Scope s(P, st, K_DFPOS); launch_df_positions(st, T, B.dP, B.nP, ctx->dActive); }
+            { Scope s(P, st, K_DFPOS); launch_df_positions(st, T, particle_chunks(B), B.nP, ctx->dActive, 0, 0); }
             // PCISPH boundary method: projection after the position update
             // (src/DFSPHSolver.cpp:65-75), which then counts the cells
-            if (anyPb) { Scope s(P, st, K_PB); launch_pb_correct(st, 0, T, B.dP, B.nP); }
+            if (anyPb) { Scope s(P, st, K_PB); launch_pb_correct(st, 0, T, particle_chunks(B), B.nP); }
             // emitters between the position update and the grid rebuild
             // (src/DFSPHSolver.cpp:77); the new particles' cells are counted
             if (anyEmit) { Scope s(P, st, K_EMIT); launch_emit(st, B.dT[0], B.dT[1], ns, 1); }
@@ -638,7 +675,7 @@ int batch_one_step(sphg_ctx* ctx, Batch& B, uint32_t& syncs) {
             // the build also forms the divergence solve's initial error,
             // kappa_v and the error partials (computeDivergenceError before
             // the loop)
-            { Scope s(P, st, K_BUILD); launch_build(st, DFSPH, T2, B.dP, B.nP); }
+            { Scope s(P, st, K_BUILD); launch_build(st, DFSPH, T2, particle_chunks(B), B.nP); }
             finalize(ctx, B, T2, 3);
         });
         if (rc) return rc;
@@ -646,32 +683,32 @@ int batch_one_step(sphg_ctx* ctx, Batch& B, uint32_t& syncs) {
         for (int it = 0; it < B.maxIt; ++it) {
             if ((rc = loop_more(ctx, it, divergence_ahead(B), more, seen, syncs))) return rc;
             if (!more) break;
-            { Scope s(P, st, K_DFVEL_DIV); launch_df_vel(st, 2, T2, B.dP, B.nP); }
-            { Scope s(P, st, K_DFERR_DIV); launch_df_err(st, 3, T2, B.dP, B.nP); }
+            { Scope s(P, st, K_DFVEL_DIV); launch_df_vel(st, 2, T2, particle_chunks(B), B.nP, it, 0); }
+            { Scope s(P, st, K_DFERR_DIV); launch_df_err(st, 3, T2, particle_chunks(B), B.nP, 0); }
             finalize(ctx, B, T2, 4);
         }
         B.lastItV = seen;
         // cube boundary after the divergence solve (src/DFSPHSolver.cpp:99-108)
-        if (anyCube) { Scope s(P, st, K_CUBE); launch_cube(st, T2, B.dP, B.nP); }
+        if (anyCube) { Scope s(P, st, K_CUBE); launch_cube(st, T2, particle_chunks(B), B.nP); }
         flip(B);
     } else if (method == WCSPH) {
         const DevScene* T = B.dT[0];
         const DevScene* T2 = B.dT[1];
         rc = run_segment(ctx, B, 0, [&] {
             // the keys kernel also starts the step (WCSPH has no loop to count)
-            { Scope s(P, st, K_KEYS); launch_keys(st, T, B.dP, B.nP, ctx->dActive); }
+            { Scope s(P, st, K_KEYS); launch_keys(st, T, particle_chunks(B), B.nP, ctx->dActive); }
             grid_sort(ctx, B, T);
-            { Scope s(P, st, K_BUILD); launch_build(st, WCSPH, T2, B.dP, B.nP); }
+            { Scope s(P, st, K_BUILD); launch_build(st, WCSPH, T2, particle_chunks(B), B.nP); }
             // PCISPH boundary method: boundary densities and pressures
             // (src/SPHSolver.cpp:123-135, src/WCSPHSolver.cpp:116-128)
             if (anyPb) { Scope s(P, st, K_PB); pbDensity(T2, 0, 0); }
-            if (anySt) { Scope s(P, st, K_NORMALS); launch_normals(st, T2, B.dP, B.nP); }
-            { Scope s(P, st, K_FORCES); launch_forces(st, WCSPH, sameFlags, T2, B.dP, B.nP); }
+            if (anySt) { Scope s(P, st, K_NORMALS); launch_normals(st, T2, particle_chunks(B), B.nP); }
+            { Scope s(P, st, K_FORCES); launch_forces(st, WCSPH, sameFlags, T2, particle_chunks(B), B.nP); }
             // cube boundary after the integration (src/WCSPHSolver.cpp:51-60),
             // or the PCISPH boundary projection (:62-73), then the emitters
             // (:75), then time += dt (:77)
-            if (anyCube) { Scope s(P, st, K_CUBE); launch_cube(st, T2, B.dP, B.nP); }
-            if (anyPb) { Scope s(P, st, K_PB); launch_pb_correct(st, 1, T2, B.dP, B.nP); }
+            if (anyCube) { Scope s(P, st, K_CUBE); launch_cube(st, T2, particle_chunks(B), B.nP); }
+            if (anyPb) { Scope s(P, st, K_PB); launch_pb_correct(st, 1, T2, particle_chunks(B), B.nP); }
             if (anyEmit) { Scope s(P, st, K_EMIT); launch_emit(st, B.dT[1], B.dT[0], ns, 0); }
             // the forces advanced the time of scenes with none of these
             if (anyCube || anyPb || anyEmit) { Scope s(P, st, K_TIME); launch_time_advance(st, T2, ns); }
@@ -685,11 +722,11 @@ int batch_one_step(sphg_ctx* ctx, Batch& B, uint32_t& syncs) {
             launch_fill_int(st, ctx->dActive, 0, 2);
             // the keys kernel also starts the step and counts the scenes
             // whose pressure loop runs
-            { Scope s(P, st, K_KEYS); launch_keys(st, T, B.dP, B.nP, ctx->dActive); }
+            { Scope s(P, st, K_KEYS); launch_keys(st, T, particle_chunks(B), B.nP, ctx->dActive); }
             grid_sort(ctx, B, T);
-            { Scope s(P, st, K_BUILD); launch_build(st, PCISPH, T2, B.dP, B.nP); }
-            if (anySt) { Scope s(P, st, K_NORMALS); launch_normals(st, T2, B.dP, B.nP); }
-            { Scope s(P, st, K_FORCES); launch_forces(st, PCISPH, sameFlags, T2, B.dP, B.nP); }
+            { Scope s(P, st, K_BUILD); launch_build(st, PCISPH, T2, particle_chunks(B), B.nP); }
+            if (anySt) { Scope s(P, st, K_NORMALS); launch_normals(st, T2, particle_chunks(B), B.nP); }
+            { Scope s(P, st, K_FORCES); launch_forces(st, PCISPH, sameFlags, T2, particle_chunks(B), B.nP); }
         });
         if (rc) return rc;
         int seen = 0;
@@ -698,27 +735,190 @@ int batch_one_step(sphg_ctx* ctx, Batch& B, uint32_t& syncs) {
             if (!more) break;
             // PCISPH boundary method: correctPredPositions after the
             // prediction (src/PCISPHSolver.cpp:370-377)
-            if (anyPb) { Scope s(P, st, K_PB); launch_pb_predcorrect(st, T2, B.dP, B.nP); }
-            { Scope s(P, st, K_PCIDENS); launch_pci_density(st, T2, B.dP, B.nP); }
+            if (anyPb) { Scope s(P, st, K_PB); launch_pb_predcorrect(st, T2, particle_chunks(B), B.nP); }
+            { Scope s(P, st, K_PCIDENS); launch_pci_density(st, T2, particle_chunks(B), B.nP, it, 0); }
             finalize(ctx, B, T2, 5);
             // boundary densities and pressures of the iteration (:151-162, :276-293)
             if (anyPb) { Scope s(P, st, K_PB); pbDensity(T2, 1, it); }
-            { Scope s(P, st, K_PCIPACC); launch_pci_pacc(st, T2, B.dP, B.nP, it); }
+            { Scope s(P, st, K_PCIPACC); launch_pci_pacc(st, T2, particle_chunks(B), B.nP, it, 0); }
         }
         B.lastIt = seen;
         rc = run_segment(ctx, B, 1, [&] {
-            { Scope s(P, st, K_PCIINT); launch_pci_integrate(st, T2, B.dP, B.nP); }
+            { Scope s(P, st, K_PCIINT); launch_pci_integrate(st, T2, particle_chunks(B), B.nP, 0, 0); }
             // cube boundary after the integration (src/PCISPHSolver.cpp:54-63),
             // or the PCISPH boundary projection (:65-76), then the emitters
             // (:78), then time += dt (:80)
-            if (anyCube) { Scope s(P, st, K_CUBE); launch_cube(st, T2, B.dP, B.nP); }
-            if (anyPb) { Scope s(P, st, K_PB); launch_pb_correct(st, 2, T2, B.dP, B.nP); }
+            if (anyCube) { Scope s(P, st, K_CUBE); launch_cube(st, T2, particle_chunks(B), B.nP); }
+            if (anyPb) { Scope s(P, st, K_PB); launch_pb_correct(st, 2, T2, particle_chunks(B), B.nP); }
             if (anyEmit) { Scope s(P, st, K_EMIT); launch_emit(st, B.dT[1], B.dT[0], ns, 0); }
             // the integration advanced the time of scenes with none of these
             if (anyCube || anyPb || anyEmit) { Scope s(P, st, K_TIME); launch_time_advance(st, T2, ns); }
         });
         if (rc) return rc;
         flip(B);
+    }
+    return SPHG_OK;
+}
+
+// ---------------------------------------------------- a lone scene's steps
+//
+// A batch's step waits for the device once or twice to learn whether its loops
+// have ended, ~14 us of idle device each time.  A lone DFSPH or PCISPH scene
+// does not wait: its loops' iterations are launched as the previous steps
+// needed them (density_ahead), the launches behind a loop return at once if it
+// has not ended (DevScene::stall), and the host reads a step's outcome from
+// pinned memory while the next step runs.  After a stall it adds iterations,
+// asking after each, and goes on from there.  Which launches run does not
+// depend on any of that, so the results are those of waiting.
+//
+// Not for scenes whose step has more launches between the loops (cube clamp,
+// PCISPH boundary, emitters).
+bool lone_scene(const Batch& B) {
+    if (B.scenes.size() != 1) return false;
+    const DevScene& V = B.scenes[0]->view[0];
+    return V.method != WCSPH && !V.pbOn && !V.cubeOn && V.nEmit == 0;
+}
+
+// One step of a lone scene, or the rest of one: from the start (from = 0),
+// or in the density (PCISPH: pressure) or divergence loop after a stall (1,
+// 2), `it` iterations of which have run.  `ask`: wait after the loops'
+// predicted iterations and add what is missing; otherwise record `seq` says
+// whether it stalled.
+int lone_step(sphg_ctx* ctx, Batch& B, int from, int it, bool ask, uint32_t seq, uint32_t& syncs) {
+    Profiler* P = &ctx->prof;
+    hipStream_t st = ctx->stream;
+    const DevScene& V = B.scenes[0]->view[0];
+    const int flags = V.flags, n = B.nP;
+    const bool st_on = (flags & F_ST) != 0;
+    const int fused = V.nChunks <= kFusedLoopChunks ? 1 : 0;
+    const DevScene *T = B.dT[0], *T2 = B.dT[1];
+    const Tables none{}, tables = ask ? Tables{} : Tables{B.dT[0], B.dT[1]};
+    int rc;
+    // launches iterations: the `ahead` predicted ones, then one at a time
+    // while the scene's record says that the loop goes on
+    auto loop = [&](int kind, int end, const DevScene* Tl, int ahead, int& reached, auto&& iterate) -> int {
+        const bool resumed = it > 0;
+        for (; it < (resumed ? it + 1 : ahead); ++it) {
+            iterate(it);
+            if (resumed) { ++it; break; }
+        }
+        while (ask) {
+            const uint32_t q = ++ctx->recSeq;
+            launch_loop_end(st, kind, end, Tl, fused, none, ctx->recs + q % kRecs, q);
+            StepRec r;
+            int e = wait_rec(ctx, q, r);
+            if (e) return e;
+            ++syncs;
+            if (r.done) {
+                reached = kind == LOOP_DIV ? r.itV : r.it;
+                break;
+            }
+            iterate(it++);
+        }
+        it = 0;
+        return SPHG_OK;
+    };
+    if (V.method == DFSPH) {
+        if (from == 0) {
+            rc = run_segment(ctx, B, 0, [&] {
+                if (flags) {
+                    if (st_on) { Scope s(P, st, K_NORMALS); launch_normals(st, T, nullptr, n); }
+                    Scope s(P, st, K_FORCES);
+                    launch_forces(st, DFSPH, flags, T, nullptr, n);
+                }
+                { Scope s(P, st, K_DT); launch_dt(st, T, nullptr, n); }
+                if (!fused) finalize(ctx, B, T, 0);
+                { Scope s(P, st, K_DFPREDICT); launch_df_predict(st, T, nullptr, n, fused); }
+                { Scope s(P, st, K_DFVEL_WARM); launch_df_vel(st, 0, T, nullptr, n, 0, fused); }
+                { Scope s(P, st, K_DFERR_DENS); launch_df_err(st, 0, T, nullptr, n, fused); }
+                if (!fused) finalize(ctx, B, T, 1);
+            });
+            if (rc) return rc;
+        }
+        if (from <= 1) {
+            rc = loop(LOOP_DENS, 0, T, density_ahead(B), B.lastIt, [&](int k) {
+                { Scope s(P, st, K_DFVEL_DENS); launch_df_vel(st, 1, T, nullptr, n, k, fused); }
+                { Scope s(P, st, K_DFERR_DENS); launch_df_err(st, 1, T, nullptr, n, fused); }
+                if (!fused) finalize(ctx, B, T, 2);
+            });
+            if (rc) return rc;
+            auto rest = [&] {
+                { Scope s(P, st, K_DFPOS); launch_df_positions(st, T, nullptr, n, ctx->dActive, fused, ask ? 0 : 1); }
+                grid_sort(ctx, B, T, tables, fused);
+                { Scope s(P, st, K_BUILD); launch_build(st, DFSPH, T2, nullptr, n, fused); }
+                if (!fused) finalize(ctx, B, T2, 3);
+            };
+            // (the captured segment is the one of steps that do not ask)
+            if (ask) rest();
+            else if ((rc = run_segment(ctx, B, 1, rest))) return rc;
+        }
+        rc = loop(LOOP_DIV, 1, T2, divergence_ahead(B), B.lastItV, [&](int k) {
+            { Scope s(P, st, K_DFVEL_DIV); launch_df_vel(st, 2, T2, nullptr, n, k, fused); }
+            { Scope s(P, st, K_DFERR_DIV); launch_df_err(st, 3, T2, nullptr, n, fused); }
+            if (!fused) finalize(ctx, B, T2, 4);
+        });
+        if (rc) return rc;
+        if (!ask) launch_loop_end(st, LOOP_DIV, 1, T2, fused, tables, ctx->recs + seq % kRecs, seq);
+    } else {
+        if (from == 0) {
+            rc = run_segment(ctx, B, 0, [&] {
+                if (!fused) launch_fill_int(st, ctx->dActive, 0, 2);
+                // the keys kernel also starts the step
+                { Scope s(P, st, K_KEYS); launch_keys(st, T, nullptr, n, ctx->dActive); }
+                grid_sort(ctx, B, T);
+                { Scope s(P, st, K_BUILD); launch_build(st, PCISPH, T2, nullptr, n); }
+                if (st_on) { Scope s(P, st, K_NORMALS); launch_normals(st, T2, nullptr, n); }
+                { Scope s(P, st, K_FORCES); launch_forces(st, PCISPH, flags, T2, nullptr, n); }
+            });
+            if (rc) return rc;
+        }
+        rc = loop(LOOP_PCI, 0, T2, density_ahead(B), B.lastIt, [&](int k) {
+            { Scope s(P, st, K_PCIDENS); launch_pci_density(st, T2, nullptr, n, k, fused); }
+            if (!fused) finalize(ctx, B, T2, 5);
+            { Scope s(P, st, K_PCIPACC); launch_pci_pacc(st, T2, nullptr, n, k, fused); }
+        });
+        if (rc) return rc;
+        { Scope s(P, st, K_PCIINT); launch_pci_integrate(st, T2, nullptr, n, fused, ask ? 0 : 1); }
+        if (!ask) launch_loop_end(st, LOOP_PCI, 1, T2, fused, tables, ctx->recs + seq % kRecs, seq);
+    }
+    flip(B);
+    return SPHG_OK;
+}
+
+int run_lone(sphg_ctx* ctx, Batch& B, uint32_t nsteps, uint32_t& syncs) {
+    uint32_t queued = 0, done = 0;   // steps launched, steps whose outcome is known
+    uint32_t seqs[2] = {0, 0};
+    int rc;
+    while (done < nsteps) {
+        // without a count to predict from, and while single launches are
+        // timed (no launch then runs twice), the step asks
+        if (queued == done && (B.lastIt == 0 || ctx->prof.on)) {
+            if ((rc = lone_step(ctx, B, 0, 0, true, 0, syncs))) return rc;
+            ++queued;
+            ++done;
+            continue;
+        }
+        // one step waits behind the one that runs
+        while (queued < nsteps && queued - done < 2) {
+            const uint32_t q = seqs[queued & 1] = ++ctx->recSeq;
+            if ((rc = lone_step(ctx, B, 0, 0, false, q, syncs))) return rc;
+            ++queued;
+        }
+        StepRec r;
+        if ((rc = wait_rec(ctx, seqs[done & 1], r))) return rc;
+        if (r.stall) {
+            // back to the stalled step's tables: the launches behind it, which
+            // return at once, have flipped them
+            if ((queued - done) & 1) flip(B);
+            queued = done;
+            launch_clear_stall(ctx->stream, Tables{B.dT[0], B.dT[1]});
+            if ((rc = lone_step(ctx, B, r.stall, r.stall == 2 ? r.itV : r.it, true, 0, syncs))) return rc;
+            ++queued;
+        } else {
+            B.lastIt = r.it;
+            B.lastItV = r.itV;
+        }
+        ++done;
     }
     return SPHG_OK;
 }
@@ -743,8 +943,9 @@ int run_batch(sphg_ctx* ctx, Batch& B, uint32_t nsteps, sphg_step_stats* stats, 
     launch_clear_overflow(st, B.dT[0], (int)B.scenes.size());
     const auto h0 = std::chrono::steady_clock::now();
     if (events) HIP_TRY(hipEventRecord(e0, st));
-    for (uint32_t k = 0; k < nsteps; ++k) {
-        int rc = batch_one_step(ctx, B, syncs);
+    const bool lone = lone_scene(B);
+    for (uint32_t k = 0; k < (lone ? 1u : nsteps); ++k) {
+        int rc = lone ? run_lone(ctx, B, nsteps, syncs) : batch_one_step(ctx, B, syncs);
         if (rc) {
             if (e0) (void)hipEventDestroy(e0);
             if (e1) (void)hipEventDestroy(e1);
@@ -1106,7 +1307,8 @@ int sphg_ctx_create(int32_t device, sphg_ctx** out) {
         }
     }
     if (e == hipSuccess) e = hipMalloc(&c->dActive, 2 * sizeof(int));
-    if (e == hipSuccess) e = hipHostMalloc(&c->hActive, 2 * sizeof(int), hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc(&c->recs, kRecs * sizeof(StepRec), hipHostMallocDefault);
+    if (e == hipSuccess) std::memset((void*)c->recs, 0, kRecs * sizeof(StepRec));
     if (e != hipSuccess) {
         const std::string msg = std::string("context set-up: ") + hipGetErrorString(e);
         (void)sphg_ctx_destroy(c);   // releases the streams and buffers made so far
@@ -1136,7 +1338,7 @@ int sphg_ctx_destroy(sphg_ctx* ctx) {
     }
     ctx->prof.collect();
     if (ctx->dActive) (void)hipFree(ctx->dActive);
-    if (ctx->hActive) (void)hipHostFree(ctx->hActive);
+    if (ctx->recs) (void)hipHostFree(ctx->recs);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     if (ctx->copyStream) (void)hipStreamDestroy(ctx->copyStream);
     delete ctx;
@@ -1532,9 +1734,9 @@ int sphg_scene_init(sphg_scene* s) {
     if (method == DFSPH) {
         // DFSPHSolver::init: insert, neighborhoodSearch, densities, alpha
         Batch& B = *s->self;
-        launch_keys(ctx->stream, B.dT[0], B.dP, B.nP);
+        launch_keys(ctx->stream, B.dT[0], particle_chunks(B), B.nP);
         grid_sort(ctx, B, B.dT[0]);
-        launch_build(ctx->stream, DFSPH, B.dT[1], B.dP, B.nP);
+        launch_build(ctx->stream, DFSPH, B.dT[1], particle_chunks(B), B.nP);
         flip(B);
     }
     HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -1574,9 +1776,9 @@ int sphg_scene_set_state(sphg_scene* s, const float* xyz, const float* vel, cons
     s->stepped = false;
     HIP_TRY(hipMemcpyAsync(s->ss, &ss, sizeof(Scalars), hipMemcpyHostToDevice, ctx->stream));
     if (s->desc.method == DFSPH) {
-        launch_keys(ctx->stream, B.dT[0], B.dP, B.nP);
+        launch_keys(ctx->stream, B.dT[0], particle_chunks(B), B.nP);
         grid_sort(ctx, B, B.dT[0]);
-        launch_build(ctx->stream, DFSPH, B.dT[1], B.dP, B.nP);
+        launch_build(ctx->stream, DFSPH, B.dT[1], particle_chunks(B), B.nP);
         flip(B);
     }
     HIP_TRY(hipStreamSynchronize(ctx->stream));

@@ -5,7 +5,8 @@
 // own constraint, src/Simulation.h:24-29 and src/AkinciBoundayModel.cpp:32).
 // Every kernel walks a chunk table: each 256-thread block owns one chunk of
 // one scene, so a launch covers any number of scenes of uneven size
-// (batching) and a single scene is a batch of one.
+// (batching).  A launch over one scene needs no table: its blocks' chunks
+// follow from their numbers.
 //
 // HBM layout per scene (FP32, struct-of-arrays, particles sorted by
 // (cell, id) every step):
@@ -99,6 +100,18 @@ struct Scalars {
     unsigned d0Valid;           // DFSPH: d0 holds the divergence of the current velocities (written by
                                 // the list build and the divergence error sweeps; cleared by the cube
                                 // clamp, which changes the velocities after them)
+    double dtNew;               // DFSPH, loops decided in the sweeps: the step's dt between the kernel
+                                // that forms it and the one that makes it dt
+};
+
+// What the host learns of a step, in pinned memory that it polls; seq is
+// written last.
+struct StepRec {
+    unsigned seq;
+    int it, itV;                // iterations of the step's loops
+    int done;                   // the loop asked about has ended
+    int stall;                  // 1 the density (PCISPH: pressure) loop, 2 the divergence loop had not
+                                // ended after the iterations launched: nothing launched later ran
 };
 
 // One emitter's constants and state (src/Emitter.h:9-55).  Its group's
@@ -137,7 +150,9 @@ struct DevScene {
     int nx, ny, nz, ncells;     // padded grid (one empty layer on every side)
     int n, nb, maxNbr, nChunks;
     int nCellChunks, cap;       // cap: particle slots (active + every emitter's remaining budget)
-    int nEmit, pad3;
+    int nEmit;
+    int stall;                  // not 0: a loop of this step needs more iterations than were launched, and
+                                // the launches behind it return at once until the host has added them
     EmitterDev *emit;
     const double *emitGroup;
     // PCISPH boundary method (src/PCISPHBoundaryModel.h:10-52): boundary

@@ -1,38 +1,62 @@
 // sphg_kernels.h -- host-side launchers of the kernels in sphg_kernels.hip.
-// Each takes the scene table and chunk table of one batch launch.
+// Each takes the scene table and chunk table of one batch launch; a null
+// chunk table is a launch over all chunks of scene 0.
 #pragma once
 
 #include "sphg_internal.h"
 
 namespace sphg {
 
+// The two tables (before and after the step's sort) of a lone scene, for the
+// kernels that write its stall flag; null pointers: a launch that does not
+struct Tables {
+    DevScene *a = nullptr, *b = nullptr;
+};
+// the solvers' loops: DFSPH density and divergence, PCISPH pressure
+enum LoopKind { LOOP_DENS, LOOP_DIV, LOOP_PCI };
+// A lone scene of up to kFusedLoopChunks chunks has its loops decided in the
+// sweeps themselves (`fused`), each block adding up the chunk partials; above
+// that the partials are too many for every block, and finalize kernels do it.
+constexpr int kFusedLoopChunks = 2048;
+
 // begin_active: also the start of a WCSPH or PCISPH step, counting the
 // scenes whose pressure loop runs in begin_active[0] (null: keys only)
 void launch_keys(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int* begin_active = nullptr);
 // maxChunks: the largest cell-chunk count of one scene; up to
 // kScanFusedChunks each final-scan block sums the totals before its chunk
-// itself (one launch fewer), above it a per-scene scan of the totals runs
+// itself (one launch fewer), above it a per-scene scan of the totals runs; up
+// to kScanOneChunks the counts are scanned in one launch.  tables, fused: a
+// lone DFSPH scene whose density iterations were launched ahead (k_df_positions)
+constexpr int kScanOneChunks = 32;
 constexpr int kScanFusedChunks = 1024;
-void launch_scan(hipStream_t st, const DevScene* T, const Chunk* CC, int ncellchunks, int nscenes, int maxChunks);
+void launch_scan(hipStream_t st, const DevScene* T, const Chunk* CC, int ncellchunks, int nscenes, int maxChunks,
+                 Tables tables = Tables{}, int fused = 0);
 void launch_scatter(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks);
 void launch_rank_reorder(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks);
 void launch_bvolume(hipStream_t st, const DevScene* T, int scene, int nb, float* tmp);
-void launch_build(hipStream_t st, int method, const DevScene* T, const Chunk* C, int nchunks);
+void launch_build(hipStream_t st, int method, const DevScene* T, const Chunk* C, int nchunks, int fused = 0);
 void launch_normals(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks);
 // flags: the non-pressure forces (Flags) of every scene of the launch, or -1
 // where they differ
 void launch_forces(hipStream_t st, int method, int flags, const DevScene* T, const Chunk* C, int nchunks);
 void launch_dt(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks);
-void launch_df_predict(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks);
-void launch_df_vel(hipStream_t st, int mode, const DevScene* T, const Chunk* C, int nchunks);
-void launch_df_err(hipStream_t st, int mode, const DevScene* T, const Chunk* C, int nchunks);
+void launch_df_predict(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int fused);
+// iter: the number of the loop iteration (mode 1, 2)
+void launch_df_vel(hipStream_t st, int mode, const DevScene* T, const Chunk* C, int nchunks, int iter, int fused);
+void launch_df_err(hipStream_t st, int mode, const DevScene* T, const Chunk* C, int nchunks, int fused);
 // kind: 0 dt, 1 density (before loop), 2 density, 3 divergence (before loop), 4 divergence, 5 PCISPH
 void launch_finalize(hipStream_t st, int kind, const DevScene* T, int nscenes, int* active);
 // also clears active[0..1] for the divergence solve
-void launch_df_positions(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int* active);
-void launch_pci_density(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks);
-void launch_pci_pacc(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int iter);
-void launch_pci_integrate(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks);
+void launch_df_positions(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int* active, int fused,
+                         int ahead);
+void launch_pci_density(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int iter, int fused);
+void launch_pci_pacc(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int iter, int fused);
+void launch_pci_integrate(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int fused, int ahead);
+// loop: LoopKind; end: the end of a step
+void launch_loop_end(hipStream_t st, int loop, int end, const DevScene* T, int fused, Tables tables, StepRec* rec,
+                     unsigned seq);
+void launch_tell_active(hipStream_t st, const int* active, StepRec* rec, unsigned seq);
+void launch_clear_stall(hipStream_t st, Tables tables);
 void launch_cube(hipStream_t st, const DevScene* T, const Chunk* C, int n);
 void launch_emit(hipStream_t st, DevScene* Tc, DevScene* To, int nscenes, int cells);
 // PCISPH boundary method

@@ -73,6 +73,19 @@ template <class T> __device__ inline void stg(T* p, uint32_t i, T v) {
 }
 
 
+// The block's chunk: entry blockIdx.x of the chunk table, or, for a launch
+// over one scene (no table), chunk number times `unit`.  Blocks go round-robin
+// to the 8 XCDs, and XCD x gets the x-th contiguous part of the chunks, as the
+// tables have it.  Without the table a block's first load is its scene's
+// entry, not the chunk and then the scene: one memory round trip (0.5-0.8 us)
+// less in each of a small step's launches.
+__device__ inline Chunk chunk_at(const Chunk* C, int unit) {
+    const int b = blockIdx.x;
+    if (C) return C[b];
+    const int x = b & 7, per = gridDim.x >> 3, more = gridDim.x & 7;
+    return Chunk{0, (x * per + min(x, more) + (b >> 3)) * unit};
+}
+
 __device__ inline double wave_sum(double v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
@@ -135,6 +148,72 @@ __device__ inline double scene_partial_max(const double* partial, int n, double*
         for (int u = 0; u < kPartU; ++u) acc = fmax(acc, v[u]);
     }
     return block_max(acc, sh);
+}
+
+// ------------------------------------------------ loop control
+//
+// A solver loop goes on while (err > eta or it < minIt) and it < maxIt, where
+// err is the scene's reduction over the last error sweep's chunk partials.
+// For a lone scene of at most kFusedLoopChunks chunks every block of the next
+// sweep forms that reduction itself, in the order k_finalize has, and decides:
+// a launch less per iteration (~3 us), and no wait of the host (run_lone): a
+// DFSPH step of 4,096 particles 197 -> 148 us, of 262,144 346 -> 309.  With
+// 3,907 chunks (1M particles) a block would read 31 KB of partials, about what
+// the finalize launch costs, so above the limit that stays.  The block
+// that holds the scene's first chunk writes the outcome: done = idx + 1, where
+// idx grows from launch to launch.  A launch takes only the ends that earlier
+// launches wrote (ended_before) and forms its own decision otherwise, so all
+// wavefronts of a block take the same branch, whenever they read the flag.
+
+// The decision after `it` iterations with error err; SUM: of an average.
+template <int KIND>
+__device__ inline bool loop_goes_on(const DevScene& S, const Scalars* ss, int it, double err) {
+    const double eta = KIND == LOOP_DIV ? S.etaV / ss->dt : S.eta;
+    return ((err > eta) || (it < (KIND == LOOP_DIV ? S.minItV : S.minIt))) && (it < S.maxIt);
+}
+// Records the end of a loop (one thread).
+template <int KIND>
+__device__ inline void loop_ended(Scalars* ss, int it, double err, int idx) {
+    if (KIND == LOOP_DENS) { ss->avgErr = err; ss->done = idx + 1; ss->sumIt += (unsigned)it; }
+    if (KIND == LOOP_DIV) { ss->avgErrV = err; ss->doneV = idx + 1; ss->sumItV += (unsigned)it; }
+    if (KIND == LOOP_PCI) { ss->maxDensErr = err; ss->done = idx + 1; ss->sumIt += (unsigned)it; }
+}
+__device__ inline bool ended_before(int done, int idx) { return done != 0 && done <= idx; }
+constexpr int kLoopLast = 1 << 30;   // idx of the launches behind a loop
+// The PCISPH loop's partials of iteration `it`: two buffers in turn, because
+// its density sweep decides and writes partials in one launch.  The second is
+// the sort's scratch, which the loop does not need.
+__device__ inline double* pci_partial(const DevScene& S, int it) { return (it & 1) ? (double*)S.perm : S.partial; }
+// Whether the loop has ended, decided by every block alike (block-uniform;
+// called where ended_before(done, idx) is false).
+template <int KIND>
+__device__ inline bool loop_over(const DevScene& S, Scalars* ss, bool firstChunk, int idx, double* sh) {
+    const int it = KIND == LOOP_DIV ? ss->itV : ss->it;
+    // below the minimum the error does not matter
+    if (it < (KIND == LOOP_DIV ? S.minItV : S.minIt) && it < S.maxIt) return false;
+    const double err = KIND == LOOP_PCI ? scene_partial_max(pci_partial(S, it - 1), S.nChunks, sh)
+                                        : scene_partial_sum(S.partial, S.nChunks, sh) / (double)S.n;
+    if (loop_goes_on<KIND>(S, ss, it, err)) return false;
+    if (firstChunk && threadIdx.x == 0) loop_ended<KIND>(ss, it, err, idx);
+    return true;
+}
+
+// CFL time step (src/DFSPHSolver.cpp:827-870) from the scene's largest
+// sqrt(|v + (a + g) dt|).
+struct NextDt {
+    double dt, maxVel, cflTs;
+};
+__device__ inline NextDt next_dt(const DevScene& S, double ts, int it, double red) {
+    NextDt o;
+    o.maxVel = fmax(0.1, red);
+    o.cflTs = S.cfl * 0.4 * 2.0 * S.r / o.maxVel;
+    double nts;
+    if (o.cflTs < ts) nts = o.cflTs;
+    else if (it > 3) nts = ts * 0.99;
+    else nts = ts * 1.001;
+    nts = fmax(nts, S.dtMin);
+    o.dt = fmin(nts, S.dtMax);
+    return o;
 }
 
 // ------------------------------------------------ SPH kernels (FP64 math)
@@ -471,13 +550,15 @@ __device__ inline bool pb_velocity(const DevScene& S, double nx, double ny, doub
 // ================================================================ grid
 
 // Cell key + histogram (src/HashTable.h:79-86 insertion, as a count).
-// Adds one to counter[key] for every lane with key >= 0 and returns the
-// counter's value before this lane's unit, a slot unique to the lane.  The
+// Adds SIGN = 1 to counter[key] for every lane with key >= 0 and returns the
+// counter's value before this lane's unit, a slot unique to the lane; SIGN =
+// -1 takes one away and returns the value after it.  The
 // particles of a wavefront are in the previous step's cell order and most
 // keep their cell, so runs of consecutive lanes share a key: each run adds
 // its length with one atomic (a dense fluid has ~8 lanes per run), and its
 // lanes take consecutive slots.  Every lane of the wavefront calls it; lanes
 // with nothing to count pass -1 and must all come after the counting ones.
+template <int SIGN = 1>
 __device__ inline int wave_count_add(int* counter, int key) {
     const int lane = threadIdx.x & 63;
     const int prev = __shfl_up(key, 1);
@@ -488,8 +569,11 @@ __device__ inline int wave_count_add(int* counter, int key) {
     const uint64_t later = heads & ~upto;
     const int end = later ? __ffsll((long long)later) - 1 : 64;             // one past the run
     int base = 0;
-    if (head && key >= 0)
-        base = __hip_atomic_fetch_add(G(counter) + key, end - lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (head && key >= 0) {
+        const int len = end - lane;
+        base = __hip_atomic_fetch_add(G(counter) + key, SIGN * len, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (SIGN < 0) base -= len;
+    }
     base = __shfl(base, first);
     return base + (lane - first);
 }
@@ -523,8 +607,9 @@ __device__ inline void step_begin(const DevScene& S, const Chunk& c, int i, int*
 template <bool BEGIN>
 __global__ __launch_bounds__(kBlock) void k_keys(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
                                                  int* active) {
-    const Chunk c = C[blockIdx.x];
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
+    if (S.stall) return;
     const int i = c.begin + threadIdx.x;
     if (BEGIN) step_begin(S, c, i, active);
     // the lists about to be built start without an overflow
@@ -537,10 +622,32 @@ __global__ __launch_bounds__(kBlock) void k_keys(const DevScene* __restrict__ T,
     (void)wave_count_add(S.cellCount, cl);
 }
 
+// DFSPH with the loops decided in the sweeps: the error before the density
+// loop, for the log, from the partials its sweep left in the sort's scratch
+// (one block, before the scatter overwrites them).
+__device__ inline void density_error0(const DevScene& S) {
+    __shared__ double sh[kWaves];
+    const double avg0 = scene_partial_sum((const double*)S.perm, S.nChunks, sh) / (double)S.n;
+    if (threadIdx.x == 0) S.ss->avgErr0 = avg0;
+}
+// The first launch behind a DFSPH density loop whose end the position update
+// has decided (`tables` not null: a lone scene whose iterations were launched
+// ahead): whether it had ended.  If not, nothing behind this launch runs.
+__device__ inline bool sort_runs(const DevScene& S, const Chunk& c, const Tables& tables, int fused) {
+    if (tables.a && !S.ss->done) {
+        if (c.begin == 0 && threadIdx.x == 0) tables.a->stall = tables.b->stall = 1;
+        return false;
+    }
+    if (fused && c.begin == 0) density_error0(S);
+    return true;
+}
+
 // Per cell chunk: total count.
-__global__ __launch_bounds__(kBlock) void k_scan_sum(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+__global__ __launch_bounds__(kBlock) void k_scan_sum(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                     Tables tables, int fused) {
+    const Chunk c = chunk_at(C, kCellChunk);
     const DevScene& S = T[c.scene];
+    if (S.stall || !sort_runs(S, c, tables, fused)) return;
     __shared__ double sh[kWaves];
     int acc = 0;
     const int c0 = c.begin + threadIdx.x * kCellPerThread;
@@ -569,6 +676,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_offsets(const DevScene* __restr
     const int s = blockIdx.x;
     if (s >= nscenes) return;
     const DevScene& S = T[s];
+    if (S.stall) return;
     __shared__ int wsum[kWaves];
     __shared__ int carry;
     if (threadIdx.x == 0) carry = 0;
@@ -590,20 +698,41 @@ __global__ __launch_bounds__(kBlock) void k_scan_offsets(const DevScene* __restr
     }
 }
 
-// Final scan: cellStart[c] = exclusive prefix of counts; counts reset.
-// FUSED: the chunk totals are still the raw ones (no k_scan_offsets ran),
-// and the block adds up those before its chunk itself; integer sums, so
-// either way gives the same offsets.
-template <bool FUSED>
-__global__ __launch_bounds__(kBlock) void k_scan_final(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+// Final scan: cellStart[c] = exclusive prefix of counts.  What comes before
+// the block's chunk:
+//   SCAN_ONE     the counts themselves, added up by the block (no other launch
+//                of the scan runs): grids of up to kScanOneChunks chunks, where
+//                the last block reads 31 K counts in ~2 us and a launch costs
+//                ~3 (2k-particle WCSPH step 84.2 -> 82.7 us)
+//   SCAN_TOTALS  the chunk totals of k_scan_sum, added up by the block
+//   SCAN_OFFSETS the chunk offsets of k_scan_offsets
+// Integer sums, so all give the same offsets.
+enum ScanKind { SCAN_ONE, SCAN_TOTALS, SCAN_OFFSETS };
+template <int KIND>
+__global__ __launch_bounds__(kBlock) void k_scan_final(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                       Tables tables, int fused) {
+    const Chunk c = chunk_at(C, kCellChunk);
     const DevScene& S = T[c.scene];
+    if (S.stall || !sort_runs(S, c, tables, fused)) return;
     __shared__ int wsum[kWaves];
     __shared__ int base;
     const int chunk = c.begin / kCellChunk;
-    if (FUSED) {
+    if (KIND != SCAN_OFFSETS) {
         int acc = 0;
-        for (int t = threadIdx.x; t < chunk; t += kBlock) acc += ldg(S.cellChunkSum, (size_t)t);
+        if (KIND == SCAN_ONE) {
+            constexpr int kU = 8;
+            typedef int v4i __attribute__((ext_vector_type(4)));
+            const gptr<const v4i> cnt = (gptr<const v4i>)S.cellCount;
+            for (int t = threadIdx.x; t < c.begin / 4; t += kBlock * kU) {
+                v4i q[kU];
+#pragma unroll
+                for (int u = 0; u < kU; ++u) q[u] = (t + u * kBlock < c.begin / 4) ? cnt[t + u * kBlock] : (v4i)0;
+#pragma unroll
+                for (int u = 0; u < kU; ++u) acc += q[u].x + q[u].y + q[u].z + q[u].w;
+            }
+        } else {
+            for (int t = threadIdx.x; t < chunk; t += kBlock) acc += ldg(S.cellChunkSum, (size_t)t);
+        }
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o);
         if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = acc;
@@ -631,27 +760,26 @@ __global__ __launch_bounds__(kBlock) void k_scan_final(const DevScene* __restric
     __syncthreads();
     int woff = 0;
     for (int q = 0; q < w; ++q) woff += wsum[q];
-    int run = (FUSED ? base : ldg(S.cellChunkSum, (size_t)chunk)) + woff + incl - local;
+    int run = (KIND != SCAN_OFFSETS ? base : ldg(S.cellChunkSum, (size_t)chunk)) + woff + incl - local;
 #pragma unroll
     for (int u = 0; u < kCellPerThread; ++u) {
         const int cc = c0 + u;
-        if (cc < S.ncells) {
-            G(S.cellStart)[cc] = run;
-            G(S.cellCount)[cc] = 0;
-        }
+        if (cc < S.ncells) G(S.cellStart)[cc] = run;
         run += vals[u];
     }
     // the chunk table covers ncells + 1 entries: the last one is the end
     if (c0 <= S.ncells && S.ncells < c0 + kCellPerThread) G(S.cellStart)[S.ncells] = S.n;
 }
 
-// Scatter the particle ids into their cells' slots (arrival order).
+// Scatter the particle ids into their cells' slots (arrival order).  Each
+// cell's count goes back to zero for the next step's.
 __global__ __launch_bounds__(kBlock) void k_scatter(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
+    if (S.stall) return;
     const int i = c.begin + threadIdx.x;
     const int cl = (i < S.n) ? ldg(S.cellU, (size_t)i) : -1;
-    const int r = wave_count_add(S.cellCount, cl);
+    const int r = wave_count_add<-1>(S.cellCount, cl);
     if (i < S.n) G(S.perm)[ldg(S.cellStart, (size_t)cl) + r] = ldg(S.id, (size_t)i);
 }
 
@@ -659,11 +787,11 @@ __global__ __launch_bounds__(kBlock) void k_scatter(const DevScene* __restrict__
 // cell with a smaller id, so every bucket lists its particles in ascending
 // id, the reference's insertion order (src/SPHSolver.cpp:188-191,
 // src/HashTable.h:79-86).  The state is written straight to that slot (the
-// other half of each double buffer); the cell counters are reset for the
-// next step.
+// other half of each double buffer).
 __global__ __launch_bounds__(kBlock) void k_rank_reorder(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
+    if (S.stall) return;
     const int i = c.begin + threadIdx.x;
     if (i >= S.n) return;
     const int cl = ldg(S.cellU, (size_t)i);
@@ -696,7 +824,6 @@ __global__ __launch_bounds__(kBlock) void k_rank_reorder(const DevScene* __restr
         if (S.pbOn) st4(S.pbn2, (size_t)d, no);
     }
     if (S.pbOn) stg(S.everOcc, (size_t)cl, (uint8_t)1);
-    stg(S.cellCount, (size_t)cl, 0);
 }
 
 // =========================================================== boundary
@@ -764,9 +891,11 @@ constexpr int kWaveStage = SPHG_BUILD_STAGE ? 816 : 1;   // candidates per wavef
 constexpr int kWaveStagePad = kWaveStage + 3;
 
 template <int M>
-__global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+__global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                  int fused) {
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
+    if (S.stall) return;
     __shared__ float2 sxy[kBlock / 64][kWaveStagePad];
     __shared__ float sz[kBlock / 64][kWaveStagePad];
     const int i = c.begin + threadIdx.x;
@@ -1191,8 +1320,19 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
     if (M == DFSPH) {
         __shared__ double sh[kWaves];
         const double bs = block_sum(e, sh);
-        if (threadIdx.x == 0) S.partial[c.begin / kBlock] = bs;
-        if (c.begin == 0 && threadIdx.x == 0) S.ss->d0Valid = 1u;
+        // `fused`: the step's time and the start of the divergence loop are
+        // written here, and the error before the loop (for the log) waits in
+        // the sort's scratch for the step's end
+        if (threadIdx.x == 0) (fused ? (double*)S.perm : S.partial)[c.begin / kBlock] = bs;
+        if (c.begin == 0 && threadIdx.x == 0) {
+            Scalars* const ss = S.ss;
+            ss->d0Valid = 1u;
+            if (fused) {
+                ss->itV = 0;
+                ss->time += ss->dt;
+                ss->doneV = loop_goes_on<LOOP_DIV>(S, ss, 0, 0.0) ? 0 : 1;
+            }
+        }
     }
 }
 
@@ -1201,8 +1341,9 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
 // Akinci surface normals n_i = h sum_j (m/rho_j) gradW_ij
 // (src/SurfaceTensionAkinci.h:46-61).  nrm.w carries rho_i - rho0 for pass 2.
 __global__ __launch_bounds__(kBlock) void k_normals(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
+    if (S.stall) return;
     const int i = c.begin + threadIdx.x;
     // a batch may hold scenes without surface tension, which have no normals
     if (i >= S.n || !(S.flags & F_ST)) return;
@@ -1268,8 +1409,9 @@ __device__ inline bool time_in_last_kernel(const DevScene& S) { return !(S.cubeO
 // 78.4 us; XSPH and cohesion, DFSPH, 35,805 particles: 30.4 -> 15 us.
 template <int M, int FL>
 __global__ __launch_bounds__(kBlock) void k_forces(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
+    if (S.stall) return;
     const int i = c.begin + threadIdx.x;
     if ((M == WCSPH) && c.begin == 0 && threadIdx.x == 0 && time_in_last_kernel(S)) advance_time(S);
     if (i >= S.n) return;
@@ -1442,8 +1584,9 @@ __global__ __launch_bounds__(kBlock) void k_forces(const DevScene* __restrict__ 
 // sqrt(|v_i + (a_i + g) dt|)); dt' = cfl if cfl < dt, else 0.99 dt after
 // more than 3 density iterations, else 1.001 dt; clamped to [min, max].
 __global__ __launch_bounds__(kBlock) void k_dt(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
+    if (S.stall) return;
     const gptr<const Scalars> ss = G((const Scalars*)S.ss);
     __shared__ double sh[kWaves];
     const int i = c.begin + threadIdx.x;
@@ -1484,12 +1627,27 @@ __device__ inline void store_u(const DevScene& S, int i, double ux, double uy, d
 // in xk.w for the warm-start sweep.  The predicted velocity is kept as
 // u = (a + g) dt beside v0 (and, with the PCISPH boundary method, the change
 // of its velocity correction).
-__global__ __launch_bounds__(kBlock) void k_df_predict(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+// `fused`: the time step from k_dt's partials is formed here, by every block.
+__global__ __launch_bounds__(kBlock) void k_df_predict(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                       int fused) {
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
+    if (S.stall) return;
+    __shared__ double sh[kWaves];
     const int i = c.begin + threadIdx.x;
+    double dt = G(S.ss)->dt;
+    if (fused) {
+        const NextDt d = next_dt(S, dt, G(S.ss)->it, scene_partial_max(S.partial, S.nChunks, sh));
+        dt = d.dt;
+        if (c.begin == 0 && threadIdx.x == 0) {
+            const gptr<Scalars> ss = G(S.ss);
+            ss->dtNew = d.dt;
+            ss->maxVel = d.maxVel;
+            ss->cflTs = d.cflTs;
+            ss->steps += 1u;
+        }
+    }
     if (i >= S.n) return;
-    const double dt = G(S.ss)->dt;
     const float4 v = ld4(S.v, (size_t)i);
     double ax = S.gx, ay = S.gy, az = S.gz;
     if (S.flags & F_FORCES) {
@@ -1524,18 +1682,35 @@ __global__ __launch_bounds__(kBlock) void k_df_predict(const DevScene* __restric
 // with s = xk.w, c = 2 for the warm start, 1 otherwise.  MODE 0 = warm start
 // (then k_i = 0, :679-689), 1 = density (k_i += (rho*_i - rho0) alpha_i,
 // :349), 2 = divergence (kv_i += divErr_i alpha_i, :534).
+// `fused`: the sweep decides whether its iteration runs (loop_over); the warm
+// start makes the new time step dt and starts the density loop.
 template <int MODE>
-__global__ __launch_bounds__(kBlock) void k_df_vel(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+__global__ __launch_bounds__(kBlock) void k_df_vel(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                   int iter, int fused) {
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
-    const Scalars* ss = S.ss;
-    if (MODE == 1 && ss->done) return;
-    if (MODE == 2 && ss->doneV) return;
+    if (S.stall) return;
+    Scalars* ss = S.ss;
+    if (MODE == 1 && ended_before(ss->done, iter + 1)) return;
+    if (MODE == 2 && ended_before(ss->doneV, iter + 1)) return;
     const int i = c.begin + threadIdx.x;
+    double dt = ss->dt;
+    if (fused) {
+        if (MODE == 0) {
+            dt = ss->dtNew;
+            if (c.begin == 0 && threadIdx.x == 0) {
+                ss->dt = dt;
+                ss->it = 0;
+                ss->done = loop_goes_on<LOOP_DENS>(S, ss, 0, 0.0) ? 0 : 1;
+            }
+        } else {
+            __shared__ double sh[kWaves];
+            if (loop_over<MODE == 1 ? LOOP_DENS : LOOP_DIV>(S, ss, c.begin == 0, iter + 1, sh)) return;
+        }
+    }
     if (i >= S.n) return;
     const KCoefD k = S.kd;
     const double eps = 1.0e-5;
-    const double dt = ss->dt;
     const float4 xi = ld4(S.xk, i);
     const double xx = xi.x, xy = xi.y, xz = xi.z;
     const double si = xi.w;
@@ -1602,13 +1777,20 @@ __global__ __launch_bounds__(kBlock) void k_df_vel(const DevScene* __restrict__ 
 // (:327, :512; the divergence loop is bounded by maxIterations):
 //   continue while (err > eta (eta_V/dt) or it < minIt) and it < maxIt.
 template <int MODE>
-__global__ __launch_bounds__(kBlock) void k_df_err(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+__global__ __launch_bounds__(kBlock) void k_df_err(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                   int fused) {
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
-    const Scalars* ss = S.ss;
+    if (S.stall) return;
+    Scalars* ss = S.ss;
     constexpr bool DENS = (MODE <= 1);
     if (MODE == 1 && ss->done) return;
     if (MODE == 3 && ss->doneV) return;
+    // `fused`: no finalize kernel counts the iteration
+    if (fused && MODE != 0 && c.begin == 0 && threadIdx.x == 0) {
+        if (DENS) ss->it += 1;
+        else ss->itV += 1;
+    }
     __shared__ double sh[kWaves];
     const int i = c.begin + threadIdx.x;
     const KCoefD k = S.kd;
@@ -1687,17 +1869,28 @@ __global__ __launch_bounds__(kBlock) void k_df_err(const DevScene* __restrict__ 
         S.xk[i] = make_float4(xi.x, xi.y, xi.z, (float)s);
     }
     const double bs = block_sum(e, sh);
-    if (threadIdx.x == 0) S.partial[c.begin / kBlock] = bs;
+    // `fused`: the error before the loop, which only the log has, waits in
+    // the sort's scratch for the cell scan to add it up
+    double* const part = (fused && MODE == 0) ? (double*)S.perm : S.partial;
+    if (threadIdx.x == 0) part[c.begin / kBlock] = bs;
 }
 
 // updatePositions (src/DFSPHSolver.cpp:216-236) fused with the cell key and
 // histogram of the grid rebuild.
 // Also clears the loop counters (scenes iterating, largest count) for the
 // divergence solve, which the list build's finalize starts counting.
+// `ahead`: the host has launched the density iterations of a lone scene
+// without asking; if the loop has not ended, nothing from here on runs (the
+// cell scan behind it tells the later launches).
 __global__ __launch_bounds__(kBlock) void k_df_positions(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
-                                                         int* active) {
-    const Chunk c = C[blockIdx.x];
+                                                         int* active, int fused, int ahead) {
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
+    if (S.stall) return;
+    if (ahead && !ended_before(S.ss->done, kLoopLast)) {
+        __shared__ double sh[kWaves];
+        if (!fused || !loop_over<LOOP_DENS>(S, S.ss, c.begin == 0, kLoopLast, sh)) return;
+    }
     if (blockIdx.x == 0 && threadIdx.x < 2) active[threadIdx.x] = 0;
     // the lists about to be built start without an overflow
     if (c.begin == 0 && threadIdx.x == 0) G(S.ss)->listOver = 0u;
@@ -1733,12 +1926,17 @@ __global__ __launch_bounds__(kBlock) void k_df_positions(const DevScene* __restr
 // included), then updatePressure (:249-295): p_i += delta max(0, rho_i -
 // rho0); the scene's max relative error decides the loop (:365), counting
 // this iteration as done (its pressure acceleration always follows).
-__global__ __launch_bounds__(kBlock) void k_pci_density(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+// `fused`: the sweep decides whether its iteration runs (loop_over).
+__global__ __launch_bounds__(kBlock) void k_pci_density(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                        int iter, int fused) {
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
-    const Scalars* ss = S.ss;
-    if (ss->done) return;
+    if (S.stall) return;
+    Scalars* ss = S.ss;
+    if (ended_before(ss->done, iter + 1)) return;
     __shared__ double sh[kWaves];
+    if (fused && loop_over<LOOP_PCI>(S, ss, c.begin == 0, iter + 1, sh)) return;
+    double* const part = fused ? pci_partial(S, ss->it) : S.partial;
     const int i = c.begin + threadIdx.x;
     const KCoefD k = S.kd;
     const bool useShell = S.pciShell && ss->shellBad == 0u;
@@ -1818,7 +2016,7 @@ __global__ __launch_bounds__(kBlock) void k_pci_density(const DevScene* __restri
         e = err / rho0;
     }
     const double bm = block_max(e, sh);
-    if (threadIdx.x == 0) S.partial[c.begin / kBlock] = bm;
+    if (threadIdx.x == 0) part[c.begin / kBlock] = bm;
     if (S.pciShell) {
         // the max is order-free: one atomic per block on non-negative FP32 bits
         const double dm = block_max(dd, sh);
@@ -1830,11 +2028,17 @@ __global__ __launch_bounds__(kBlock) void k_pci_density(const DevScene* __restri
 // predicted densities (src/PCISPHSolver.cpp:297-358), then the prediction of
 // the next iteration (:122-149).  Runs after every k_pci_density, including
 // the one that ended the loop.
-__global__ __launch_bounds__(kBlock) void k_pci_pacc(const DevScene* __restrict__ T, const Chunk* __restrict__ C, int iter) {
-    const Chunk c = C[blockIdx.x];
+__global__ __launch_bounds__(kBlock) void k_pci_pacc(const DevScene* __restrict__ T, const Chunk* __restrict__ C, int iter,
+                                                     int fused) {
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
-    const Scalars* ss = S.ss;
-    if (ss->it <= iter) return;   // this scene finished before this iteration
+    if (S.stall) return;
+    Scalars* ss = S.ss;
+    // this scene finished before this iteration (the finalize kernel counts
+    // the iteration; with `fused` the density sweep sets done instead, and the
+    // iteration is counted here)
+    if (fused ? ss->done : ss->it <= iter) return;
+    if (fused && c.begin == 0 && threadIdx.x == 0) ss->it += 1;
     const int i = c.begin + threadIdx.x;
     if (i >= S.n) return;
     const KCoefD k = S.kd;
@@ -1880,9 +2084,16 @@ __global__ __launch_bounds__(kBlock) void k_pci_pacc(const DevScene* __restrict_
 }
 
 // PCISPH integrate (src/PCISPHSolver.cpp:444-474): a += g + pacc.
-__global__ __launch_bounds__(kBlock) void k_pci_integrate(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+// `ahead`: as in k_df_positions; the launch behind this one tells the rest.
+__global__ __launch_bounds__(kBlock) void k_pci_integrate(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                          int fused, int ahead) {
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
+    if (S.stall) return;
+    if (ahead && !ended_before(S.ss->done, kLoopLast)) {
+        __shared__ double sh[kWaves];
+        if (!fused || !loop_over<LOOP_PCI>(S, S.ss, c.begin == 0, kLoopLast, sh)) return;
+    }
     const int i = c.begin + threadIdx.x;
     if (c.begin == 0 && threadIdx.x == 0 && time_in_last_kernel(S)) advance_time(S);
     if (i >= S.n) return;
@@ -1922,6 +2133,7 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict_
     const int sc = blockIdx.x;
     if (sc >= nscenes) return;
     const DevScene& S = T[sc];
+    if (S.stall) return;
     const gptr<Scalars> ss = G(S.ss);
     if ((KIND == FIN_DENS || KIND == FIN_PCI) && ss->done) return;
     if (KIND == FIN_DIV && ss->doneV) return;
@@ -1935,18 +2147,10 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict_
             active[0] = 0;
             active[1] = 0;
         }
-        const double maxVel = fmax(0.1, red);
-        const double ts = ss->dt;
-        const double cflTs = S.cfl * 0.4 * 2.0 * S.r / maxVel;
-        double nts;
-        if (cflTs < ts) nts = cflTs;
-        else if (ss->it > 3) nts = ts * 0.99;
-        else nts = ts * 1.001;
-        nts = fmax(nts, S.dtMin);
-        nts = fmin(nts, S.dtMax);
-        ss->dt = nts;
-        ss->maxVel = maxVel;
-        ss->cflTs = cflTs;
+        const NextDt d = next_dt(S, ss->dt, ss->it, red);
+        ss->dt = d.dt;
+        ss->maxVel = d.maxVel;
+        ss->cflTs = d.cflTs;
         ss->steps += 1u;
     } else if (KIND == FIN_PCI) {
         ss->maxDensErr = red;
@@ -1999,6 +2203,53 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict_
     }
 }
 
+// Where a lone scene's loop stands, for the host (one block): after the
+// iterations launched of the density loop (LOOP_DENS), the PCISPH loop, or the
+// divergence loop.  END: the end of a step.  With `tables` the host has not
+// asked after the step's loops and the next step's launches wait behind this
+// one: they return at once if a loop has not ended.
+template <int KIND, bool END>
+__global__ __launch_bounds__(kBlock) void k_loop_end(const DevScene* __restrict__ T, int fused, Tables tables, StepRec* rec,
+                                                     unsigned seq) {
+    const DevScene& S = T[0];
+    Scalars* ss = S.ss;
+    int stall = S.stall;
+    __shared__ double sh[kWaves];
+    if (!stall) {
+        bool over = (KIND == LOOP_DIV ? ss->doneV : ss->done) != 0;
+        __syncthreads();   // every thread has read the flag before it is set
+        if (!over && fused && !(END && KIND == LOOP_PCI)) over = loop_over<KIND>(S, ss, true, kLoopLast, sh);
+        if (END && KIND == LOOP_DIV && fused) {
+            const double avg0 = scene_partial_sum((const double*)S.perm, S.nChunks, sh) / (double)S.n;
+            if (threadIdx.x == 0) ss->avgErrV0 = avg0;
+        }
+        if (END && !over && tables.a) {
+            stall = KIND == LOOP_PCI ? 1 : 2;
+            if (threadIdx.x == 0) tables.a->stall = tables.b->stall = stall;
+        }
+        if (threadIdx.x == 0) rec->done = over ? 1 : 0;
+    }
+    if (threadIdx.x == 0) {
+        rec->it = ss->it;
+        rec->itV = ss->itV;
+        rec->stall = stall;
+        __hip_atomic_store(&rec->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+// A batch's loop counters for the host: the scenes still iterating (done) and
+// the largest count reached (it).
+__global__ void k_tell_active(const int* active, StepRec* rec, unsigned seq) {
+    if (threadIdx.x == 0) {
+        rec->done = active[0];
+        rec->it = active[1];
+        __hip_atomic_store(&rec->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+// The host has taken notice of a stall.
+__global__ void k_clear_stall(Tables tables) {
+    if (threadIdx.x == 0) tables.a->stall = tables.b->stall = 0;
+}
+
 // CubeBoundaryModel::correctPositionAndVelocity (src/CubeBoundaryModel.cpp:
 // 16-94): per axis in x, y, z order, a position below the minimum (above
 // the maximum) is set to it, the axis velocity is multiplied by -normalFct if
@@ -2007,7 +2258,7 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict_
 // clamped particles is the FP64 comparison's, and a particle left on a face
 // is not clamped again on later steps (FP64 positions sit exactly on it).
 __global__ __launch_bounds__(kBlock) void k_cube(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
     const int i = c.begin + threadIdx.x;
     if (!S.cubeOn) return;
@@ -2199,7 +2450,7 @@ __global__ __launch_bounds__(kBlock) void k_pb_bdensity(const DevScene* __restri
 // correction starts from its predicted velocity.
 template <int MODE>
 __global__ __launch_bounds__(kBlock) void k_pb_correct(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
     if (!S.pbOn) return;
     const int i = c.begin + threadIdx.x;
@@ -2244,7 +2495,7 @@ __global__ __launch_bounds__(kBlock) void k_pb_correct(const DevScene* __restric
 // Keeps the corrected d and the predicted velocity for the projection after
 // the integration.
 __global__ __launch_bounds__(kBlock) void k_pb_predcorrect(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = C[blockIdx.x];
+    const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
     if (!S.pbOn || S.ss->done) return;
     const int i = c.begin + threadIdx.x;
@@ -2344,15 +2595,20 @@ void launch_keys(hipStream_t st, const DevScene* T, const Chunk* C, int n, int* 
     if (begin_active) LAUNCH(k_keys<true>, n, st, T, C, begin_active);
     else LAUNCH(k_keys<false>, n, st, T, C, nullptr);
 }
-void launch_scan(hipStream_t st, const DevScene* T, const Chunk* CC, int ncc, int nscenes, int maxChunks) {
+void launch_scan(hipStream_t st, const DevScene* T, const Chunk* CC, int ncc, int nscenes, int maxChunks, Tables tables,
+                 int fused) {
     if (!ncc) return;
-    LAUNCH(k_scan_sum, ncc, st, T, CC);
+    if (maxChunks <= kScanOneChunks) {
+        LAUNCH(k_scan_final<SCAN_ONE>, ncc, st, T, CC, tables, fused);
+        return;
+    }
+    LAUNCH(k_scan_sum, ncc, st, T, CC, tables, fused);
     if (maxChunks <= kScanFusedChunks) {
-        LAUNCH(k_scan_final<true>, ncc, st, T, CC);
+        LAUNCH(k_scan_final<SCAN_TOTALS>, ncc, st, T, CC, Tables{}, 0);
         return;
     }
     LAUNCH(k_scan_offsets, nscenes, st, T, nscenes);
-    LAUNCH(k_scan_final<false>, ncc, st, T, CC);
+    LAUNCH(k_scan_final<SCAN_OFFSETS>, ncc, st, T, CC, Tables{}, 0);
 }
 void launch_scatter(hipStream_t st, const DevScene* T, const Chunk* C, int n) { if (n) LAUNCH(k_scatter, n, st, T, C); }
 void launch_rank_reorder(hipStream_t st, const DevScene* T, const Chunk* C, int n) { if (n) LAUNCH(k_rank_reorder, n, st, T, C); }
@@ -2362,11 +2618,11 @@ void launch_bvolume(hipStream_t st, const DevScene* T, int scene, int nb, float*
     LAUNCH(k_bvolume, g, st, T, scene, tmp);
     LAUNCH(k_bvolume_pack, g, st, T, scene, (const float*)tmp);
 }
-void launch_build(hipStream_t st, int method, const DevScene* T, const Chunk* C, int n) {
+void launch_build(hipStream_t st, int method, const DevScene* T, const Chunk* C, int n, int fused) {
     if (!n) return;
-    if (method == DFSPH) LAUNCH(k_build<DFSPH>, n, st, T, C);
-    else if (method == WCSPH) LAUNCH(k_build<WCSPH>, n, st, T, C);
-    else LAUNCH(k_build<PCISPH>, n, st, T, C);
+    if (method == DFSPH) LAUNCH(k_build<DFSPH>, n, st, T, C, fused);
+    else if (method == WCSPH) LAUNCH(k_build<WCSPH>, n, st, T, C, 0);
+    else LAUNCH(k_build<PCISPH>, n, st, T, C, 0);
 }
 void launch_normals(hipStream_t st, const DevScene* T, const Chunk* C, int n) { if (n) LAUNCH(k_normals, n, st, T, C); }
 // The combinations of XSPH and cohesion get a kernel of their own; the two
@@ -2389,18 +2645,20 @@ void launch_forces(hipStream_t st, int method, int flags, const DevScene* T, con
     else launch_forces_m<PCISPH>(st, flags, T, C, n);
 }
 void launch_dt(hipStream_t st, const DevScene* T, const Chunk* C, int n) { if (n) LAUNCH(k_dt, n, st, T, C); }
-void launch_df_predict(hipStream_t st, const DevScene* T, const Chunk* C, int n) { if (n) LAUNCH(k_df_predict, n, st, T, C); }
-void launch_df_vel(hipStream_t st, int mode, const DevScene* T, const Chunk* C, int n) {
-    if (!n) return;
-    if (mode == 0) LAUNCH(k_df_vel<0>, n, st, T, C);
-    else if (mode == 1) LAUNCH(k_df_vel<1>, n, st, T, C);
-    else LAUNCH(k_df_vel<2>, n, st, T, C);
+void launch_df_predict(hipStream_t st, const DevScene* T, const Chunk* C, int n, int fused) {
+    if (n) LAUNCH(k_df_predict, n, st, T, C, fused);
 }
-void launch_df_err(hipStream_t st, int mode, const DevScene* T, const Chunk* C, int n) {
+void launch_df_vel(hipStream_t st, int mode, const DevScene* T, const Chunk* C, int n, int iter, int fused) {
     if (!n) return;
-    if (mode == 0) LAUNCH(k_df_err<0>, n, st, T, C);
-    else if (mode == 1) LAUNCH(k_df_err<1>, n, st, T, C);
-    else LAUNCH(k_df_err<3>, n, st, T, C);
+    if (mode == 0) LAUNCH(k_df_vel<0>, n, st, T, C, iter, fused);
+    else if (mode == 1) LAUNCH(k_df_vel<1>, n, st, T, C, iter, fused);
+    else LAUNCH(k_df_vel<2>, n, st, T, C, iter, fused);
+}
+void launch_df_err(hipStream_t st, int mode, const DevScene* T, const Chunk* C, int n, int fused) {
+    if (!n) return;
+    if (mode == 0) LAUNCH(k_df_err<0>, n, st, T, C, fused);
+    else if (mode == 1) LAUNCH(k_df_err<1>, n, st, T, C, fused);
+    else LAUNCH(k_df_err<3>, n, st, T, C, fused);
 }
 void launch_finalize(hipStream_t st, int kind, const DevScene* T, int nscenes, int* active) {
     if (!nscenes) return;
@@ -2413,12 +2671,29 @@ void launch_finalize(hipStream_t st, int kind, const DevScene* T, int nscenes, i
         default: LAUNCH(k_finalize<FIN_PCI>, nscenes, st, T, nscenes, active); break;
     }
 }
-void launch_df_positions(hipStream_t st, const DevScene* T, const Chunk* C, int n, int* active) {
-    if (n) LAUNCH(k_df_positions, n, st, T, C, active);
+void launch_df_positions(hipStream_t st, const DevScene* T, const Chunk* C, int n, int* active, int fused, int ahead) {
+    if (n) LAUNCH(k_df_positions, n, st, T, C, active, fused, ahead);
 }
-void launch_pci_density(hipStream_t st, const DevScene* T, const Chunk* C, int n) { if (n) LAUNCH(k_pci_density, n, st, T, C); }
-void launch_pci_pacc(hipStream_t st, const DevScene* T, const Chunk* C, int n, int iter) { if (n) LAUNCH(k_pci_pacc, n, st, T, C, iter); }
-void launch_pci_integrate(hipStream_t st, const DevScene* T, const Chunk* C, int n) { if (n) LAUNCH(k_pci_integrate, n, st, T, C); }
+void launch_pci_density(hipStream_t st, const DevScene* T, const Chunk* C, int n, int iter, int fused) {
+    if (n) LAUNCH(k_pci_density, n, st, T, C, iter, fused);
+}
+void launch_pci_pacc(hipStream_t st, const DevScene* T, const Chunk* C, int n, int iter, int fused) {
+    if (n) LAUNCH(k_pci_pacc, n, st, T, C, iter, fused);
+}
+void launch_pci_integrate(hipStream_t st, const DevScene* T, const Chunk* C, int n, int fused, int ahead) {
+    if (n) LAUNCH(k_pci_integrate, n, st, T, C, fused, ahead);
+}
+void launch_loop_end(hipStream_t st, int loop, int end, const DevScene* T, int fused, Tables t, StepRec* rec, unsigned seq) {
+    if (loop == LOOP_PCI && end) LAUNCH((k_loop_end<LOOP_PCI, true>), 1, st, T, fused, t, rec, seq);
+    else if (loop == LOOP_PCI) LAUNCH((k_loop_end<LOOP_PCI, false>), 1, st, T, fused, t, rec, seq);
+    else if (loop == LOOP_DENS) LAUNCH((k_loop_end<LOOP_DENS, false>), 1, st, T, fused, t, rec, seq);
+    else if (end) LAUNCH((k_loop_end<LOOP_DIV, true>), 1, st, T, fused, t, rec, seq);
+    else LAUNCH((k_loop_end<LOOP_DIV, false>), 1, st, T, fused, t, rec, seq);
+}
+void launch_tell_active(hipStream_t st, const int* active, StepRec* rec, unsigned seq) {
+    hipLaunchKernelGGL(k_tell_active, dim3(1), dim3(64), 0, st, active, rec, seq);
+}
+void launch_clear_stall(hipStream_t st, Tables t) { hipLaunchKernelGGL(k_clear_stall, dim3(1), dim3(64), 0, st, t); }
 void launch_cube(hipStream_t st, const DevScene* T, const Chunk* C, int n) { if (n) LAUNCH(k_cube, n, st, T, C); }
 void launch_pb_bself(hipStream_t st, const DevScene* T, int scene, int nb) {
     if (nb) hipLaunchKernelGGL(k_pb_bself, dim3((nb + kBlock - 1) / kBlock), dim3(kBlock), 0, st, T, scene);

@@ -44,3 +44,107 @@ def test_forces_kernel_of_one_and_of_mixed_options(ctx, method, forces):
     assert same(alone, mixed)
     for s in (alone, mixed, extra):
         s.close()
+
+
+def scalars(scene):
+    s = scene.scalars()
+    return [(n, getattr(s, n)) for n, _ in s._fields_]
+
+
+def moving(spec, seed=5, speed=1.0):
+    """Random velocities: iteration counts that change from step to step, so
+    that steps launched ahead need more iterations than were predicted."""
+    return np.random.default_rng(seed).uniform(-speed, speed, spec.fluid.shape).astype(np.float32)
+
+
+LOOPS = {
+    "plain": {},
+    "none_at_least": dict(min_iterations=0, min_iterations_v=0),
+    "one_at_least": dict(min_iterations=1),
+    "many_at_least": dict(min_iterations=5, min_iterations_v=3),
+    "to_the_cap": dict(eta=0.0, eta_v=0.0, max_iterations=7),
+    "cap_below_minimum": dict(min_iterations=4, min_iterations_v=4, max_iterations=2),
+    "no_iterations": dict(max_iterations=0),
+    "loose": dict(eta=10.0, eta_v=1e6),
+}
+
+
+@pytest.mark.parametrize("method", [sphg.DFSPH, sphg.PCISPH])
+@pytest.mark.parametrize("loops", sorted(LOOPS))
+@pytest.mark.parametrize("size", [(3, 3, 3), (9, 7, 8), (31, 17, 9)])
+def test_lone_scene_steps_like_one_of_a_batch(ctx, method, loops, size):
+    """A lone scene decides its loops in the sweeps and launches its steps
+    ahead; in a batch the host asks after finalize kernels.  Uneven calls, so
+    that predictions are carried over, and single steps."""
+    spec = configs.small_scene(method, n_side=size, box=tuple(0.05 * (s + 4) for s in size), **LOOPS[loops])
+    v = moving(spec)
+    alone, mixed, extra = [sphg.Scene(ctx, spec.params, spec.fluid, spec.boundary, v) for _ in range(3)]
+    for steps in (1, 6, 2, 9):
+        a, b = alone.step(steps), ctx.batch_step([mixed, extra], steps)
+        assert 2 * a.iterations == b.iterations and 2 * a.iterations_v == b.iterations_v
+        assert scalars(alone) == scalars(mixed)
+    assert same(alone, mixed)
+    for s in (alone, mixed, extra):
+        s.close()
+
+
+@pytest.mark.parametrize("method", [sphg.DFSPH, sphg.PCISPH])
+def test_loops_decided_by_finalize_kernels_in_a_large_lone_scene(ctx, method):
+    """2,048 chunks of 256 are the most whose partials every block adds up."""
+    for size in ((128, 64, 64), (129, 64, 64)):
+        spec = configs.small_scene(method, n_side=size, spacing=0.02, box=tuple(0.02 * (s + 4) for s in size))
+        other = configs.small_scene(method, n_side=5)
+        v = moving(spec, speed=0.3)
+        alone, mixed = [sphg.Scene(ctx, spec.params, spec.fluid, spec.boundary, v) for _ in range(2)]
+        extra = sphg.Scene(ctx, other.params, other.fluid, other.boundary)
+        alone.step(5)
+        ctx.batch_step([mixed, extra], 5)
+        assert scalars(alone) == scalars(mixed) and same(alone, mixed)
+        for s in (alone, mixed, extra):
+            s.close()
+
+
+@pytest.mark.parametrize("method", [sphg.DFSPH, sphg.PCISPH])
+def test_lone_scene_with_replay_schedules_and_timing(ctx, method):
+    """Captured segments, launch schedules and kernel timing change which
+    launches are made ahead, not what they compute."""
+    spec = configs.small_scene(method, n_side=(12, 9, 8), box=(0.9, 0.65, 0.6))
+    v = moving(spec)
+    base, replay, timed = [sphg.Scene(ctx, spec.params, spec.fluid, spec.boundary, v) for _ in range(3)]
+    base.step(24)
+    ctx.set_graphs(True)
+    for steps in (1, 3, 10, 10):
+        replay.step(steps)
+    ctx.set_graphs(False)
+    timed.step(3)
+    ctx.kernel_timing(True)
+    timed.step(4)
+    launches = ctx.kernel_time("build")[0]
+    ctx.kernel_timing(False)
+    timed.step(17)
+    assert launches == 4
+    assert scalars(base) == scalars(replay) == scalars(timed)
+    assert same(base, replay) and same(base, timed)
+    for s in (base, replay, timed):
+        s.close()
+
+
+@pytest.mark.parametrize("cells", [31 * 1024 + 1, 32 * 1024, 33 * 1024, 90 * 1024])
+def test_cell_scan_in_one_and_two_launches(ctx, cells):
+    """Up to 32 scan chunks of 1,024 cells the counts are scanned in one
+    launch.  A domain stretched along z keeps every cell's index."""
+    from dataclasses import replace
+    spec = configs.small_scene(sphg.WCSPH, n_side=(9, 7, 8), box=(0.9, 0.55, 0.8))
+    pts = np.concatenate([spec.fluid, spec.boundary]).astype(np.float64)
+    lo, hi = pts.min(axis=0), pts.max(axis=0)
+    g = sphg.Scene(ctx, replace(spec.params, domain_min=tuple(lo), domain_max=tuple(hi)), spec.fluid, spec.boundary)
+    h = spec.params.support_radius
+    layer = np.prod([np.floor(hi[a] / h) - np.floor(lo[a] / h) + 5 for a in (0, 1)])
+    tall = replace(spec.params, domain_min=tuple(lo), domain_max=(hi[0], hi[1], h * np.ceil(cells / layer)))
+    t = sphg.Scene(ctx, tall, spec.fluid, spec.boundary)
+    assert g.info()["ncells"] <= 32 * 1024 and abs(t.info()["ncells"] - cells) <= 8 * layer
+    g.step(6)
+    t.step(6)
+    assert same(g, t)
+    g.close()
+    t.close()
