@@ -79,12 +79,12 @@ template <class T> __device__ inline void stg(T* p, uint32_t i, T v) {
 // tables have it.  Without the table a block's first load is its scene's
 // entry, not the chunk and then the scene: one memory round trip (0.5-0.8 us)
 // less in each of a small step's launches.
-__device__ inline Chunk chunk_at(const Chunk* C, int unit) {
-    const int b = blockIdx.x;
+__device__ inline Chunk chunk_at(const Chunk* C, int unit, int b, int nchunks) {
     if (C) return C[b];
-    const int x = b & 7, per = gridDim.x >> 3, more = gridDim.x & 7;
+    const int x = b & 7, per = nchunks >> 3, more = nchunks & 7;
     return Chunk{0, (x * per + min(x, more) + (b >> 3)) * unit};
 }
+__device__ inline Chunk chunk_at(const Chunk* C, int unit) { return chunk_at(C, unit, blockIdx.x, gridDim.x); }
 
 __device__ inline double wave_sum(double v) {
 #pragma unroll
@@ -135,6 +135,21 @@ __device__ inline double scene_partial_sum(const double* partial, int n, double*
         for (int u = 0; u < kPartU; ++u) v[u] = (b + u * kBlock < n) ? ldg(partial, (size_t)(b + u * kBlock)) : 0.0;
 #pragma unroll
         for (int u = 0; u < kPartU; ++u) acc += v[u];
+    }
+    return block_sum(acc, sh);
+}
+// The same over n chunks whose wavefronts' sums are in `wp`, kWaves a chunk:
+// a chunk's sum is formed as block_sum forms it.
+__device__ inline double scene_wave_sum(const double* wp, int n, double* sh) {
+    double acc = 0.0;
+    for (int b = threadIdx.x; b < n; b += kBlock) {
+        double v[kWaves];
+#pragma unroll
+        for (int k = 0; k < kWaves; ++k) v[k] = ldg(wp, (size_t)b * kWaves + k);
+        double r = v[0];
+#pragma unroll
+        for (int k = 1; k < kWaves; ++k) r += v[k];
+        acc += r;
     }
     return block_sum(acc, sh);
 }
@@ -890,6 +905,106 @@ constexpr int kWaveStage = SPHG_BUILD_STAGE ? 816 : 1;   // candidates per wavef
 // to 3 entries past the staged ones, so the stage has 3 more.
 constexpr int kWaveStagePad = kWaveStage + 3;
 
+// FP64 test of a candidate: whether the reference's sums hold it, its W and
+// gradient factor, and whether its gradient is nonzero.
+// 1e-9 <= r2 < hlo2: |r| > 1e-5 and q < 1, where W and the gradient take
+// their inner forms and the gradient is nonzero.  The reference's gradient
+// (src/CubicSpline.h:55-73) vanishes only at |r| <= 1e-5 and q = 1; near those
+// two, and near q = 1 for the list membership, the test is repeated
+// operation-exact in FP64.
+__device__ inline bool member_of(const Pair& p, const float4& xi, const float4& xj, double hD, const KCoefD& k, double& g,
+                                 double& wq, bool& gnz) {
+    if (!(p.r2 <= k.hhi2)) return false;
+    g = G_in(p, k);
+    wq = W_in(p.q, k);
+    gnz = true;
+    if (p.r2 >= k.hlo2 || p.r2 < 1e-9) {
+        const Exact e = exact_q(xi, xj, hD);
+        if (!(e.q <= 1.0)) return false;
+        gnz = grad_nonzero64(e);
+        g = G_d(p, k);
+        wq = W_d(p.q, k);
+    }
+    return true;
+}
+
+// A particle's sums over its neighbors and boundary neighbors.
+struct BuildSums {
+    double ws = 0.0, sgx = 0.0, sgy = 0.0, sgz = 0.0, ssq = 0.0;
+    double dv = 0.0;                             // DFSPH: sum_j g_ij (v_i - v_j).(x_i - x_j)
+    double bw = 0.0, bgx = 0.0, bgy = 0.0, bgz = 0.0;
+    double sx2 = 0.0, sy2 = 0.0, sz2 = 0.0;      // spiky boundary sum (PCISPH)
+    double ax = 0.0, ay = 0.0, az = 0.0;         // adhesion sum
+};
+
+// What a particle's list and sums give, stored: `cnt` members, `own` of them
+// in the list.  Returns its share of the average divergence error (DFSPH).
+template <int M>
+__device__ inline double build_finish(const DevScene& S, int i, const float4& xi, const float4& vi, const BuildSums& b,
+                                      int cnt, int own, int ngr) {
+    const KCoefD& k = S.kd;
+    const double rho0 = S.rho0D, m = S.mD;
+    if (cnt > S.maxNbr) {
+        atomicMax(&S.ss->overflow, (unsigned)cnt);
+        atomicMax(&S.ss->listOver, (unsigned)cnt);
+    }
+    stg(S.nnb, (size_t)i, (uint16_t)own);
+    stg(S.ngrad, (size_t)i, (uint8_t)min(ngr, 255));
+    const double drho = (m * (k.ck + b.ws) + b.bw) - rho0;
+    const double rho = rho0 + drho;
+    stg(S.drho, (size_t)i, (float)drho);
+    st4(S.gb, i, make_float4((float)b.bgx, (float)b.bgy, (float)b.bgz, (float)b.bw));
+    if (S.flags & F_ADH) st4(S.adh, i, make_float4((float)b.ax, (float)b.ay, (float)b.az, 0.f));
+    if (M == DFSPH) {
+        const double tx = m * b.sgx + b.bgx, ty = m * b.sgy + b.bgy, tz = m * b.sgz + b.bgz;
+        const double den = tx * tx + ty * ty + tz * tz + m * m * b.ssq;
+        const float alpha = (fabs(den) > 1e-5) ? (float)(rho / den) : 0.0f;
+        stg(S.alpha, (size_t)i, alpha);
+        // initial divergence error of the step's divergence solve
+        // (computeDivergenceError, src/DFSPHSolver.cpp:408-492, and kappa_v,
+        // :531), from the pairs above; stored values are read back as the
+        // later sweeps read them (FP32 gb, delta rho, alpha)
+        const float4 gbf = make_float4((float)b.bgx, (float)b.bgy, (float)b.bgz, (float)b.bw);
+        const double ux = vi.x, uy = vi.y, uz = vi.z;
+        const double dc = m * b.dv + (ux * (double)gbf.x + uy * (double)gbf.y + uz * (double)gbf.z);
+        const double de = (ngr < 20) ? 0.0 : fmax(dc, 0.0);
+        const double rhof = rho0 + (double)(float)drho;
+        // the divergence of the velocities: the next step's D0 unless a
+        // divergence iteration replaces it
+        ((gptr<double>)S.d0)[i] = dc;
+        stg(S.divErr, (size_t)i, (float)de);
+        st4(S.xk, i, make_float4(xi.x, xi.y, xi.z, (float)(de * (double)alpha / (S.ss->dt * rhof))));
+        return de / rho0;
+    }
+    if (M == WCSPH) {
+        // p = max(0, kappa rho0/gamma ((rho/rho0)^gamma - 1)), written
+        // (1+x)^g - 1 = expm1(g log1p(x)) with x = (rho - rho0)/rho0
+        const double x = drho / rho0;
+        const double pr = fmax(0.0, (double)S.stiffness * rho0 / (double)S.gammaEos * expm1((double)S.gammaEos * log1p(x)));
+        stg(S.p, (size_t)i, (float)pr);
+        st4(S.xk, i, make_float4(xi.x, xi.y, xi.z, (float)(pr / (rho * rho))));
+        const float4 v = ld4(S.v, i);
+        st4(S.aux, i, make_float4(v.x, v.y, v.z, (float)(m / rho)));
+    } else {
+        st4(S.gbs, i, make_float4((float)b.sx2, (float)b.sy2, (float)b.sz2, 0.f));
+    }
+    return 0.0;
+}
+
+// The end of a DFSPH list build: each wavefront's share of the error before
+// the divergence loop (only the log has it) goes to the sort's scratch; one
+// thread of a scene starts the divergence loop (`fused`: no finalize kernel
+// does).
+__device__ inline void build_starts_divergence(const DevScene& S, int fused) {
+    Scalars* const ss = S.ss;
+    ss->d0Valid = 1u;
+    if (fused) {
+        ss->itV = 0;
+        ss->time += ss->dt;
+        ss->doneV = loop_goes_on<LOOP_DIV>(S, ss, 0, 0.0) ? 0 : 1;
+    }
+}
+
 template <int M>
 __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
                                                   int fused) {
@@ -999,9 +1114,7 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
     int ns = 0;
     bool shellLost = false;
     int cnt = 0, ngr = 0;
-    double ws = 0.0, sgx = 0.0, sgy = 0.0, sgz = 0.0, ssq = 0.0;
-    // DFSPH: sum_j g_ij (v_i - v_j).(x_i - x_j) of the divergence error
-    double dv = 0.0;
+    BuildSums b;
     const float4 vi = (M == DFSPH && valid) ? ld4(S.v, i) : make_float4(0.f, 0.f, 0.f, 0.f);
     const double ux = vi.x, uy = vi.y, uz = vi.z;
     // FP64 test and sums of one candidate that passed the FP32 test
@@ -1017,36 +1130,21 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
     // entry is written only where the compaction moves it
     auto visit = [&](uint32_t j, const float4& xj, const float4& vj, int pos) {
         const Pair p = pair_of(xx, xy, xz, xj, k);
-        if (!(p.r2 <= k.hhi2)) {
+        double g, wq;
+        bool gnz;
+        if (!member_of(p, xi, xj, S.hD, k, g, wq, gnz)) {
             toShell(j);
             return;
-        }
-        // 1e-9 <= r2 < hlo2: |r| > 1e-5 and q < 1, where W and the gradient
-        // take their inner forms and the gradient is nonzero.  The
-        // reference's gradient (src/CubicSpline.h:55-73) vanishes only at
-        // |r| <= 1e-5 and q = 1; near those two, and near q = 1 for the list
-        // membership, the test is repeated operation-exact in FP64.
-        double g = G_in(p, k), wq = W_in(p.q, k);
-        bool gnz = true;
-        if (p.r2 >= k.hlo2 || p.r2 < 1e-9) {
-            const Exact e = exact_q(xi, xj, S.hD);
-            if (!(e.q <= 1.0)) {
-                toShell(j);
-                return;
-            }
-            gnz = grad_nonzero64(e);
-            g = G_d(p, k);
-            wq = W_d(p.q, k);
         }
         if (cnt < maxN && cnt != pos) stg(L, (size_t)slot_of(cnt), j);
         ++cnt;
         ngr += gnz ? 1 : 0;
-        ws += wq;
-        sgx += g * p.dx;
-        sgy += g * p.dy;
-        sgz += g * p.dz;
-        ssq += g * g * p.r2;
-        if (M == DFSPH) dv += g * ((ux - (double)vj.x) * p.dx + (uy - (double)vj.y) * p.dy + (uz - (double)vj.z) * p.dz);
+        b.ws += wq;
+        b.sgx += g * p.dx;
+        b.sgy += g * p.dy;
+        b.sgz += g * p.dz;
+        b.ssq += g * g * p.r2;
+        if (M == DFSPH) b.dv += g * ((ux - (double)vj.x) * p.dx + (uy - (double)vj.y) * p.dy + (uz - (double)vj.z) * p.dz);
     };
     auto vel = [&](uint32_t j) { return (M == DFSPH) ? ld3o(S.v, j) : make_float4(0.f, 0.f, 0.f, 0.f); };
     // pass 1 over the 27 cells as 9 rows (walk27 order), candidate positions
@@ -1189,9 +1287,6 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
     for (int o = 32; o > 0; o >>= 1) pad = max(pad, __shfl_xor(pad, o));
     double e = 0.0;   // DFSPH: this particle's share of the average divergence error
     if (valid) {
-    double bw = 0.0, bgx = 0.0, bgy = 0.0, bgz = 0.0;
-    double sx2 = 0.0, sy2 = 0.0, sz2 = 0.0;   // spiky boundary sum (PCISPH)
-    double ax = 0.0, ay = 0.0, az = 0.0;      // adhesion sum
     const bool wantAdh = (S.flags & F_ADH) != 0;
     const double rho0 = S.rho0D;
     // boundary sums, in two passes like the fluid: FP32 survivors go to the
@@ -1200,22 +1295,22 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
         const Pair p = pair_of(xx, xy, xz, y, k);
         if (!(p.q <= 1.0)) return;
         const double cb = rho0 * (double)y.w;
-        bw += cb * W_d(p.q, k);
+        b.bw += cb * W_d(p.q, k);
         const double g = cb * G_d(p, k);
-        bgx += g * p.dx;
-        bgy += g * p.dy;
-        bgz += g * p.dz;
+        b.bgx += g * p.dx;
+        b.bgy += g * p.dy;
+        b.bgz += g * p.dz;
         if (M == PCISPH) {
             const double gs = cb * Gs_d(p, k);
-            sx2 += gs * p.dx;
-            sy2 += gs * p.dy;
-            sz2 += gs * p.dz;
+            b.sx2 += gs * p.dx;
+            b.sy2 += gs * p.dy;
+            b.sz2 += gs * p.dz;
         }
         if (wantAdh && p.r2 > 0.0) {
             const double sa = cb * A_d(p.rl, k) * p.inv;
-            ax += sa * p.dx;
-            ay += sa * p.dy;
-            az += sa * p.dz;
+            b.ax += sa * p.dx;
+            b.ay += sa * p.dy;
+            b.az += sa * p.dz;
         }
     };
     // the boundary survivors use the free slots between the list and the shell
@@ -1259,8 +1354,8 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
                 if (q0 + u < nbc) bvisit(yb[u]);
         }
     } else {
-        walk27(S.bCellStart, ci, nx, nxny, [&](int b) {
-            const float4 y = ld4(S.xb, b);
+        walk27(S.bCellStart, ci, nx, nxny, [&](int jb) {
+            const float4 y = ld4(S.xb, jb);
             const float fx = xi.x - y.x, fy = xi.y - y.y, fz = xi.z - y.z;
             if (fx * fx + fy * fy + fz * fz <= hh) bvisit(y);
         });
@@ -1273,66 +1368,384 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
         stg(S.nsh, (size_t)i, (uint16_t)(shellLost ? 0xFFFF : ns));
     }
     if ((i & 63) == 0) stg(S.gcnt, (size_t)(i >> 6), (uint16_t)pad);
-    if (cnt > maxN) {
-        atomicMax(&S.ss->overflow, (unsigned)cnt);
-        atomicMax(&S.ss->listOver, (unsigned)cnt);
-    }
-    stg(S.nnb, (size_t)i, (uint16_t)own);
-    stg(S.ngrad, (size_t)i, (uint8_t)min(ngr, 255));
-    const double m = S.mD;
-    const double drho = (m * (k.ck + ws) + bw) - rho0;
-    const double rho = rho0 + drho;
-    stg(S.drho, (size_t)i, (float)drho);
-    st4(S.gb, i, make_float4((float)bgx, (float)bgy, (float)bgz, (float)bw));
-    if (wantAdh) st4(S.adh, i, make_float4((float)ax, (float)ay, (float)az, 0.f));
-    if (M == DFSPH) {
-        const double tx = m * sgx + bgx, ty = m * sgy + bgy, tz = m * sgz + bgz;
-        const double den = tx * tx + ty * ty + tz * tz + m * m * ssq;
-        const float alpha = (fabs(den) > 1e-5) ? (float)(rho / den) : 0.0f;
-        stg(S.alpha, (size_t)i, alpha);
-        // initial divergence error of the step's divergence solve
-        // (computeDivergenceError, src/DFSPHSolver.cpp:408-492, and kappa_v,
-        // :531), from the pairs above; stored values are read back as the
-        // later sweeps read them (FP32 gb, delta rho, alpha)
-        const float4 gbf = make_float4((float)bgx, (float)bgy, (float)bgz, (float)bw);
-        const double dc = m * dv + (ux * (double)gbf.x + uy * (double)gbf.y + uz * (double)gbf.z);
-        const double de = (ngr < 20) ? 0.0 : fmax(dc, 0.0);
-        const double rhof = rho0 + (double)(float)drho;
-        // the divergence of the velocities: the next step's D0 unless a
-        // divergence iteration replaces it
-        ((gptr<double>)S.d0)[i] = dc;
-        stg(S.divErr, (size_t)i, (float)de);
-        st4(S.xk, i, make_float4(xi.x, xi.y, xi.z, (float)(de * (double)alpha / (S.ss->dt * rhof))));
-        e = de / rho0;
-    } else if (M == WCSPH) {
-        // p = max(0, kappa rho0/gamma ((rho/rho0)^gamma - 1)), written
-        // (1+x)^g - 1 = expm1(g log1p(x)) with x = (rho - rho0)/rho0
-        const double x = drho / rho0;
-        const double pr = fmax(0.0, (double)S.stiffness * rho0 / (double)S.gammaEos * expm1((double)S.gammaEos * log1p(x)));
-        stg(S.p, (size_t)i, (float)pr);
-        st4(S.xk, i, make_float4(xi.x, xi.y, xi.z, (float)(pr / (rho * rho))));
-        const float4 vi = ld4(S.v, i);
-        st4(S.aux, i, make_float4(vi.x, vi.y, vi.z, (float)(m / rho)));
-    } else {
-        st4(S.gbs, i, make_float4((float)sx2, (float)sy2, (float)sz2, 0.f));
-    }
+    e = build_finish<M>(S, i, xi, vi, b, cnt, own, ngr);
     }
     if (M == DFSPH) {
-        __shared__ double sh[kWaves];
-        const double bs = block_sum(e, sh);
-        // `fused`: the step's time and the start of the divergence loop are
-        // written here, and the error before the loop (for the log) waits in
-        // the sort's scratch for the step's end
-        if (threadIdx.x == 0) (fused ? (double*)S.perm : S.partial)[c.begin / kBlock] = bs;
-        if (c.begin == 0 && threadIdx.x == 0) {
-            Scalars* const ss = S.ss;
-            ss->d0Valid = 1u;
-            if (fused) {
-                ss->itV = 0;
-                ss->time += ss->dt;
-                ss->doneV = loop_goes_on<LOOP_DIV>(S, ss, 0, 0.0) ? 0 : 1;
+        const double es = wave_sum(e);
+        if (lane == 0) ((gptr<double>)S.perm)[wb >> 6] = es;
+        if (c.begin == 0 && threadIdx.x == 0) build_starts_divergence(S, fused);
+    }
+}
+
+// The same build with 4 lanes a particle, for launches too small to fill the
+// chip.  A block of 4 wavefronts holds one list group: lane 4 q + u of
+// wavefront w works on particle 16 w + q of the group, on every 4th candidate
+// from u on.  The block stages its group's rows once, for the fluid and for
+// the boundary.  Where k_build's wavefront walks its 27 cells 4 candidates at
+// a time in ~50 passes, each waiting on LDS, its four stores and, later, ~10
+// passes over the survivors' data in memory, a quad has a quarter of the
+// instructions in each of them.  Survivors keep their order (their slots are
+// counted within the quad), and the four lanes' FP64 terms are added one after
+// the other in list order, in every lane alike, so the sums are k_build's bit
+// for bit. A step (most of the difference is this kernel): WCSPH 2,197
+// particles 83 -> 55 us, 32,768 71 -> 54, PCISPH 4,845 239 -> 204, DFSPH 4,096
+// 149 -> 122, 35,805 184 -> 164.
+constexpr int kQuadStage = 816, kQuadPad = 8;    // fluid candidates staged (12 B each); reads past a row's end
+constexpr int kQuadBound = 512;                  // boundary candidates staged (16 B each)
+
+// x of lane V of the quad
+template <int V>
+__device__ inline int quad_lane(int x) {
+    return __builtin_amdgcn_update_dpp(0, x, V * 0x55, 0xf, 0xf, true);
+}
+template <int V>
+__device__ inline double quad_lane(double x) {
+    return __hiloint2double(quad_lane<V>(__double2hiint(x)), quad_lane<V>(__double2loint(x)));
+}
+
+template <int M>
+__global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__ T, const Chunk* __restrict__ C, int nchunks,
+                                                    int fused) {
+    // a chunk's groups run on one XCD, like the chunk
+    const int slot = ((int)(blockIdx.x >> 3) / kWaves) * 8 + (int)(blockIdx.x & 7), sub = (int)(blockIdx.x >> 3) % kWaves;
+    if (slot >= nchunks) return;
+    const Chunk c = chunk_at(C, kBlock, slot, nchunks);
+    const DevScene& S = T[c.scene];
+    if (S.stall) return;
+    __shared__ float2 sxy[kQuadStage + kQuadPad];
+    __shared__ float sz[kQuadStage + kQuadPad];
+    __shared__ float4 sb[kQuadBound];
+    __shared__ double se[kGroup];
+    __shared__ int spad[4];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, u = lane & 3;
+    const int g0 = c.begin + sub * kGroup;   // the group's first particle
+    const int pl = w * 16 + (lane >> 2);     // the lane's particle in the group
+    const int i = g0 + pl;
+    if (g0 >= S.n) {
+        if (M == DFSPH && tid == 0) ((gptr<double>)S.perm)[g0 >> 6] = 0.0;
+        return;
+    }
+    const bool valid = i < S.n;
+    const int il = min(i, S.n - 1);
+    const KCoefD k = S.kd;
+    const float hh = S.kc.hhi2 * (1.0f + 1e-5f);   // conservative FP32 pre-filter
+    const float4 xi = ld4(S.x, (size_t)il);
+    const int ci = ldg(S.cell, (size_t)il);
+    const int cF = ldg(S.cell, (size_t)g0), cL = ldg(S.cell, (size_t)min(g0 + kGroup - 1, S.n - 1));
+    const float4 vi = (M == DFSPH) ? ld4(S.v, (size_t)il) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const double xx = xi.x, xy = xi.y, xz = xi.z;
+    const double ux = vi.x, uy = vi.y, uz = vi.z;
+    const int nx = S.nx, nxny = S.nx * S.ny;
+    // the particle's 9 rows, and the group's 9 fluid (lanes 0..8) and boundary
+    // (lanes 16..24) rows with their offsets in the stages
+    int rs[9], re[9];
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+        const int off = (r % 3 - 1) * nx + (r / 3 - 1) * nxny;
+        rs[r] = ldg(S.cellStart, (size_t)(ci - 1 + off));
+        re[r] = ldg(S.cellStart, (size_t)(ci + 2 + off));
+    }
+    int rfirst = 0, rcnt = 0;
+    const int lr = lane & 15;
+    if (lane < 32 && lr < 9) {
+        const int off = (lr % 3 - 1) * nx + (lr / 3 - 1) * nxny;
+        const int* const tab = lane < 16 ? S.cellStart : S.bCellStart;
+        rfirst = ldg(tab, (size_t)(cF - 1 + off));
+        rcnt = ldg(tab, (size_t)(cL + 2 + off)) - rfirst;
+    }
+    int incl = rcnt;
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) {
+        const int t = __shfl_up(incl, o);
+        if (lr >= o) incl += t;
+    }
+    int first[9], base[10], bfirst[9], bbase[10];
+    base[0] = bbase[0] = 0;
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+        first[r] = __builtin_amdgcn_readlane(rfirst, r);
+        base[r + 1] = __builtin_amdgcn_readlane(incl, r);
+        bfirst[r] = __builtin_amdgcn_readlane(rfirst, 16 + r);
+        bbase[r + 1] = __builtin_amdgcn_readlane(incl, 16 + r);
+    }
+    // the leading fluid rows that fit are staged, and the boundary rows where
+    // all of them fit; what is not staged is read from memory
+    int nStaged = 0;
+#pragma unroll
+    for (int r = 0; r < 9; ++r)
+        if (base[r + 1] <= kQuadStage) nStaged = r + 1;
+    const int tot = base[nStaged];
+    const bool bStaged = bbase[9] <= kQuadBound;
+    const int btot = bStaged ? bbase[9] : 0;
+    {
+        auto at = [&](int t, const int* f, const int* bs) {
+            int o = f[0];
+#pragma unroll
+            for (int q = 1; q < 9; ++q)
+                if (t >= bs[q]) o = f[q] - bs[q];
+            return o + t;
+        };
+        float4 p[4], y[2];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (tid + 256 * q < tot) p[q] = ld3o(S.x, (uint32_t)at(tid + 256 * q, first, base));
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            if (tid + 256 * q < btot) y[q] = ld4o(S.xb, (uint32_t)at(tid + 256 * q, bfirst, bbase));
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (tid + 256 * q < tot) {
+                sxy[tid + 256 * q] = make_float2(p[q].x, p[q].y);
+                sz[tid + 256 * q] = p[q].z;
+            }
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            if (tid + 256 * q < btot) sb[tid + 256 * q] = y[q];
+    }
+    __syncthreads();
+
+    uint32_t* const L = list_of_w(S, g0 + pl);
+    const int maxN = S.maxNbr;
+    const uint32_t below = (1u << u) - 1u;
+    const int qshift = lane & ~3;
+    // the quad's 4 flags, lane u in bit u
+    auto quad_bits = [&](bool f) { return (uint32_t)(__ballot(f) >> qshift) & 15u; };
+    float hsk = 0.f;
+    if (M == PCISPH && S.pciShell) {
+        const float hs = S.kc.h + pci_skin(S);
+        hsk = hs * hs * (1.0f + 1e-4f);
+    }
+    int nc = 0, ns = 0;
+    bool shellLost = false;
+    // pass 1: this lane's candidate j at squared distance d2 (in: it is one)
+    auto scan = [&](bool in, uint32_t j, float d2) {
+        const bool ok = in & (d2 <= hh);
+        const uint32_t okb = quad_bits(ok);
+        if (M == PCISPH) {
+            const bool sh = in & (d2 > hh) & (d2 <= hsk);
+            const uint32_t shb = quad_bits(sh);
+            const int sn = ns + __popc(shb & below);
+            if (sh) {
+                // below the list's slots only (list writes that later reach
+                // the shell are caught by nc + ns > maxN)
+                if (nc + __popc(okb & below) + sn < maxN) stg(L, (size_t)slot_of(maxN - 1 - sn), j);
+                else shellLost = true;
+            }
+            ns += __popc(shb);
+        }
+        // past the last slot the particle takes the walk over all candidates,
+        // which rewrites its list: the store is clamped to the last slot
+        if (ok) stg(L, (size_t)slot_of(min(nc + __popc(okb & below), maxN - 1)), j);
+        nc += __popc(okb);
+    };
+    if (valid) {
+        static_for<9>([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
+            const int s0 = rs[r], e0 = re[r];
+            if (r < nStaged) {
+                const int t0 = base[r] - first[r] + u;
+                for (int j0 = s0; j0 < e0; j0 += 8) {
+                    float d2[2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const float2 a = sxy[t0 + j0 + 4 * h];
+                        const float fx = xi.x - a.x, fy = xi.y - a.y, fz = xi.z - sz[t0 + j0 + 4 * h];
+                        d2[h] = fx * fx + fy * fy + fz * fz;
+                    }
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const int j = j0 + 4 * h + u;
+                        // particle i itself can only lie in row 4
+                        scan((j < e0) & (r != 4 || j != i), (uint32_t)j, d2[h]);
+                    }
+                }
+            } else {
+                for (int j0 = s0; j0 < e0; j0 += 4) {
+                    const int j = j0 + u;
+                    const float4 a = ld4(S.x, (size_t)min(j, e0 - 1));
+                    const float fx = xi.x - a.x, fy = xi.y - a.y, fz = xi.z - a.z;
+                    scan((j < e0) & (j != i), (uint32_t)j, fx * fx + fy * fy + fz * fz);
+                }
+            }
+        });
+    }
+    shellLost = quad_bits(shellLost) != 0u;
+    int cnt = 0, ngr = 0;
+    BuildSums b;
+    if (M == PCISPH && nc + ns > maxN) shellLost = true;
+    if (valid && nc <= maxN) {
+        // pass 2, 8 survivors at a time
+        const uint32_t* const Lu = L + u;
+        uint32_t jn[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) jn[h] = ldg(Lu, (size_t)slot_of(min(4 * h, maxN - 4)));
+        for (int q0 = 0; q0 < nc; q0 += 8) {
+            uint32_t j[2];
+            float4 xj[2], vj[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                j[h] = (q0 + 4 * h + u < nc) ? jn[h] : (uint32_t)i;   // past the last: a valid index
+                xj[h] = ld3o(S.x, j[h]);
+                vj[h] = (M == DFSPH) ? ld3o(S.v, j[h]) : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+            // maxN is a multiple of 4: the block after the last is re-read
+#pragma unroll
+            for (int h = 0; h < 2; ++h) jn[h] = ldg(Lu, (size_t)slot_of(q0 + 8 + 4 * h < nc ? q0 + 8 + 4 * h : q0));
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int pos = q0 + 4 * h + u;
+                const Pair p = pair_of(xx, xy, xz, xj[h], k);
+                double g = 0.0, wq = 0.0;
+                bool gnz = false;
+                const bool cand = pos < nc;
+                const bool in = cand && member_of(p, xi, xj[h], S.hD, k, g, wq, gnz);
+                const uint32_t inb = quad_bits(in);
+                if (M == PCISPH) {
+                    // what the FP64 test rejects goes to the shell
+                    const uint32_t rj = quad_bits(cand && !in);
+                    const int sn = ns + __popc(rj & below);
+                    if (cand && !in) {
+                        if (sn < maxN - nc) stg(L, (size_t)slot_of(maxN - 1 - sn), j[h]);
+                        else shellLost = true;
+                    }
+                    ns += __popc(rj);
+                }
+                // an entry is written only where the compaction moves it
+                const int to = cnt + __popc(inb & below);
+                if (in && to != pos) stg(L, (size_t)slot_of(to), j[h]);
+                cnt += __popc(inb);
+                ngr += __popc(quad_bits(in && gnz));
+                // in list order; a lane without a member adds zeros, which
+                // change no sum
+                if (!in) g = wq = 0.0;
+                const double gg = g * g;
+                const double dot = (M == DFSPH) ? (ux - (double)vj[h].x) * p.dx + (uy - (double)vj[h].y) * p.dy +
+                                                      (uz - (double)vj[h].z) * p.dz
+                                                : 0.0;
+                static_for<4>([&](auto vc) {
+                    constexpr int v = decltype(vc)::value;
+                    b.ws += quad_lane<v>(wq);
+                    if (M == DFSPH) {
+                        const double gv = quad_lane<v>(g);
+                        b.sgx = fma(gv, quad_lane<v>(p.dx), b.sgx);
+                        b.sgy = fma(gv, quad_lane<v>(p.dy), b.sgy);
+                        b.sgz = fma(gv, quad_lane<v>(p.dz), b.sgz);
+                        b.ssq = fma(quad_lane<v>(gg), quad_lane<v>(p.r2), b.ssq);
+                        b.dv = fma(gv, quad_lane<v>(dot), b.dv);
+                    }
+                });
             }
         }
+    } else if (valid) {
+        // more survivors than slots: all candidates one after the other, the
+        // four lanes alike
+        shellLost = true;
+        walk27(S.cellStart, ci, nx, nxny, [&](int j) {
+            const float4 xj = ld4(S.x, j);
+            const float fx = xi.x - xj.x, fy = xi.y - xj.y, fz = xi.z - xj.z;
+            if (!(fx * fx + fy * fy + fz * fz <= hh) || j == i) return;
+            const Pair p = pair_of(xx, xy, xz, xj, k);
+            double g, wq;
+            bool gnz;
+            if (!member_of(p, xi, xj, S.hD, k, g, wq, gnz)) return;
+            if (cnt < maxN && u == 0) stg(L, (size_t)slot_of(cnt), (uint32_t)j);
+            ++cnt;
+            ngr += gnz ? 1 : 0;
+            b.ws += wq;
+            if (M == DFSPH) {
+                const float4 vj = ld3o(S.v, (uint32_t)j);
+                b.sgx = fma(g, p.dx, b.sgx);
+                b.sgy = fma(g, p.dy, b.sgy);
+                b.sgz = fma(g, p.dz, b.sgz);
+                b.ssq = fma(g * g, p.r2, b.ssq);
+                b.dv = fma(g, (ux - (double)vj.x) * p.dx + (uy - (double)vj.y) * p.dy + (uz - (double)vj.z) * p.dz, b.dv);
+            }
+        });
+    }
+    // the list is padded with the particle itself up to the group's longest
+    // list rounded to 4
+    const int own = min(cnt, maxN);
+    int pad = min((own + 3) & ~3, maxN);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) pad = max(pad, __shfl_xor(pad, o));
+    if (lane == 0) spad[w] = pad;
+    __syncthreads();
+    pad = max(max(spad[0], spad[1]), max(spad[2], spad[3]));
+    const bool wantAdh = (S.flags & F_ADH) != 0;
+    const double rho0 = S.rho0D;
+    // boundary sums, 4 candidates at a time
+    if (bbase[9] > 0 && valid) {
+        int bs[9], be[9];
+#pragma unroll
+        for (int r = 0; r < 9; ++r) {
+            const int off = (r % 3 - 1) * nx + (r / 3 - 1) * nxny;
+            bs[r] = be[r] = 0;
+            if (bbase[r + 1] > bbase[r]) {
+                bs[r] = ldg(S.bCellStart, (size_t)(ci - 1 + off));
+                be[r] = ldg(S.bCellStart, (size_t)(ci + 2 + off));
+            }
+        }
+        static_for<9>([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
+            for (int b0 = bs[r]; b0 < be[r]; b0 += 4) {
+                const int t = min(b0 + u, be[r] - 1);
+                const float4 y = bStaged ? sb[t - bfirst[r] + bbase[r]] : ld4(S.xb, (size_t)t);
+                const float fx = xi.x - y.x, fy = xi.y - y.y, fz = xi.z - y.z;
+                const bool ok = (b0 + u < be[r]) & (fx * fx + fy * fy + fz * fz <= hh);
+                if (!__any(ok)) continue;
+                const Pair p = pair_of(xx, xy, xz, y, k);
+                const bool in = ok && p.q <= 1.0;
+                const double cb = in ? rho0 * (double)y.w : 0.0;
+                const double wq = in ? W_d(p.q, k) : 0.0;
+                const double g = in ? cb * G_d(p, k) : 0.0;
+                const double gs = (M == PCISPH && in) ? cb * Gs_d(p, k) : 0.0;
+                const double sa = (wantAdh && in && p.r2 > 0.0) ? cb * A_d(p.rl, k) * p.inv : 0.0;
+                static_for<4>([&](auto vc) {
+                    constexpr int v = decltype(vc)::value;
+                    const double dx = quad_lane<v>(p.dx), dy = quad_lane<v>(p.dy), dz = quad_lane<v>(p.dz);
+                    b.bw = fma(quad_lane<v>(cb), quad_lane<v>(wq), b.bw);
+                    const double gv = quad_lane<v>(g);
+                    b.bgx = fma(gv, dx, b.bgx);
+                    b.bgy = fma(gv, dy, b.bgy);
+                    b.bgz = fma(gv, dz, b.bgz);
+                    if (M == PCISPH) {
+                        const double gsv = quad_lane<v>(gs);
+                        b.sx2 = fma(gsv, dx, b.sx2);
+                        b.sy2 = fma(gsv, dy, b.sy2);
+                        b.sz2 = fma(gsv, dz, b.sz2);
+                    }
+                    if (wantAdh) {
+                        const double sav = quad_lane<v>(sa);
+                        b.ax = fma(sav, dx, b.ax);
+                        b.ay = fma(sav, dy, b.ay);
+                        b.az = fma(sav, dz, b.az);
+                    }
+                });
+            }
+        });
+    }
+    double e = 0.0;
+    if (M == PCISPH) {
+        if (pad + ns > maxN) shellLost = true;   // the padding reached the shell
+        shellLost = quad_bits(shellLost) != 0u;
+    }
+    if (valid) {
+        for (int q = own + u; q < pad; q += 4) stg(L, (size_t)slot_of(q), (uint32_t)i);
+        if (u == 0) {
+            if (M == PCISPH) stg(S.nsh, (size_t)i, (uint16_t)(shellLost ? 0xFFFF : ns));
+            if (pl == 0) stg(S.gcnt, (size_t)(i >> 6), (uint16_t)pad);
+            e = build_finish<M>(S, i, xi, vi, b, cnt, own, ngr);
+        }
+    }
+    if (M == DFSPH) {
+        if (u == 0) se[pl] = e;
+        __syncthreads();
+        if (w == 0) {
+            const double es = wave_sum(se[lane]);
+            if (lane == 0) ((gptr<double>)S.perm)[g0 >> 6] = es;
+        }
+        if (g0 == 0 && tid == 0) build_starts_divergence(S, fused);
     }
 }
 
@@ -2139,7 +2552,8 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict_
     if (KIND == FIN_DIV && ss->doneV) return;
     __shared__ double sh[kWaves];
     const double red = (KIND == FIN_DT || KIND == FIN_PCI) ? scene_partial_max(S.partial, S.nChunks, sh)
-                                                           : scene_partial_sum(S.partial, S.nChunks, sh);
+                       : KIND == FIN_DIV0 ? scene_wave_sum((const double*)S.perm, S.nChunks, sh)
+                                          : scene_partial_sum(S.partial, S.nChunks, sh);
     if (threadIdx.x != 0) return;
     if (KIND == FIN_DT) {
         // the density solve's loop counters start here (counted by FIN_DENS0)
@@ -2220,7 +2634,7 @@ __global__ __launch_bounds__(kBlock) void k_loop_end(const DevScene* __restrict_
         __syncthreads();   // every thread has read the flag before it is set
         if (!over && fused && !(END && KIND == LOOP_PCI)) over = loop_over<KIND>(S, ss, true, kLoopLast, sh);
         if (END && KIND == LOOP_DIV && fused) {
-            const double avg0 = scene_partial_sum((const double*)S.perm, S.nChunks, sh) / (double)S.n;
+            const double avg0 = scene_wave_sum((const double*)S.perm, S.nChunks, sh) / (double)S.n;
             if (threadIdx.x == 0) ss->avgErrV0 = avg0;
         }
         if (END && !over && tables.a) {
@@ -2620,6 +3034,17 @@ void launch_bvolume(hipStream_t st, const DevScene* T, int scene, int nb, float*
 }
 void launch_build(hipStream_t st, int method, const DevScene* T, const Chunk* C, int n, int fused) {
     if (!n) return;
+    // Up to where 4 lanes a particle are faster (us a step; one lane / four):
+    // WCSPH 125k particles 97.2 / 93.9, 157k 110.6 / 109.0, 195k 115.4 / 119.5;
+    // PCISPH 64k 200.8 / 191.3, 97k 223.3 / 222.6, 125k 240.0 / 247.6; DFSPH 64k
+    // 161.7 / 157.2, 97k 200.9 / 199.4, 125k 210.2 / 218.8.
+    if (n <= (method == WCSPH ? 512 : 320)) {
+        const int blocks = (n + 7) / 8 * 8 * kWaves;
+        if (method == DFSPH) hipLaunchKernelGGL(k_build_quad<DFSPH>, dim3(blocks), dim3(256), 0, st, T, C, n, fused);
+        else if (method == WCSPH) hipLaunchKernelGGL(k_build_quad<WCSPH>, dim3(blocks), dim3(256), 0, st, T, C, n, 0);
+        else hipLaunchKernelGGL(k_build_quad<PCISPH>, dim3(blocks), dim3(256), 0, st, T, C, n, 0);
+        return;
+    }
     if (method == DFSPH) LAUNCH(k_build<DFSPH>, n, st, T, C, fused);
     else if (method == WCSPH) LAUNCH(k_build<WCSPH>, n, st, T, C, 0);
     else LAUNCH(k_build<PCISPH>, n, st, T, C, 0);

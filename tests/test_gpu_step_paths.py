@@ -148,3 +148,107 @@ def test_cell_scan_in_one_and_two_launches(ctx, cells):
     assert same(g, t)
     g.close()
     t.close()
+
+
+def build_fields(scene):
+    out = fields(scene) + [scene.get(sphg.FIELD_NNB), scene.get(sphg.FIELD_NGRAD)]
+    if scene.params.method == sphg.DFSPH:
+        out += [scene.get(sphg.FIELD_ALPHA), scene.get(sphg.FIELD_DIVERR)]
+    if scene.params.method == sphg.PCISPH:
+        out += [scene.get(sphg.FIELD_NSH)]
+    counts, ids = scene.neighbors(((scene.params.max_neighbors or 96) + 3) & ~3)
+    return out + [counts, np.where(np.arange(ids.shape[1])[None, :] < counts[:, None], ids, 0)]
+
+
+def block_of(n, spacing, jitter, seed, at=0.06):
+    side = int(np.ceil(n ** (1.0 / 3.0)))
+    grid = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    rng = np.random.default_rng(seed)
+    return ((grid + rng.uniform(-jitter, jitter, grid.shape)) * spacing + at).astype(np.float32)
+
+
+@pytest.fixture(scope="module")
+def crowd(ctx):
+    """For each method a scene that brings a launch past the sizes at which a
+    particle has 4 lanes in the list build."""
+    out = {}
+    for m in METHODS:
+        spec = configs.small_scene(m, n_side=53, spacing=0.02)
+        out[m] = sphg.Scene(ctx, spec.params, spec.fluid, spec.boundary)
+    yield out
+    for s in out.values():
+        s.close()
+
+
+BUILDS = {
+    # name: (particles, spacing in 2r, jitter, boundary sampling in h, more)
+    "one": (1, 1.0, 0.0, 1.0, {}),
+    "group_less_one": (63, 1.0, 0.2, 1.0, {}),
+    "group": (64, 1.0, 0.2, 1.0, {}),
+    "group_and_one": (65, 1.0, 0.2, 1.0, {}),
+    "chunk_and_one": (257, 1.0, 0.3, 1.0, {}),
+    "disordered": (3000, 0.9, 0.5, 1.0, FORCES["adhesion"]),
+    "sparse": (700, 3.0, 0.9, 1.0, FORCES["adhesion"]),
+    # rows that do not fit the stage, boundary candidates that do not, lists
+    # of several hundred
+    "half_spacing": (1500, 0.5, 0.1, 1.0, dict(max_neighbors=500)),
+    "dense_walls": (1200, 1.0, 0.1, 0.25, FORCES["adhesion"]),
+    "few_slots": (500, 1.3, 0.1, 1.0, dict(max_neighbors=29)),
+}
+
+
+@pytest.mark.parametrize("method", METHODS)
+@pytest.mark.parametrize("name", sorted(BUILDS))
+def test_list_build_with_four_lanes_a_particle(ctx, crowd, method, name):
+    """A small scene's lists are built with 4 lanes a particle, in a large
+    launch with one: the same lists, sums and steps, bit for bit."""
+    n, gap, jitter, walls, more = BUILDS[name]
+    r = 0.01
+    p = configs.small_scene(method, n_side=2, spacing=2 * r, **more).params
+    p.domain_min, p.domain_max = (-0.1, -0.1, -0.1), (0.5, 0.4, 0.4)   # some leave it: cells clamped
+    x = block_of(n, gap * 2 * r, jitter, 11)
+    v = np.random.default_rng(2).uniform(-0.5, 0.5, x.shape).astype(np.float32)
+    b = sphg.sample_box((0.02, 0.02, 0.02), (0.6, 0.4, 0.45), walls * 4 * r)
+    alone, mixed = [sphg.Scene(ctx, p, x, b, v) for _ in range(2)]
+    most = 0
+    for _ in range(3):
+        alone.step(1)
+        ctx.batch_step([mixed, crowd[method]], 1)
+        for a, m in zip(build_fields(alone), build_fields(mixed)):
+            assert np.array_equal(a, m, equal_nan=True)
+        most = max(most, alone.get(sphg.FIELD_NNB).max())
+    assert most > (12 if name in ("disordered", "half_spacing", "dense_walls") else -1)
+    alone.close()
+    mixed.close()
+
+
+@pytest.mark.parametrize("method", METHODS)
+def test_four_lane_build_with_overflow_and_nan(ctx, crowd, method):
+    """Too many neighbors are refused alike, and a NaN position stays its own
+    particle's."""
+    r = 0.01
+    p = configs.small_scene(method, n_side=2, spacing=2 * r, max_neighbors=40).params
+    b = sphg.sample_box((0.0, 0.0, 0.0), (0.4, 0.4, 0.4), 4 * r)
+    x = block_of(700, 0.7 * 2 * r, 0.1, 3)
+    alone, mixed = [sphg.Scene(ctx, p, x, b) for _ in range(2)]
+    for step in (lambda: alone.step(1), lambda: ctx.batch_step([mixed, crowd[method]], 1)):
+        with pytest.raises(sphg.SphgError) as err:
+            step()
+        assert err.value.code == sphg.EOVERFLOW
+    assert alone.scalars().neighbor_overflow == mixed.scalars().neighbor_overflow > 40
+    assert np.array_equal(alone.get(sphg.FIELD_NNB), mixed.get(sphg.FIELD_NNB))
+    alone.close()
+    mixed.close()
+    p.max_neighbors = 0
+    x = block_of(300, 2 * r, 0.1, 4)
+    alone, mixed = [sphg.Scene(ctx, p, x, b) for _ in range(2)]
+    x = x.copy()
+    x[77, 1] = np.nan
+    for s in (alone, mixed):
+        s.set_state(x, np.zeros_like(x))
+    alone.step(1)
+    ctx.batch_step([mixed, crowd[method]], 1)
+    assert all(np.array_equal(a, m, equal_nan=True) for a, m in zip(build_fields(alone), build_fields(mixed)))
+    assert np.isfinite(np.delete(alone.get(sphg.FIELD_X), 77, 0)).all()
+    alone.close()
+    mixed.close()
