@@ -545,7 +545,7 @@ int self_tables(sphg_scene* s) {
 // Finalize kernel of a reduction (one block per scene).
 void finalize(sphg_ctx* ctx, Batch& B, const DevScene* T, int kind) {
     Scope s(&ctx->prof, ctx->stream, K_FINALIZE);
-    launch_finalize(ctx->stream, kind, T, (int)B.scenes.size(), ctx->dActive);
+    launch_finalize(ctx->stream, kind, T, (int)B.scenes.size(), ctx->dActive, B.nP);
 }
 
 // Whether iteration `it` of a loop is to be launched.  Below `ahead` --

@@ -93,8 +93,8 @@ struct Scalars {
     unsigned listOver;          // the same for the lists built last (reset by the key pass before each build)
     unsigned nActive;           // active particles (the emitters raise it)
     unsigned shellBad;          // PCISPH: this step's shell lists cannot stand in for the 27-cell walk
-    unsigned maxD2, maxD2Prev;  // PCISPH: largest squared predicted displacement (FP32 bits) of this
-                                // step so far and of the previous step, which sizes this step's shell
+    unsigned maxD2Prev;         // PCISPH: largest squared predicted displacement (FP32 bits) of the
+                                // previous step, which sizes this step's shell
     unsigned shellSteps, walkSteps;  // PCISPH: steps whose predicted densities used the shell lists /
                                      // took the 27-cell walk for every particle
     unsigned d0Valid;           // DFSPH: d0 holds the divergence of the current velocities (written by

@@ -18,6 +18,9 @@ enum LoopKind { LOOP_DENS, LOOP_DIV, LOOP_PCI };
 // sweeps themselves (`fused`), each block adding up the chunk partials; above
 // that the partials are too many for every block, and finalize kernels do it.
 constexpr int kFusedLoopChunks = 2048;
+// Launches of up to so many chunks give the list build and the PCISPH density
+// sweep 4 lanes a particle (figures: launch_build, launch_pci_density).
+constexpr int kQuadChunks = 320, kQuadChunksWcsph = 512, kQuadPciChunks = 768;
 
 // begin_active: also the start of a WCSPH or PCISPH step, counting the
 // scenes whose pressure loop runs in begin_active[0] (null: keys only)
@@ -45,7 +48,7 @@ void launch_df_predict(hipStream_t st, const DevScene* T, const Chunk* C, int nc
 void launch_df_vel(hipStream_t st, int mode, const DevScene* T, const Chunk* C, int nchunks, int iter, int fused);
 void launch_df_err(hipStream_t st, int mode, const DevScene* T, const Chunk* C, int nchunks, int fused);
 // kind: 0 dt, 1 density (before loop), 2 density, 3 divergence (before loop), 4 divergence, 5 PCISPH
-void launch_finalize(hipStream_t st, int kind, const DevScene* T, int nscenes, int* active);
+void launch_finalize(hipStream_t st, int kind, const DevScene* T, int nscenes, int* active, int nchunks);
 // also clears active[0..1] for the divergence solve
 void launch_df_positions(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int* active, int fused,
                          int ahead);

@@ -109,6 +109,8 @@ __device__ inline double block_sum(double v, double* sh) {
     __syncthreads();
     return r;
 }
+// BT: the block's threads.
+template <int BT = kBlock>
 __device__ inline double block_max(double v, double* sh) {
     v = wave_max(v);
     const int w = threadIdx.x >> 6;
@@ -116,7 +118,7 @@ __device__ inline double block_max(double v, double* sh) {
     __syncthreads();
     double r = sh[0];
 #pragma unroll
-    for (int k = 1; k < kWaves; ++k) r = fmax(r, sh[k]);
+    for (int k = 1; k < BT / 64; ++k) r = fmax(r, sh[k]);
     __syncthreads();
     return r;
 }
@@ -153,16 +155,17 @@ __device__ inline double scene_wave_sum(const double* wp, int n, double* sh) {
     }
     return block_sum(acc, sh);
 }
+template <int BT = kBlock>
 __device__ inline double scene_partial_max(const double* partial, int n, double* sh) {
     double acc = -1e300;
-    for (int b = threadIdx.x; b < n; b += kBlock * kPartU) {
+    for (int b = threadIdx.x; b < n; b += BT * kPartU) {
         double v[kPartU];
 #pragma unroll
-        for (int u = 0; u < kPartU; ++u) v[u] = (b + u * kBlock < n) ? ldg(partial, (size_t)(b + u * kBlock)) : -1e300;
+        for (int u = 0; u < kPartU; ++u) v[u] = (b + u * BT < n) ? ldg(partial, (size_t)(b + u * BT)) : -1e300;
 #pragma unroll
         for (int u = 0; u < kPartU; ++u) acc = fmax(acc, v[u]);
     }
-    return block_max(acc, sh);
+    return block_max<BT>(acc, sh);
 }
 
 // ------------------------------------------------ loop control
@@ -199,15 +202,31 @@ constexpr int kLoopLast = 1 << 30;   // idx of the launches behind a loop
 // its density sweep decides and writes partials in one launch.  The second is
 // the sort's scratch, which the loop does not need.
 __device__ inline double* pci_partial(const DevScene& S, int it) { return (it & 1) ? (double*)S.perm : S.partial; }
+// The density sweep with 4 lanes a particle (launches of at most
+// kQuadPciChunks chunks) leaves a partial per 64-particle group, both buffers in the scratch.
+__device__ inline double* pci_wide_partial(const DevScene& S, int it) {
+    return (double*)S.perm + (size_t)(it & 1) * S.nChunks * kWaves;
+}
+// The largest squared predicted displacement of each 64-particle group over a
+// PCISPH step's iterations, behind the partials in the scratch; the next
+// step's start reads it, before the sort.  (One atomic maximum per block
+// into the scene's scalars was free with 1,371 blocks, but with the 4 times as
+// many of 4 lanes a particle it took the step of 350,835 particles from 461 to
+// 1,434 us.)
+__device__ inline float* pci_displacements(const DevScene& S) {
+    return (float*)((double*)S.perm + (size_t)2 * S.nChunks * kWaves);
+}
 // Whether the loop has ended, decided by every block alike (block-uniform;
 // called where ended_before(done, idx) is false).
-template <int KIND>
+template <int KIND, int BT = kBlock>
 __device__ inline bool loop_over(const DevScene& S, Scalars* ss, bool firstChunk, int idx, double* sh) {
     const int it = KIND == LOOP_DIV ? ss->itV : ss->it;
     // below the minimum the error does not matter
     if (it < (KIND == LOOP_DIV ? S.minItV : S.minIt) && it < S.maxIt) return false;
-    const double err = KIND == LOOP_PCI ? scene_partial_max(pci_partial(S, it - 1), S.nChunks, sh)
-                                        : scene_partial_sum(S.partial, S.nChunks, sh) / (double)S.n;
+    double err;
+    if (KIND != LOOP_PCI) err = scene_partial_sum(S.partial, S.nChunks, sh) / (double)S.n;
+    else if (S.nChunks <= kQuadPciChunks) err = scene_partial_max<BT>(pci_wide_partial(S, it - 1), S.nChunks * kWaves, sh);
+    else err = scene_partial_max<BT>(pci_partial(S, it - 1), S.nChunks, sh);
     if (loop_goes_on<KIND>(S, ss, it, err)) return false;
     if (firstChunk && threadIdx.x == 0) loop_ended<KIND>(ss, it, err, idx);
     return true;
@@ -602,12 +621,28 @@ __device__ inline void step_begin(const DevScene& S, const Chunk& c, int i, int*
         S.p[i] = 0.0f;
         S.pacc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    if (c.begin == 0 && threadIdx.x == 0) {
-        Scalars* ss = S.ss;
+    if (c.begin != 0) return;
+    Scalars* ss = S.ss;
+    // the previous step's largest predicted displacement (none if no
+    // iteration of it ran)
+    double d2 = 0.0;
+    if (S.pciShell && ss->it > 0) {
+        __shared__ double sh[kWaves];
+        float m = 0.f;
+        const float* const disp = pci_displacements(S);
+        for (int t = threadIdx.x; t < S.nChunks * kWaves; t += kBlock * 16) {
+            float q[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) q[u] = (t + u * kBlock < S.nChunks * kWaves) ? ldg(disp, (size_t)(t + u * kBlock)) : 0.f;
+#pragma unroll
+            for (int u = 0; u < 16; ++u) m = fmaxf(m, q[u]);
+        }
+        d2 = block_max((double)m, sh);
+    }
+    if (threadIdx.x == 0) {
         ss->steps += 1u;
         ss->shellBad = 0u;
-        ss->maxD2Prev = ss->maxD2;
-        ss->maxD2 = 0u;
+        ss->maxD2Prev = __float_as_uint((float)d2);
         if (S.method == PCISPH) {
             ss->it = 0;
             const bool run = (ss->maxDensErr > S.eta || 0 < S.minIt) && 0 < S.maxIt;
@@ -938,10 +973,11 @@ struct BuildSums {
 };
 
 // What a particle's list and sums give, stored: `cnt` members, `own` of them
-// in the list.  Returns its share of the average divergence error (DFSPH).
+// in the list; nearBound (PCISPH): its cells hold boundary particles.  Returns
+// its share of the average divergence error (DFSPH).
 template <int M>
 __device__ inline double build_finish(const DevScene& S, int i, const float4& xi, const float4& vi, const BuildSums& b,
-                                      int cnt, int own, int ngr) {
+                                      int cnt, int own, int ngr, bool nearBound) {
     const KCoefD& k = S.kd;
     const double rho0 = S.rho0D, m = S.mD;
     if (cnt > S.maxNbr) {
@@ -986,7 +1022,7 @@ __device__ inline double build_finish(const DevScene& S, int i, const float4& xi
         const float4 v = ld4(S.v, i);
         st4(S.aux, i, make_float4(v.x, v.y, v.z, (float)(m / rho)));
     } else {
-        st4(S.gbs, i, make_float4((float)b.sx2, (float)b.sy2, (float)b.sz2, 0.f));
+        st4(S.gbs, i, make_float4((float)b.sx2, (float)b.sy2, (float)b.sz2, nearBound ? 1.f : 0.f));
     }
     return 0.0;
 }
@@ -1316,6 +1352,7 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
     // the boundary survivors use the free slots between the list and the shell
     const int room = max(0, maxN - own - ((M == PCISPH && !shellLost) ? ns : 0));
     int nbc = 0;
+    bool nearBound = false;
     {
         // the 9 rows' ranges first, then 4 candidates' loads at a time: a
         // wait for a load also waits for the survivor stores before it
@@ -1325,6 +1362,10 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
             const int off = (r % 3 - 1) * nx + (r / 3 - 1) * nxny;
             bs[r] = ldg(S.bCellStart, (size_t)(ci - 1 + off));
             be[r] = ldg(S.bCellStart, (size_t)(ci + 2 + off));
+        }
+        if (M == PCISPH) {
+#pragma unroll
+            for (int r = 0; r < 9; ++r) nearBound |= be[r] > bs[r];
         }
 #pragma unroll 1
         for (int r = 0; r < 9; ++r) {
@@ -1368,7 +1409,7 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
         stg(S.nsh, (size_t)i, (uint16_t)(shellLost ? 0xFFFF : ns));
     }
     if ((i & 63) == 0) stg(S.gcnt, (size_t)(i >> 6), (uint16_t)pad);
-    e = build_finish<M>(S, i, xi, vi, b, cnt, own, ngr);
+    e = build_finish<M>(S, i, xi, vi, b, cnt, own, ngr, nearBound);
     }
     if (M == DFSPH) {
         const double es = wave_sum(e);
@@ -1675,6 +1716,7 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
     const bool wantAdh = (S.flags & F_ADH) != 0;
     const double rho0 = S.rho0D;
     // boundary sums, 4 candidates at a time
+    bool nearBound = false;
     if (bbase[9] > 0 && valid) {
         int bs[9], be[9];
 #pragma unroll
@@ -1686,6 +1728,8 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
                 be[r] = ldg(S.bCellStart, (size_t)(ci + 2 + off));
             }
         }
+#pragma unroll
+        for (int r = 0; r < 9; ++r) nearBound |= be[r] > bs[r];
         static_for<9>([&](auto rc) {
             constexpr int r = decltype(rc)::value;
             for (int b0 = bs[r]; b0 < be[r]; b0 += 4) {
@@ -1735,7 +1779,7 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
         if (u == 0) {
             if (M == PCISPH) stg(S.nsh, (size_t)i, (uint16_t)(shellLost ? 0xFFFF : ns));
             if (pl == 0) stg(S.gcnt, (size_t)(i >> 6), (uint16_t)pad);
-            e = build_finish<M>(S, i, xi, vi, b, cnt, own, ngr);
+            e = build_finish<M>(S, i, xi, vi, b, cnt, own, ngr, nearBound);
         }
     }
     if (M == DFSPH) {
@@ -2339,6 +2383,66 @@ __global__ __launch_bounds__(kBlock) void k_df_positions(const DevScene* __restr
 // included), then updatePressure (:249-295): p_i += delta max(0, rho_i -
 // rho0); the scene's max relative error decides the loop (:365), counting
 // this iteration as done (its pressure acceleration always follows).
+// The nine rows of a particle's boundary (or fluid) candidates.
+struct Rows {
+    int s[9], e[9];
+};
+__device__ inline Rows rows_of(const int* start, int c, int nx, int nxny) {
+    Rows o;
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+        const int off = (r % 3 - 1) * nx + (r / 3 - 1) * nxny;
+        o.s[r] = ldg(start, (size_t)(c - 1 + off));
+        o.e[r] = ldg(start, (size_t)(c + 2 + off));
+    }
+    return o;
+}
+// x* = x + d with d = v* dt held separately: x*_i - x*_j = (x_i - x_j) +
+// (d_i - d_j) keeps FP64 accuracy from FP32 storage.
+struct Predicted {
+    double px, py, pz, ex, ey, ez;
+};
+// W at the predicted distance to a particle at y + d, zero past h.
+__device__ inline double predicted_w(const Predicted& a, const float4& y, const float4& d, const KCoefD& k) {
+    const double dx = (a.px - (double)y.x) + (a.ex - (double)d.x);
+    const double dy = (a.py - (double)y.y) + (a.ey - (double)d.y);
+    const double dz = (a.pz - (double)y.z) + (a.ez - (double)d.z);
+    const double r2 = dx * dx + dy * dy + dz * dz;
+    return r2 <= k.hhi2 ? W_d(sqrt(r2) * k.invh, k) : 0.0;
+}
+// The same to a boundary particle.
+__device__ inline double predicted_wb(const Predicted& a, const float4& y, const KCoefD& k) {
+    const double dx = (a.px - (double)y.x) + a.ex, dy = (a.py - (double)y.y) + a.ey, dz = (a.pz - (double)y.z) + a.ez;
+    const double r2 = dx * dx + dy * dy + dz * dz;
+    return r2 <= k.hhi2 ? W_d(sqrt(r2) * k.invh, k) : 0.0;
+}
+// What the sums give: the density, p_i and p_i / rho_i^2; returns the error.
+__device__ inline double pci_pressure(const DevScene& S, int i, const float4& xi, double ws, double bw) {
+    const double rho0 = S.rho0D;
+    const double drho = (S.mD * ws + rho0 * bw) - rho0;
+    const double rho = rho0 + drho;
+    S.drho[i] = (float)drho;
+    const double err = fmax(0.0, drho);
+    const double pr = (double)S.p[i] + S.pciDeltaD * err;
+    S.p[i] = (float)pr;
+    S.xk[i] = make_float4(xi.x, xi.y, xi.z, (float)(pr / (rho * rho)));
+    return err / rho0;
+}
+
+// A group's largest squared displacement, kept over the step's iterations (one
+// lane of each wavefront of the group stores it).
+__device__ inline void store_displacement(const DevScene& S, int group, double d2, int iter) {
+    if ((threadIdx.x & 63) != 0) return;
+    float* const p = pci_displacements(S) + group;
+    *p = iter == 0 ? (float)d2 : fmaxf(*p, (float)d2);
+}
+
+// Every candidate of the 27 cells that can come within h at x* is the
+// particle itself, a list member (|x_i - x_j| <= h) or a shell member (<= h +
+// skin): the walk's terms in another order.  Shell member s is in slot maxN -
+// 1 - s.  ~60 FP64 instructions a term (a square root among them) bound it in
+// a large scene; the next entries are requested before the current ones' data
+// is used, and particles whose cells hold no boundary skip its 9 rows.
 // `fused`: the sweep decides whether its iteration runs (loop_over).
 __global__ __launch_bounds__(kBlock) void k_pci_density(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
                                                         int iter, int fused) {
@@ -2356,84 +2460,167 @@ __global__ __launch_bounds__(kBlock) void k_pci_density(const DevScene* __restri
     double e = 0.0;
     double dd = 0.0;   // squared predicted displacement, for the next step's shell width
     if (i < S.n) {
-        // x* = x + d with d = v* dt held separately: x*_i - x*_j =
-        // (x_i - x_j) + (d_i - d_j) keeps FP64 accuracy from FP32 storage
-        const float4 xi = S.x[i];
-        const float4 di = S.xs[i];
-        dd = (double)(di.x * di.x + di.y * di.y + di.z * di.z);
-        const double px = xi.x, py = xi.y, pz = xi.z;
-        const double ex = di.x, ey = di.y, ez = di.z;
-        const int ci = S.cell[i];
+        const float4 xi = ld4(S.x, (size_t)i);
+        const float4 di = ld4(S.xs, (size_t)i);
+        const int ci = ldg(S.cell, (size_t)i);
+        const float nearBound = ldg(&S.gbs[i].w, 0);
         const int nx = S.nx, nxny = S.nx * S.ny;
+        dd = (double)(di.x * di.x + di.y * di.y + di.z * di.z);
+        const Predicted a{xi.x, xi.y, xi.z, di.x, di.y, di.z};
         double ws = 0.0;
-        auto term = [&](const XV& q) {
-            const double dx = (px - (double)q.x.x) + (ex - (double)q.v.x);
-            const double dy = (py - (double)q.x.y) + (ey - (double)q.v.y);
-            const double dz = (pz - (double)q.x.z) + (ez - (double)q.v.z);
-            const double r2 = dx * dx + dy * dy + dz * dz;
-            if (r2 <= k.hhi2) ws += W_d(sqrt(r2) * k.invh, k);
-        };
         auto xv = [&](uint32_t j) { XV r; r.x = ld4o(S.x, j); r.v = ld4o(S.xs, j); return r; };
-        const int nsi = useShell ? (int)S.nsh[i] : 0xFFFF;
+        const int nsi = useShell ? (int)ldg(S.nsh, (size_t)i) : 0xFFFF;
         if (nsi != 0xFFFF) {
-            // every candidate of the 27 cells that can come within h at x*
-            // is the particle itself, a list member (|x_i - x_j| <= h) or a
-            // shell member (<= h + skin): the same terms in another order
             ws = W_d(0.0, k);
             const uint32_t* L = list_of(S, i);
-            const int own = S.nnb[i];
-            for (int q0 = 0; q0 < own; q0 += 4) {
-                const v4u b = ld_block(L, q0 >> 2);
-                const uint32_t jj[4] = {b.x, q0 + 1 < own ? b.y : b.x, q0 + 2 < own ? b.z : b.x,
-                                        q0 + 3 < own ? b.w : b.x};
-                XV d[4];
+            // `count` entries in list order, from the first slot up or the
+            // last one down
+            auto run = [&](int count, bool down) {
+                const int last = (S.maxNbr >> 2) - 1;
+                if (count == 0) return;
+                v4u bn = ld_block(L, down ? last : 0);
+                for (int q0 = 0; q0 < count; q0 += 4) {
+                    const uint32_t j0 = down ? bn.w : bn.x;
+                    const uint32_t jj[4] = {j0, q0 + 1 < count ? (down ? bn.z : bn.y) : j0,
+                                            q0 + 2 < count ? (down ? bn.y : bn.z) : j0,
+                                            q0 + 3 < count ? (down ? bn.x : bn.w) : j0};
+                    XV d[4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) d[u] = xv(jj[u]);
+                    for (int u = 0; u < 4; ++u) d[u] = xv(jj[u]);
+                    const int nb = (q0 + 4 < count ? q0 + 4 : q0) >> 2;
+                    bn = ld_block(L, down ? last - nb : nb);
+                    asm volatile("" ::: "memory");
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (q0 + u < own) term(d[u]);
-            }
-            // shell member s is in slot maxN - 1 - s: block maxN/4 - 1 - s/4,
-            // component 3 - s%4
-            const int maxN = S.maxNbr;
-            for (int s0 = 0; s0 < nsi; s0 += 4) {
-                const v4u b = ld_block(L, (maxN >> 2) - 1 - (s0 >> 2));
-                const uint32_t jj[4] = {b.w, s0 + 1 < nsi ? b.z : b.w, s0 + 2 < nsi ? b.y : b.w,
-                                        s0 + 3 < nsi ? b.x : b.w};
-                XV d[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) d[u] = xv(jj[u]);
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (s0 + u < nsi) term(d[u]);
-            }
+                    for (int u = 0; u < 4; ++u)
+                        if (q0 + u < count) ws += predicted_w(a, d[u].x, d[u].v, k);
+                }
+            };
+            run((int)ldg(S.nnb, (size_t)i), false);
+            run(nsi, true);
         } else {
             walk27x4(S.cellStart, ci, nx, nxny, [&](int j) { return xv((uint32_t)j); },
-                     [&](int, const XV& q) { term(q); });
+                     [&](int, const XV& q) { ws += predicted_w(a, q.x, q.v, k); });
         }
         double bw = 0.0;
-        walk27x4(S.bCellStart, ci, nx, nxny, [&](int b) { return ld4(S.xb, b); },
-                 [&](int, const float4& y) {
-                     const double dx = (px - (double)y.x) + ex, dy = (py - (double)y.y) + ey, dz = (pz - (double)y.z) + ez;
-                     const double r2 = dx * dx + dy * dy + dz * dz;
-                     if (r2 <= k.hhi2) bw += (double)y.w * W_d(sqrt(r2) * k.invh, k);
-                 });
-        const double rho0 = S.rho0D;
-        const double drho = (S.mD * ws + rho0 * bw) - rho0;
-        const double rho = rho0 + drho;
-        S.drho[i] = (float)drho;
-        const double err = fmax(0.0, drho);
-        const double pr = (double)S.p[i] + S.pciDeltaD * err;
-        S.p[i] = (float)pr;
-        S.xk[i] = make_float4(xi.x, xi.y, xi.z, (float)(pr / (rho * rho)));
-        e = err / rho0;
+        if (nearBound != 0.f)
+            walk27x4(S.bCellStart, ci, nx, nxny, [&](int b) { return ld4(S.xb, b); },
+                     [&](int, const float4& y) { bw += (double)y.w * predicted_wb(a, y, k); });
+        e = pci_pressure(S, i, xi, ws, bw);
     }
     const double bm = block_max(e, sh);
     if (threadIdx.x == 0) part[c.begin / kBlock] = bm;
-    if (S.pciShell) {
-        // the max is order-free: one atomic per block on non-negative FP32 bits
-        const double dm = block_max(dd, sh);
-        if (threadIdx.x == 0) atomicMax(&S.ss->maxD2, __float_as_uint((float)dm));
+    if (S.pciShell) store_displacement(S, i >> 6, wave_max(dd), iter);
+}
+
+// The same with 4 lanes a particle, a block per list group, for small
+// launches (see k_build_quad): a lane takes every 4th entry and the terms are
+// added in list order.  PCISPH, 4,845 particles: 28 -> 13 us a launch, the step
+// 204 -> 144.
+template <int V>
+__device__ inline double quad_sum(double s, double t) {
+    s += quad_lane<V>(t);
+    if constexpr (V < 3) return quad_sum<V + 1>(s, t);
+    else return s;
+}
+__global__ __launch_bounds__(256) void k_pci_density_quad(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                          int nchunks, int iter, int fused) {
+    const int slot = ((int)(blockIdx.x >> 3) / kWaves) * 8 + (int)(blockIdx.x & 7), sub = (int)(blockIdx.x >> 3) % kWaves;
+    if (slot >= nchunks) return;
+    const Chunk c = chunk_at(C, kBlock, slot, nchunks);
+    const DevScene& S = T[c.scene];
+    if (S.stall) return;
+    Scalars* ss = S.ss;
+    if (ended_before(ss->done, iter + 1)) return;
+    __shared__ double sh[4];
+    const int tid = threadIdx.x, lane = tid & 63, u = lane & 3;
+    const int g0 = c.begin + sub * kGroup;
+    const int i = g0 + (tid >> 2);
+    if (fused && loop_over<LOOP_PCI, 256>(S, ss, g0 == 0, iter + 1, sh)) return;
+    const int il = min(i, S.n - 1);
+    const KCoefD k = S.kd;
+    const bool useShell = S.pciShell && ss->shellBad == 0u;
+    double e = 0.0, dd = 0.0;
+    if (i < S.n) {
+        const float4 xi = ld4(S.x, (size_t)il);
+        const float4 di = ld4(S.xs, (size_t)il);
+        const int ci = ldg(S.cell, (size_t)il);
+        const int nx = S.nx, nxny = S.nx * S.ny;
+        const Rows br = rows_of(S.bCellStart, ci, nx, nxny);
+        dd = (double)(di.x * di.x + di.y * di.y + di.z * di.z);
+        const Predicted a{xi.x, xi.y, xi.z, di.x, di.y, di.z};
+        const int nsi = useShell ? (int)ldg(S.nsh, (size_t)i) : 0xFFFF;
+        double ws = 0.0;
+        if (nsi != 0xFFFF) {
+            ws = W_d(0.0, k);
+            const uint32_t* const L = list_of(S, i);
+            const int maxN = S.maxNbr;
+            // two entries a lane at a time
+            auto run = [&](int count, bool down) {
+                auto at = [&](int q) {
+                    const int t = q < count ? q : (q & 3) < count ? (q & 3) : 0;
+                    return ldg(L, (size_t)slot_of(down ? maxN - 1 - t : t));
+                };
+                if (count == 0) return;
+                uint32_t jn[2] = {at(u), at(4 + u)};
+                for (int q0 = 0; q0 < count; q0 += 8) {
+                    float4 x[2], d[2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        x[h] = ld4o(S.x, jn[h]);
+                        d[h] = ld4o(S.xs, jn[h]);
+                    }
+                    jn[0] = at(q0 + 8 + u);
+                    jn[1] = at(q0 + 12 + u);
+                    asm volatile("" ::: "memory");
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        ws = quad_sum<0>(ws, q0 + 4 * h + u < count ? predicted_w(a, x[h], d[h], k) : 0.0);
+                }
+            };
+            run((int)ldg(S.nnb, (size_t)i), false);
+            run(nsi, true);
+        } else {
+            const Rows fr = rows_of(S.cellStart, ci, nx, nxny);
+            static_for<9>([&](auto rc) {
+                constexpr int r = decltype(rc)::value;
+                for (int j0 = fr.s[r]; j0 < fr.e[r]; j0 += 4) {
+                    const uint32_t j = (uint32_t)min(j0 + u, fr.e[r] - 1);
+                    const float4 x = ld4o(S.x, j), d = ld4o(S.xs, j);
+                    ws = quad_sum<0>(ws, j0 + u < fr.e[r] ? predicted_w(a, x, d, k) : 0.0);
+                }
+            });
+        }
+        double bw = 0.0;
+        static_for<9>([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
+            for (int b0 = br.s[r]; b0 < br.e[r]; b0 += 8) {
+                float4 y[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) y[h] = ld4(S.xb, (size_t)min(b0 + 4 * h + u, br.e[r] - 1));
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const double w = b0 + 4 * h + u < br.e[r] ? predicted_wb(a, y[h], k) : 0.0, vb = y[h].w;
+                    static_for<4>([&](auto vc) {
+                        constexpr int v = decltype(vc)::value;
+                        bw = fma(quad_lane<v>(vb), quad_lane<v>(w), bw);
+                    });
+                }
+            }
+        });
+        if (u == 0) e = pci_pressure(S, i, xi, ws, bw);
+    }
+    // one partial a group
+    e = wave_max(e);
+    dd = wave_max(dd);
+    __shared__ double sm[8];
+    if (lane == 0) {
+        sm[tid >> 6] = e;
+        sm[4 + (tid >> 6)] = dd;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        pci_wide_partial(S, fused ? ss->it : 0)[g0 >> 6] = fmax(fmax(sm[0], sm[1]), fmax(sm[2], sm[3]));
+        if (S.pciShell) store_displacement(S, g0 >> 6, fmax(fmax(sm[4], sm[5]), fmax(sm[6], sm[7])), iter);
     }
 }
 
@@ -2541,8 +2728,9 @@ __global__ __launch_bounds__(kBlock) void k_pci_integrate(const DevScene* __rest
 // scenes still iterating, active[1] is the largest iteration count reached.
 enum FinKind { FIN_DT = 0, FIN_DENS0, FIN_DENS, FIN_DIV0, FIN_DIV, FIN_PCI };
 
+// wide: the PCISPH partials are one a group (k_pci_density_quad)
 template <int KIND>
-__global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict__ T, int nscenes, int* active) {
+__global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict__ T, int nscenes, int* active, int wide) {
     const int sc = blockIdx.x;
     if (sc >= nscenes) return;
     const DevScene& S = T[sc];
@@ -2551,7 +2739,8 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict_
     if ((KIND == FIN_DENS || KIND == FIN_PCI) && ss->done) return;
     if (KIND == FIN_DIV && ss->doneV) return;
     __shared__ double sh[kWaves];
-    const double red = (KIND == FIN_DT || KIND == FIN_PCI) ? scene_partial_max(S.partial, S.nChunks, sh)
+    const double red = (KIND == FIN_PCI && wide) ? scene_partial_max(pci_wide_partial(S, 0), S.nChunks * kWaves, sh)
+                       : (KIND == FIN_DT || KIND == FIN_PCI) ? scene_partial_max(S.partial, S.nChunks, sh)
                        : KIND == FIN_DIV0 ? scene_wave_sum((const double*)S.perm, S.nChunks, sh)
                                           : scene_partial_sum(S.partial, S.nChunks, sh);
     if (threadIdx.x != 0) return;
@@ -3038,7 +3227,7 @@ void launch_build(hipStream_t st, int method, const DevScene* T, const Chunk* C,
     // WCSPH 125k particles 97.2 / 93.9, 157k 110.6 / 109.0, 195k 115.4 / 119.5;
     // PCISPH 64k 200.8 / 191.3, 97k 223.3 / 222.6, 125k 240.0 / 247.6; DFSPH 64k
     // 161.7 / 157.2, 97k 200.9 / 199.4, 125k 210.2 / 218.8.
-    if (n <= (method == WCSPH ? 512 : 320)) {
+    if (n <= (method == WCSPH ? kQuadChunksWcsph : kQuadChunks)) {
         const int blocks = (n + 7) / 8 * 8 * kWaves;
         if (method == DFSPH) hipLaunchKernelGGL(k_build_quad<DFSPH>, dim3(blocks), dim3(256), 0, st, T, C, n, fused);
         else if (method == WCSPH) hipLaunchKernelGGL(k_build_quad<WCSPH>, dim3(blocks), dim3(256), 0, st, T, C, n, 0);
@@ -3085,22 +3274,27 @@ void launch_df_err(hipStream_t st, int mode, const DevScene* T, const Chunk* C, 
     else if (mode == 1) LAUNCH(k_df_err<1>, n, st, T, C, fused);
     else LAUNCH(k_df_err<3>, n, st, T, C, fused);
 }
-void launch_finalize(hipStream_t st, int kind, const DevScene* T, int nscenes, int* active) {
+void launch_finalize(hipStream_t st, int kind, const DevScene* T, int nscenes, int* active, int nchunks) {
     if (!nscenes) return;
     switch (kind) {
-        case FIN_DT: LAUNCH(k_finalize<FIN_DT>, nscenes, st, T, nscenes, active); break;
-        case FIN_DENS0: LAUNCH(k_finalize<FIN_DENS0>, nscenes, st, T, nscenes, active); break;
-        case FIN_DENS: LAUNCH(k_finalize<FIN_DENS>, nscenes, st, T, nscenes, active); break;
-        case FIN_DIV0: LAUNCH(k_finalize<FIN_DIV0>, nscenes, st, T, nscenes, active); break;
-        case FIN_DIV: LAUNCH(k_finalize<FIN_DIV>, nscenes, st, T, nscenes, active); break;
-        default: LAUNCH(k_finalize<FIN_PCI>, nscenes, st, T, nscenes, active); break;
+        case FIN_DT: LAUNCH(k_finalize<FIN_DT>, nscenes, st, T, nscenes, active, 0); break;
+        case FIN_DENS0: LAUNCH(k_finalize<FIN_DENS0>, nscenes, st, T, nscenes, active, 0); break;
+        case FIN_DENS: LAUNCH(k_finalize<FIN_DENS>, nscenes, st, T, nscenes, active, 0); break;
+        case FIN_DIV0: LAUNCH(k_finalize<FIN_DIV0>, nscenes, st, T, nscenes, active, 0); break;
+        case FIN_DIV: LAUNCH(k_finalize<FIN_DIV>, nscenes, st, T, nscenes, active, 0); break;
+        default: LAUNCH(k_finalize<FIN_PCI>, nscenes, st, T, nscenes, active, nchunks <= kQuadPciChunks ? 1 : 0); break;
     }
 }
 void launch_df_positions(hipStream_t st, const DevScene* T, const Chunk* C, int n, int* active, int fused, int ahead) {
     if (n) LAUNCH(k_df_positions, n, st, T, C, active, fused, ahead);
 }
 void launch_pci_density(hipStream_t st, const DevScene* T, const Chunk* C, int n, int iter, int fused) {
-    if (n) LAUNCH(k_pci_density, n, st, T, C, iter, fused);
+    if (!n) return;
+    // (us a step, one lane / four: 64,000 particles 191 / 156, 97k 221 / 199, 195k
+    // 283 / 281, 373k 427 / 453)
+    if (n <= kQuadPciChunks)
+        hipLaunchKernelGGL(k_pci_density_quad, dim3((n + 7) / 8 * 8 * kWaves), dim3(256), 0, st, T, C, n, iter, fused);
+    else LAUNCH(k_pci_density, n, st, T, C, iter, fused);
 }
 void launch_pci_pacc(hipStream_t st, const DevScene* T, const Chunk* C, int n, int iter, int fused) {
     if (n) LAUNCH(k_pci_pacc, n, st, T, C, iter, fused);

@@ -170,10 +170,10 @@ def block_of(n, spacing, jitter, seed, at=0.06):
 @pytest.fixture(scope="module")
 def crowd(ctx):
     """For each method a scene that brings a launch past the sizes at which a
-    particle has 4 lanes in the list build."""
+    particle has 4 lanes in the list build and the PCISPH density sweep."""
     out = {}
     for m in METHODS:
-        spec = configs.small_scene(m, n_side=53, spacing=0.02)
+        spec = configs.small_scene(m, n_side=59, spacing=0.02)
         out[m] = sphg.Scene(ctx, spec.params, spec.fluid, spec.boundary)
     yield out
     for s in out.values():
