@@ -140,21 +140,6 @@ __device__ inline double scene_partial_sum(const double* partial, int n, double*
     }
     return block_sum(acc, sh);
 }
-// The same over n chunks whose wavefronts' sums are in `wp`, kWaves a chunk:
-// a chunk's sum is formed as block_sum forms it.
-__device__ inline double scene_wave_sum(const double* wp, int n, double* sh) {
-    double acc = 0.0;
-    for (int b = threadIdx.x; b < n; b += kBlock) {
-        double v[kWaves];
-#pragma unroll
-        for (int k = 0; k < kWaves; ++k) v[k] = ldg(wp, (size_t)b * kWaves + k);
-        double r = v[0];
-#pragma unroll
-        for (int k = 1; k < kWaves; ++k) r += v[k];
-        acc += r;
-    }
-    return block_sum(acc, sh);
-}
 template <int BT = kBlock>
 __device__ inline double scene_partial_max(const double* partial, int n, double* sh) {
     double acc = -1e300;
@@ -230,6 +215,24 @@ __device__ inline bool loop_over(const DevScene& S, Scalars* ss, bool firstChunk
     if (loop_goes_on<KIND>(S, ss, it, err)) return false;
     if (firstChunk && threadIdx.x == 0) loop_ended<KIND>(ss, it, err, idx);
     return true;
+}
+
+// The list build's error partials (in the sort's scratch) added up; wide: one
+// a group, from which a chunk's sum is formed as block_sum forms it.
+__device__ inline double build_error_sum(const DevScene& S, bool wide, double* sh) {
+    const double* const part = (const double*)S.perm;
+    if (!wide) return scene_partial_sum(part, S.nChunks, sh);
+    double acc = 0.0;
+    for (int b = threadIdx.x; b < S.nChunks; b += kBlock) {
+        double v[kWaves];
+#pragma unroll
+        for (int k = 0; k < kWaves; ++k) v[k] = ldg(part, (size_t)b * kWaves + k);
+        double r = v[0];
+#pragma unroll
+        for (int k = 1; k < kWaves; ++k) r += v[k];
+        acc += r;
+    }
+    return block_sum(acc, sh);
 }
 
 // CFL time step (src/DFSPHSolver.cpp:827-870) from the scene's largest
@@ -976,9 +979,8 @@ struct BuildSums {
 // in the list; nearBound (PCISPH): its cells hold boundary particles.  Returns
 // its share of the average divergence error (DFSPH).
 template <int M>
-__device__ inline double build_finish(const DevScene& S, int i, const float4& xi, const float4& vi, const BuildSums& b,
-                                      int cnt, int own, int ngr, bool nearBound) {
-    const KCoefD& k = S.kd;
+__device__ inline double build_finish(const DevScene& S, const KCoefD& k, int i, const float4& xi, const float4& vi,
+                                      const BuildSums& b, int cnt, int own, int ngr, bool nearBound) {
     const double rho0 = S.rho0D, m = S.mD;
     if (cnt > S.maxNbr) {
         atomicMax(&S.ss->overflow, (unsigned)cnt);
@@ -1027,10 +1029,10 @@ __device__ inline double build_finish(const DevScene& S, int i, const float4& xi
     return 0.0;
 }
 
-// The end of a DFSPH list build: each wavefront's share of the error before
-// the divergence loop (only the log has it) goes to the sort's scratch; one
-// thread of a scene starts the divergence loop (`fused`: no finalize kernel
-// does).
+// The end of a DFSPH list build: the chunks' shares of the error before the
+// divergence loop (only the log has it; k_build_quad: the groups') go to the
+// sort's scratch, and one thread of a scene starts the divergence loop
+// (`fused`: no finalize kernel does).
 __device__ inline void build_starts_divergence(const DevScene& S, int fused) {
     Scalars* const ss = S.ss;
     ss->d0Valid = 1u;
@@ -1409,11 +1411,12 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
         stg(S.nsh, (size_t)i, (uint16_t)(shellLost ? 0xFFFF : ns));
     }
     if ((i & 63) == 0) stg(S.gcnt, (size_t)(i >> 6), (uint16_t)pad);
-    e = build_finish<M>(S, i, xi, vi, b, cnt, own, ngr, nearBound);
+    e = build_finish<M>(S, k, i, xi, vi, b, cnt, own, ngr, nearBound);
     }
     if (M == DFSPH) {
-        const double es = wave_sum(e);
-        if (lane == 0) ((gptr<double>)S.perm)[wb >> 6] = es;
+        __shared__ double sh[kWaves];
+        const double bs = block_sum(e, sh);
+        if (threadIdx.x == 0) ((gptr<double>)S.perm)[c.begin / kBlock] = bs;
         if (c.begin == 0 && threadIdx.x == 0) build_starts_divergence(S, fused);
     }
 }
@@ -1779,7 +1782,7 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
         if (u == 0) {
             if (M == PCISPH) stg(S.nsh, (size_t)i, (uint16_t)(shellLost ? 0xFFFF : ns));
             if (pl == 0) stg(S.gcnt, (size_t)(i >> 6), (uint16_t)pad);
-            e = build_finish<M>(S, i, xi, vi, b, cnt, own, ngr, nearBound);
+            e = build_finish<M>(S, k, i, xi, vi, b, cnt, own, ngr, nearBound);
         }
     }
     if (M == DFSPH) {
@@ -2728,7 +2731,8 @@ __global__ __launch_bounds__(kBlock) void k_pci_integrate(const DevScene* __rest
 // scenes still iterating, active[1] is the largest iteration count reached.
 enum FinKind { FIN_DT = 0, FIN_DENS0, FIN_DENS, FIN_DIV0, FIN_DIV, FIN_PCI };
 
-// wide: the PCISPH partials are one a group (k_pci_density_quad)
+// wide: the partials of the PCISPH density sweep (k_pci_density_quad) or the
+// list build (k_build_quad) are one a group
 template <int KIND>
 __global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict__ T, int nscenes, int* active, int wide) {
     const int sc = blockIdx.x;
@@ -2741,7 +2745,7 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict_
     __shared__ double sh[kWaves];
     const double red = (KIND == FIN_PCI && wide) ? scene_partial_max(pci_wide_partial(S, 0), S.nChunks * kWaves, sh)
                        : (KIND == FIN_DT || KIND == FIN_PCI) ? scene_partial_max(S.partial, S.nChunks, sh)
-                       : KIND == FIN_DIV0 ? scene_wave_sum((const double*)S.perm, S.nChunks, sh)
+                       : KIND == FIN_DIV0 ? build_error_sum(S, wide, sh)
                                           : scene_partial_sum(S.partial, S.nChunks, sh);
     if (threadIdx.x != 0) return;
     if (KIND == FIN_DT) {
@@ -2823,7 +2827,7 @@ __global__ __launch_bounds__(kBlock) void k_loop_end(const DevScene* __restrict_
         __syncthreads();   // every thread has read the flag before it is set
         if (!over && fused && !(END && KIND == LOOP_PCI)) over = loop_over<KIND>(S, ss, true, kLoopLast, sh);
         if (END && KIND == LOOP_DIV && fused) {
-            const double avg0 = scene_wave_sum((const double*)S.perm, S.nChunks, sh) / (double)S.n;
+            const double avg0 = build_error_sum(S, S.nChunks <= kQuadChunks, sh) / (double)S.n;
             if (threadIdx.x == 0) ss->avgErrV0 = avg0;
         }
         if (END && !over && tables.a) {
@@ -3280,7 +3284,7 @@ void launch_finalize(hipStream_t st, int kind, const DevScene* T, int nscenes, i
         case FIN_DT: LAUNCH(k_finalize<FIN_DT>, nscenes, st, T, nscenes, active, 0); break;
         case FIN_DENS0: LAUNCH(k_finalize<FIN_DENS0>, nscenes, st, T, nscenes, active, 0); break;
         case FIN_DENS: LAUNCH(k_finalize<FIN_DENS>, nscenes, st, T, nscenes, active, 0); break;
-        case FIN_DIV0: LAUNCH(k_finalize<FIN_DIV0>, nscenes, st, T, nscenes, active, 0); break;
+        case FIN_DIV0: LAUNCH(k_finalize<FIN_DIV0>, nscenes, st, T, nscenes, active, nchunks <= kQuadChunks ? 1 : 0); break;
         case FIN_DIV: LAUNCH(k_finalize<FIN_DIV>, nscenes, st, T, nscenes, active, 0); break;
         default: LAUNCH(k_finalize<FIN_PCI>, nscenes, st, T, nscenes, active, nchunks <= kQuadPciChunks ? 1 : 0); break;
     }
