@@ -663,7 +663,7 @@ int batch_one_step(sphg_ctx* ctx, Batch& B, uint32_t& syncs) {
         B.lastIt = seen;
         const DevScene* T2 = B.dT[1];
         rc = run_segment(ctx, B, 1, [&] {
-            { Scope s(P, st, K_DFPOS); launch_df_positions(st, T, particle_chunks(B), B.nP, ctx->dActive, 0, 0); }
+            { Scope s(P, st, K_DFPOS); launch_df_positions(st, T, particle_chunks(B), B.nP, ctx->dActive, 0); }
             // PCISPH boundary method: projection after the position update
             // (src/DFSPHSolver.cpp:65-75), which then counts the cells
             if (anyPb) { Scope s(P, st, K_PB); launch_pb_correct(st, 0, T, particle_chunks(B), B.nP); }
@@ -744,7 +744,7 @@ int batch_one_step(sphg_ctx* ctx, Batch& B, uint32_t& syncs) {
         }
         B.lastIt = seen;
         rc = run_segment(ctx, B, 1, [&] {
-            { Scope s(P, st, K_PCIINT); launch_pci_integrate(st, T2, particle_chunks(B), B.nP, 0, 0); }
+            { Scope s(P, st, K_PCIINT); launch_pci_integrate(st, T2, particle_chunks(B), B.nP, 0); }
             // cube boundary after the integration (src/PCISPHSolver.cpp:54-63),
             // or the PCISPH boundary projection (:65-76), then the emitters
             // (:78), then time += dt (:80)
@@ -790,21 +790,25 @@ int lone_step(sphg_ctx* ctx, Batch& B, int from, int it, bool ask, uint32_t seq,
     const DevScene& V = B.scenes[0]->view[0];
     const int flags = V.flags, n = B.nP;
     const bool st_on = (flags & F_ST) != 0;
-    const int fused = V.nChunks <= kFusedLoopChunks ? 1 : 0;
+    const bool large = V.nChunks > kFusedLoopChunks;
     const DevScene *T = B.dT[0], *T2 = B.dT[1];
     const Tables none{}, tables = ask ? Tables{} : Tables{B.dT[0], B.dT[1]};
     int rc;
     // launches iterations: the `ahead` predicted ones, then one at a time
     // while the scene's record says that the loop goes on
     auto loop = [&](int kind, int end, const DevScene* Tl, int ahead, int& reached, auto&& iterate) -> int {
+        const int least = kind == LOOP_DIV ? V.minItV : V.minIt;
         const bool resumed = it > 0;
-        for (; it < (resumed ? it + 1 : ahead); ++it) {
-            iterate(it);
-            if (resumed) { ++it; break; }
-        }
+        auto run = [&] {
+            iterate(it++);
+            if (large && !ask && it >= least) launch_loop_end(st, kind, 0, Tl, none, nullptr, 0, it);
+        };
+        if (resumed) run();
+        else
+            while (it < ahead) run();
         while (ask) {
             const uint32_t q = ++ctx->recSeq;
-            launch_loop_end(st, kind, end, Tl, fused, none, ctx->recs + q % kRecs, q);
+            launch_loop_end(st, kind, end, Tl, none, ctx->recs + q % kRecs, q, it);
             StepRec r;
             int e = wait_rec(ctx, q, r);
             if (e) return e;
@@ -813,7 +817,7 @@ int lone_step(sphg_ctx* ctx, Batch& B, int from, int it, bool ask, uint32_t seq,
                 reached = kind == LOOP_DIV ? r.itV : r.it;
                 break;
             }
-            iterate(it++);
+            run();
         }
         it = 0;
         return SPHG_OK;
@@ -827,42 +831,37 @@ int lone_step(sphg_ctx* ctx, Batch& B, int from, int it, bool ask, uint32_t seq,
                     launch_forces(st, DFSPH, flags, T, nullptr, n);
                 }
                 { Scope s(P, st, K_DT); launch_dt(st, T, nullptr, n); }
-                if (!fused) finalize(ctx, B, T, 0);
-                { Scope s(P, st, K_DFPREDICT); launch_df_predict(st, T, nullptr, n, fused); }
-                { Scope s(P, st, K_DFVEL_WARM); launch_df_vel(st, 0, T, nullptr, n, 0, fused); }
-                { Scope s(P, st, K_DFERR_DENS); launch_df_err(st, 0, T, nullptr, n, fused); }
-                if (!fused) finalize(ctx, B, T, 1);
+                if (large) finalize(ctx, B, T, 0);
+                { Scope s(P, st, K_DFPREDICT); launch_df_predict(st, T, nullptr, n, 1); }
+                { Scope s(P, st, K_DFVEL_WARM); launch_df_vel(st, 0, T, nullptr, n, 0, 1); }
+                { Scope s(P, st, K_DFERR_DENS); launch_df_err(st, 0, T, nullptr, n, 1); }
             });
             if (rc) return rc;
         }
         if (from <= 1) {
             rc = loop(LOOP_DENS, 0, T, density_ahead(B), B.lastIt, [&](int k) {
-                { Scope s(P, st, K_DFVEL_DENS); launch_df_vel(st, 1, T, nullptr, n, k, fused); }
-                { Scope s(P, st, K_DFERR_DENS); launch_df_err(st, 1, T, nullptr, n, fused); }
-                if (!fused) finalize(ctx, B, T, 2);
+                { Scope s(P, st, K_DFVEL_DENS); launch_df_vel(st, 1, T, nullptr, n, k, 1); }
+                { Scope s(P, st, K_DFERR_DENS); launch_df_err(st, 1, T, nullptr, n, 1); }
             });
             if (rc) return rc;
             auto rest = [&] {
-                { Scope s(P, st, K_DFPOS); launch_df_positions(st, T, nullptr, n, ctx->dActive, fused, ask ? 0 : 1); }
-                grid_sort(ctx, B, T, tables, fused);
-                { Scope s(P, st, K_BUILD); launch_build(st, DFSPH, T2, nullptr, n, fused); }
-                if (!fused) finalize(ctx, B, T2, 3);
+                { Scope s(P, st, K_DFPOS); launch_df_positions(st, T, nullptr, n, ctx->dActive, ask ? 0 : 1); }
+                grid_sort(ctx, B, T, tables, 1);
+                { Scope s(P, st, K_BUILD); launch_build(st, DFSPH, T2, nullptr, n, 1); }
             };
             // (the captured segment is the one of steps that do not ask)
             if (ask) rest();
             else if ((rc = run_segment(ctx, B, 1, rest))) return rc;
         }
         rc = loop(LOOP_DIV, 1, T2, divergence_ahead(B), B.lastItV, [&](int k) {
-            { Scope s(P, st, K_DFVEL_DIV); launch_df_vel(st, 2, T2, nullptr, n, k, fused); }
-            { Scope s(P, st, K_DFERR_DIV); launch_df_err(st, 3, T2, nullptr, n, fused); }
-            if (!fused) finalize(ctx, B, T2, 4);
+            { Scope s(P, st, K_DFVEL_DIV); launch_df_vel(st, 2, T2, nullptr, n, k, 1); }
+            { Scope s(P, st, K_DFERR_DIV); launch_df_err(st, 3, T2, nullptr, n, 1); }
         });
         if (rc) return rc;
-        if (!ask) launch_loop_end(st, LOOP_DIV, 1, T2, fused, tables, ctx->recs + seq % kRecs, seq);
+        if (!ask) launch_loop_end(st, LOOP_DIV, 1, T2, tables, ctx->recs + seq % kRecs, seq, 0);
     } else {
         if (from == 0) {
             rc = run_segment(ctx, B, 0, [&] {
-                if (!fused) launch_fill_int(st, ctx->dActive, 0, 2);
                 // the keys kernel also starts the step
                 { Scope s(P, st, K_KEYS); launch_keys(st, T, nullptr, n, ctx->dActive); }
                 grid_sort(ctx, B, T);
@@ -873,13 +872,12 @@ int lone_step(sphg_ctx* ctx, Batch& B, int from, int it, bool ask, uint32_t seq,
             if (rc) return rc;
         }
         rc = loop(LOOP_PCI, 0, T2, density_ahead(B), B.lastIt, [&](int k) {
-            { Scope s(P, st, K_PCIDENS); launch_pci_density(st, T2, nullptr, n, k, fused); }
-            if (!fused) finalize(ctx, B, T2, 5);
-            { Scope s(P, st, K_PCIPACC); launch_pci_pacc(st, T2, nullptr, n, k, fused); }
+            { Scope s(P, st, K_PCIDENS); launch_pci_density(st, T2, nullptr, n, k, 1); }
+            { Scope s(P, st, K_PCIPACC); launch_pci_pacc(st, T2, nullptr, n, k, 1); }
         });
         if (rc) return rc;
-        { Scope s(P, st, K_PCIINT); launch_pci_integrate(st, T2, nullptr, n, fused, ask ? 0 : 1); }
-        if (!ask) launch_loop_end(st, LOOP_PCI, 1, T2, fused, tables, ctx->recs + seq % kRecs, seq);
+        { Scope s(P, st, K_PCIINT); launch_pci_integrate(st, T2, nullptr, n, ask ? 0 : 1); }
+        if (!ask) launch_loop_end(st, LOOP_PCI, 1, T2, tables, ctx->recs + seq % kRecs, seq, 0);
     }
     flip(B);
     return SPHG_OK;

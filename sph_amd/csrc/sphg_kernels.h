@@ -14,9 +14,11 @@ struct Tables {
 };
 // the solvers' loops: DFSPH density and divergence, PCISPH pressure
 enum LoopKind { LOOP_DENS, LOOP_DIV, LOOP_PCI };
-// A lone scene of up to kFusedLoopChunks chunks has its loops decided in the
-// sweeps themselves (`fused`), each block adding up the chunk partials; above
-// that the partials are too many for every block, and finalize kernels do it.
+// A lone scene's sweeps control its loops (`fused`).  Up to kFusedLoopChunks
+// chunks each block of a sweep adds up the last one's partials; above that they
+// are too many for every block, and launch_loop_end decides after an iteration
+// that may be the last (1M particles: 973 -> 960 us a step against finalize
+// kernels before the loops and after every iteration).
 constexpr int kFusedLoopChunks = 2048;
 // Launches of up to so many chunks give the list build and the PCISPH density
 // sweep 4 lanes a particle (figures: launch_build, launch_pci_density).
@@ -50,14 +52,14 @@ void launch_df_err(hipStream_t st, int mode, const DevScene* T, const Chunk* C, 
 // kind: 0 dt, 1 density (before loop), 2 density, 3 divergence (before loop), 4 divergence, 5 PCISPH
 void launch_finalize(hipStream_t st, int kind, const DevScene* T, int nscenes, int* active, int nchunks);
 // also clears active[0..1] for the divergence solve
-void launch_df_positions(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int* active, int fused,
-                         int ahead);
+void launch_df_positions(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int* active, int ahead);
 void launch_pci_density(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int iter, int fused);
 void launch_pci_pacc(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int iter, int fused);
-void launch_pci_integrate(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int fused, int ahead);
-// loop: LoopKind; end: the end of a step
-void launch_loop_end(hipStream_t st, int loop, int end, const DevScene* T, int fused, Tables tables, StepRec* rec,
-                     unsigned seq);
+void launch_pci_integrate(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int ahead);
+// loop: LoopKind; end: the end of a step; iter: iterations launched so far; a
+// null rec: decides only
+void launch_loop_end(hipStream_t st, int loop, int end, const DevScene* T, Tables tables, StepRec* rec, unsigned seq,
+                     int iter);
 void launch_tell_active(hipStream_t st, const int* active, StepRec* rec, unsigned seq);
 void launch_clear_stall(hipStream_t st, Tables tables);
 void launch_cube(hipStream_t st, const DevScene* T, const Chunk* C, int n);

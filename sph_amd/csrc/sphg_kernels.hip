@@ -204,7 +204,9 @@ __device__ inline float* pci_displacements(const DevScene& S) {
 // Whether the loop has ended, decided by every block alike (block-uniform;
 // called where ended_before(done, idx) is false).
 template <int KIND, int BT = kBlock>
-__device__ inline bool loop_over(const DevScene& S, Scalars* ss, bool firstChunk, int idx, double* sh) {
+__device__ inline bool loop_over(const DevScene& S, Scalars* ss, bool firstChunk, int idx, double* sh, bool large = false) {
+    // too many partials for every block: k_loop_end decides
+    if (!large && S.nChunks > kFusedLoopChunks) return false;
     const int it = KIND == LOOP_DIV ? ss->itV : ss->it;
     // below the minimum the error does not matter
     if (it < (KIND == LOOP_DIV ? S.minItV : S.minIt) && it < S.maxIt) return false;
@@ -2096,7 +2098,7 @@ __global__ __launch_bounds__(kBlock) void k_df_predict(const DevScene* __restric
     __shared__ double sh[kWaves];
     const int i = c.begin + threadIdx.x;
     double dt = G(S.ss)->dt;
-    if (fused) {
+    if (fused && S.nChunks <= kFusedLoopChunks) {
         const NextDt d = next_dt(S, dt, G(S.ss)->it, scene_partial_max(S.partial, S.nChunks, sh));
         dt = d.dt;
         if (c.begin == 0 && threadIdx.x == 0) {
@@ -2157,9 +2159,10 @@ __global__ __launch_bounds__(kBlock) void k_df_vel(const DevScene* __restrict__ 
     double dt = ss->dt;
     if (fused) {
         if (MODE == 0) {
-            dt = ss->dtNew;
+            // (a large scene's finalize kernel has written dt itself)
+            if (S.nChunks <= kFusedLoopChunks) dt = ss->dtNew;
             if (c.begin == 0 && threadIdx.x == 0) {
-                ss->dt = dt;
+                if (S.nChunks <= kFusedLoopChunks) ss->dt = dt;
                 ss->it = 0;
                 ss->done = loop_goes_on<LOOP_DENS>(S, ss, 0, 0.0) ? 0 : 1;
             }
@@ -2343,13 +2346,13 @@ __global__ __launch_bounds__(kBlock) void k_df_err(const DevScene* __restrict__ 
 // without asking; if the loop has not ended, nothing from here on runs (the
 // cell scan behind it tells the later launches).
 __global__ __launch_bounds__(kBlock) void k_df_positions(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
-                                                         int* active, int fused, int ahead) {
+                                                         int* active, int ahead) {
     const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
     if (S.stall) return;
     if (ahead && !ended_before(S.ss->done, kLoopLast)) {
         __shared__ double sh[kWaves];
-        if (!fused || !loop_over<LOOP_DENS>(S, S.ss, c.begin == 0, kLoopLast, sh)) return;
+        if (!loop_over<LOOP_DENS>(S, S.ss, c.begin == 0, kLoopLast, sh)) return;
     }
     if (blockIdx.x == 0 && threadIdx.x < 2) active[threadIdx.x] = 0;
     // the lists about to be built start without an overflow
@@ -2689,13 +2692,13 @@ __global__ __launch_bounds__(kBlock) void k_pci_pacc(const DevScene* __restrict_
 // PCISPH integrate (src/PCISPHSolver.cpp:444-474): a += g + pacc.
 // `ahead`: as in k_df_positions; the launch behind this one tells the rest.
 __global__ __launch_bounds__(kBlock) void k_pci_integrate(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
-                                                          int fused, int ahead) {
+                                                          int ahead) {
     const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
     if (S.stall) return;
     if (ahead && !ended_before(S.ss->done, kLoopLast)) {
         __shared__ double sh[kWaves];
-        if (!fused || !loop_over<LOOP_PCI>(S, S.ss, c.begin == 0, kLoopLast, sh)) return;
+        if (!loop_over<LOOP_PCI>(S, S.ss, c.begin == 0, kLoopLast, sh)) return;
     }
     const int i = c.begin + threadIdx.x;
     if (c.begin == 0 && threadIdx.x == 0 && time_in_last_kernel(S)) advance_time(S);
@@ -2815,9 +2818,11 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict_
 // divergence loop.  END: the end of a step.  With `tables` the host has not
 // asked after the step's loops and the next step's launches wait behind this
 // one: they return at once if a loop has not ended.
+// Without `rec` it only decides, for a scene whose sweeps leave that to it;
+// idx: see loop_over.
 template <int KIND, bool END>
-__global__ __launch_bounds__(kBlock) void k_loop_end(const DevScene* __restrict__ T, int fused, Tables tables, StepRec* rec,
-                                                     unsigned seq) {
+__global__ __launch_bounds__(kBlock) void k_loop_end(const DevScene* __restrict__ T, Tables tables, StepRec* rec,
+                                                     unsigned seq, int idx) {
     const DevScene& S = T[0];
     Scalars* ss = S.ss;
     int stall = S.stall;
@@ -2825,8 +2830,9 @@ __global__ __launch_bounds__(kBlock) void k_loop_end(const DevScene* __restrict_
     if (!stall) {
         bool over = (KIND == LOOP_DIV ? ss->doneV : ss->done) != 0;
         __syncthreads();   // every thread has read the flag before it is set
-        if (!over && fused && !(END && KIND == LOOP_PCI)) over = loop_over<KIND>(S, ss, true, kLoopLast, sh);
-        if (END && KIND == LOOP_DIV && fused) {
+        // (the PCISPH integration has decided where the sweeps do)
+        if (!over && !(END && KIND == LOOP_PCI)) over = loop_over<KIND>(S, ss, true, idx, sh, true);
+        if (END && KIND == LOOP_DIV) {
             const double avg0 = build_error_sum(S, S.nChunks <= kQuadChunks, sh) / (double)S.n;
             if (threadIdx.x == 0) ss->avgErrV0 = avg0;
         }
@@ -2834,9 +2840,9 @@ __global__ __launch_bounds__(kBlock) void k_loop_end(const DevScene* __restrict_
             stall = KIND == LOOP_PCI ? 1 : 2;
             if (threadIdx.x == 0) tables.a->stall = tables.b->stall = stall;
         }
-        if (threadIdx.x == 0) rec->done = over ? 1 : 0;
+        if (threadIdx.x == 0 && rec) rec->done = over ? 1 : 0;
     }
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0 && rec) {
         rec->it = ss->it;
         rec->itV = ss->itV;
         rec->stall = stall;
@@ -3289,8 +3295,8 @@ void launch_finalize(hipStream_t st, int kind, const DevScene* T, int nscenes, i
         default: LAUNCH(k_finalize<FIN_PCI>, nscenes, st, T, nscenes, active, nchunks <= kQuadPciChunks ? 1 : 0); break;
     }
 }
-void launch_df_positions(hipStream_t st, const DevScene* T, const Chunk* C, int n, int* active, int fused, int ahead) {
-    if (n) LAUNCH(k_df_positions, n, st, T, C, active, fused, ahead);
+void launch_df_positions(hipStream_t st, const DevScene* T, const Chunk* C, int n, int* active, int ahead) {
+    if (n) LAUNCH(k_df_positions, n, st, T, C, active, ahead);
 }
 void launch_pci_density(hipStream_t st, const DevScene* T, const Chunk* C, int n, int iter, int fused) {
     if (!n) return;
@@ -3303,15 +3309,16 @@ void launch_pci_density(hipStream_t st, const DevScene* T, const Chunk* C, int n
 void launch_pci_pacc(hipStream_t st, const DevScene* T, const Chunk* C, int n, int iter, int fused) {
     if (n) LAUNCH(k_pci_pacc, n, st, T, C, iter, fused);
 }
-void launch_pci_integrate(hipStream_t st, const DevScene* T, const Chunk* C, int n, int fused, int ahead) {
-    if (n) LAUNCH(k_pci_integrate, n, st, T, C, fused, ahead);
+void launch_pci_integrate(hipStream_t st, const DevScene* T, const Chunk* C, int n, int ahead) {
+    if (n) LAUNCH(k_pci_integrate, n, st, T, C, ahead);
 }
-void launch_loop_end(hipStream_t st, int loop, int end, const DevScene* T, int fused, Tables t, StepRec* rec, unsigned seq) {
-    if (loop == LOOP_PCI && end) LAUNCH((k_loop_end<LOOP_PCI, true>), 1, st, T, fused, t, rec, seq);
-    else if (loop == LOOP_PCI) LAUNCH((k_loop_end<LOOP_PCI, false>), 1, st, T, fused, t, rec, seq);
-    else if (loop == LOOP_DENS) LAUNCH((k_loop_end<LOOP_DENS, false>), 1, st, T, fused, t, rec, seq);
-    else if (end) LAUNCH((k_loop_end<LOOP_DIV, true>), 1, st, T, fused, t, rec, seq);
-    else LAUNCH((k_loop_end<LOOP_DIV, false>), 1, st, T, fused, t, rec, seq);
+void launch_loop_end(hipStream_t st, int loop, int end, const DevScene* T, Tables t, StepRec* rec, unsigned seq, int iter) {
+    const int idx = end ? kLoopLast : iter;
+    if (loop == LOOP_PCI && end) LAUNCH((k_loop_end<LOOP_PCI, true>), 1, st, T, t, rec, seq, idx);
+    else if (loop == LOOP_PCI) LAUNCH((k_loop_end<LOOP_PCI, false>), 1, st, T, t, rec, seq, idx);
+    else if (loop == LOOP_DENS) LAUNCH((k_loop_end<LOOP_DENS, false>), 1, st, T, t, rec, seq, idx);
+    else if (end) LAUNCH((k_loop_end<LOOP_DIV, true>), 1, st, T, t, rec, seq, idx);
+    else LAUNCH((k_loop_end<LOOP_DIV, false>), 1, st, T, t, rec, seq, idx);
 }
 void launch_tell_active(hipStream_t st, const int* active, StepRec* rec, unsigned seq) {
     hipLaunchKernelGGL(k_tell_active, dim3(1), dim3(64), 0, st, active, rec, seq);
