@@ -20,9 +20,18 @@ enum LoopKind { LOOP_DENS, LOOP_DIV, LOOP_PCI };
 // that may be the last (1M particles: 973 -> 960 us a step against finalize
 // kernels before the loops and after every iteration).
 constexpr int kFusedLoopChunks = 2048;
-// Launches of up to so many chunks give the list build and the PCISPH density
-// sweep 4 lanes a particle (figures: launch_build, launch_pci_density).
-constexpr int kQuadChunks = 320, kQuadChunksWcsph = 512, kQuadPciChunks = 768;
+// Launches of up to so many chunks give a particle 4 lanes (figures at the
+// launchers).
+constexpr int kQuadChunks = 320, kQuadChunksWcsph = 512;    // list build
+constexpr int kQuadPciChunks = 768, kQuadPaccChunks = 128;  // PCISPH loop
+constexpr int kQuadForcesChunks = 384;                      // forces without cohesion
+constexpr int kQuadTensionChunks = 128;                     // WCSPH forces with cohesion
+// The DFSPH sweeps, normals, cohesion: 4 lanes a particle take a block of 64
+// particles ~1/3 of the time, and a sweep lasts as long as the compute units
+// (256) with the most blocks.
+constexpr bool quad_sweep(int nchunks) {
+    return nchunks <= 384 && (nchunks * kWaves + 255) / 256 <= 3 * ((nchunks + 255) / 256);
+}
 
 // begin_active: also the start of a WCSPH or PCISPH step, counting the
 // scenes whose pressure loop runs in begin_active[0] (null: keys only)

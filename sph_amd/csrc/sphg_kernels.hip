@@ -86,6 +86,50 @@ __device__ inline Chunk chunk_at(const Chunk* C, int unit, int b, int nchunks) {
 }
 __device__ inline Chunk chunk_at(const Chunk* C, int unit) { return chunk_at(C, unit, blockIdx.x, gridDim.x); }
 
+// Kernels that give a particle Q = 4 lanes: a block of 4 wavefronts holds one
+// 64-particle group, lane 4 q + u of wavefront w works on the group's particle
+// 16 w + q, and a chunk's groups run on one XCD, like the chunk.  Q = 1: a
+// block holds a chunk.  The block's first particle goes to i0, the thread's to
+// i; false: there is no such chunk.
+template <int Q>
+__device__ inline bool part_at(const Chunk* C, int nchunks, Chunk& c, int& i0, int& i) {
+    if (Q == 1) {
+        c = chunk_at(C, kBlock);
+        i0 = c.begin;
+        i = i0 + threadIdx.x;
+        return true;
+    }
+    const int g = (int)blockIdx.x >> 3, slot = (g / kWaves) * 8 + (int)(blockIdx.x & 7);
+    if (slot >= nchunks) return false;
+    c = chunk_at(C, kBlock, slot, nchunks);
+    i0 = c.begin + (g % kWaves) * kGroup;
+    i = i0 + (threadIdx.x >> 2);
+    return true;
+}
+template <int Q> constexpr int kPartBlock = Q == 1 ? kBlock : 256;
+
+// x of lane V of the quad
+template <int V>
+__device__ inline int quad_lane(int x) {
+    return __builtin_amdgcn_update_dpp(0, x, V * 0x55, 0xf, 0xf, true);
+}
+template <int V>
+__device__ inline double quad_lane(double x) {
+    return __hiloint2double(quad_lane<V>(__double2hiint(x)), quad_lane<V>(__double2loint(x)));
+}
+// N doubles that go from lane to lane together
+template <int N>
+struct Terms {
+    double v[N];
+};
+template <int V, int N>
+__device__ inline Terms<N> quad_lane(const Terms<N>& t) {
+    Terms<N> o;
+#pragma unroll
+    for (int k = 0; k < N; ++k) o.v[k] = quad_lane<V>(t.v[k]);
+    return o;
+}
+
 __device__ inline double wave_sum(double v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
@@ -97,7 +141,8 @@ __device__ inline double wave_max(double v) {
     return v;
 }
 // Result valid in every thread; the wave results are added in wave order.
-// sh: kWaves doubles of shared memory.
+// BT: the block's threads; sh: BT / 64 doubles of shared memory.
+template <int BT = kBlock>
 __device__ inline double block_sum(double v, double* sh) {
     v = wave_sum(v);
     const int w = threadIdx.x >> 6;
@@ -105,11 +150,10 @@ __device__ inline double block_sum(double v, double* sh) {
     __syncthreads();
     double r = sh[0];
 #pragma unroll
-    for (int k = 1; k < kWaves; ++k) r += sh[k];
+    for (int k = 1; k < BT / 64; ++k) r += sh[k];
     __syncthreads();
     return r;
 }
-// BT: the block's threads.
 template <int BT = kBlock>
 __device__ inline double block_max(double v, double* sh) {
     v = wave_max(v);
@@ -129,16 +173,34 @@ __device__ inline double block_max(double v, double* sh) {
 // the loop waits on memory once for up to 4096 partials (a 1M-particle
 // scene's chunks) instead of once per partial.
 constexpr int kPartU = 4096 / kBlock;
+template <int BT = kBlock>
 __device__ inline double scene_partial_sum(const double* partial, int n, double* sh) {
     double acc = 0.0;
-    for (int b = threadIdx.x; b < n; b += kBlock * kPartU) {
+    for (int b = threadIdx.x; b < n; b += BT * kPartU) {
         double v[kPartU];
 #pragma unroll
-        for (int u = 0; u < kPartU; ++u) v[u] = (b + u * kBlock < n) ? ldg(partial, (size_t)(b + u * kBlock)) : 0.0;
+        for (int u = 0; u < kPartU; ++u) v[u] = (b + u * BT < n) ? ldg(partial, (size_t)(b + u * BT)) : 0.0;
 #pragma unroll
         for (int u = 0; u < kPartU; ++u) acc += v[u];
     }
-    return block_sum(acc, sh);
+    return block_sum<BT>(acc, sh);
+}
+// The same over n chunks whose 64-particle groups have a partial each (the
+// kernels with 4 lanes a particle): a chunk's sum is formed as block_sum forms
+// it.
+template <int BT = kBlock>
+__device__ inline double scene_group_sum(const double* partial, int n, double* sh) {
+    double acc = 0.0;
+    for (int b = threadIdx.x; b < n; b += BT) {
+        double v[kWaves];
+#pragma unroll
+        for (int k = 0; k < kWaves; ++k) v[k] = ldg(partial, (size_t)b * kWaves + k);
+        double r = v[0];
+#pragma unroll
+        for (int k = 1; k < kWaves; ++k) r += v[k];
+        acc += r;
+    }
+    return block_sum<BT>(acc, sh);
 }
 template <int BT = kBlock>
 __device__ inline double scene_partial_max(const double* partial, int n, double* sh) {
@@ -187,10 +249,12 @@ constexpr int kLoopLast = 1 << 30;   // idx of the launches behind a loop
 // its density sweep decides and writes partials in one launch.  The second is
 // the sort's scratch, which the loop does not need.
 __device__ inline double* pci_partial(const DevScene& S, int it) { return (it & 1) ? (double*)S.perm : S.partial; }
-// The density sweep with 4 lanes a particle (launches of at most
-// kQuadPciChunks chunks) leaves a partial per 64-particle group, both buffers in the scratch.
-__device__ inline double* pci_wide_partial(const DevScene& S, int it) {
-    return (double*)S.perm + (size_t)(it & 1) * S.nChunks * kWaves;
+// Partials of 64-particle groups (kernels with 4 lanes a particle), one of two
+// buffers in the sort's scratch: 0 also holds the partials of the errors
+// before the DFSPH loops, 1 those of their iterations; the PCISPH loop uses
+// both in turn.
+__device__ inline double* group_partial(const DevScene& S, int buffer) {
+    return (double*)S.perm + (size_t)buffer * S.nChunks * kWaves;
 }
 // The largest squared predicted displacement of each 64-particle group over a
 // PCISPH step's iterations, behind the partials in the scratch; the next
@@ -211,30 +275,26 @@ __device__ inline bool loop_over(const DevScene& S, Scalars* ss, bool firstChunk
     // below the minimum the error does not matter
     if (it < (KIND == LOOP_DIV ? S.minItV : S.minIt) && it < S.maxIt) return false;
     double err;
-    if (KIND != LOOP_PCI) err = scene_partial_sum(S.partial, S.nChunks, sh) / (double)S.n;
-    else if (S.nChunks <= kQuadPciChunks) err = scene_partial_max<BT>(pci_wide_partial(S, it - 1), S.nChunks * kWaves, sh);
+    if (KIND != LOOP_PCI)
+        err = (quad_sweep(S.nChunks) ? scene_group_sum<BT>(group_partial(S, 1), S.nChunks, sh)
+                                             : scene_partial_sum<BT>(S.partial, S.nChunks, sh)) / (double)S.n;
+    else if (S.nChunks <= kQuadPciChunks) err = scene_partial_max<BT>(group_partial(S, (it - 1) & 1), S.nChunks * kWaves, sh);
     else err = scene_partial_max<BT>(pci_partial(S, it - 1), S.nChunks, sh);
     if (loop_goes_on<KIND>(S, ss, it, err)) return false;
     if (firstChunk && threadIdx.x == 0) loop_ended<KIND>(ss, it, err, idx);
     return true;
 }
 
-// The list build's error partials (in the sort's scratch) added up; wide: one
-// a group, from which a chunk's sum is formed as block_sum forms it.
-__device__ inline double build_error_sum(const DevScene& S, bool wide, double* sh) {
-    const double* const part = (const double*)S.perm;
-    if (!wide) return scene_partial_sum(part, S.nChunks, sh);
-    double acc = 0.0;
-    for (int b = threadIdx.x; b < S.nChunks; b += kBlock) {
-        double v[kWaves];
-#pragma unroll
-        for (int k = 0; k < kWaves; ++k) v[k] = ldg(part, (size_t)b * kWaves + k);
-        double r = v[0];
-#pragma unroll
-        for (int k = 1; k < kWaves; ++k) r += v[k];
-        acc += r;
+// A group's sum of e (in the first lane of each quad), formed as a wavefront
+// that holds the 64 particles forms it.
+__device__ inline void group_error(const DevScene& S, int buffer, int i0, double e) {
+    __shared__ double se[kGroup];
+    if ((threadIdx.x & 3) == 0) se[threadIdx.x >> 2] = e;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const double es = wave_sum(se[threadIdx.x]);
+        if (threadIdx.x == 0) group_partial(S, buffer)[i0 >> 6] = es;
     }
-    return block_sum(acc, sh);
 }
 
 // CFL time step (src/DFSPHSolver.cpp:827-870) from the scene's largest
@@ -429,6 +489,39 @@ __device__ inline void sweep4(const DevScene& S, int i, Load&& load, Body&& body
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int u = 0; u < 4; ++u) body(jj[u], dd[u]);
+    }
+}
+
+// A particle's list with Q lanes: term(data) of every entry, added in list
+// order (add).  Q = 1 is sweep4.  With 4 lanes a lane takes every 4th entry,
+// two at a time, and every lane adds the quad's terms one after the other, so
+// the sums are the same bit for bit.  A small launch has a wavefront or so a
+// SIMD, whose chain of gathers and FP64 math bounds it: a DFSPH sweep of 4,032
+// particles 8 -> 5.3 us, the WCSPH forces of 2,197 15.8 -> 6.3.
+template <int Q, class Load, class Term, class Add>
+__device__ inline void sweep(const DevScene& S, int i, Load&& load, Term&& term, Add&& add) {
+    if constexpr (Q == 1) {
+        sweep4(S, i, load, [&](uint32_t, const auto& d) { add(term(d)); });
+    } else {
+        const uint32_t* const L = list_of(S, i) + (threadIdx.x & 3);
+        const int nb = group_count(S, i) >> 2;
+        if (nb == 0) return;
+        auto at = [&](int b) { return ldg(L, (size_t)slot_of(4 * min(b, nb - 1))); };
+        uint32_t jn[2] = {at(0), at(1)};
+        for (int q = 0; q < nb; q += 2) {
+            decltype(load(0u)) d[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) d[h] = load(jn[h]);
+            jn[0] = at(q + 2);
+            jn[1] = at(q + 3);
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if (h == 1 && q + 1 >= nb) break;
+                const auto t = term(d[h]);
+                static_for<4>([&](auto vc) { add(quad_lane<decltype(vc)::value>(t)); });
+            }
+        }
     }
 }
 
@@ -682,7 +775,8 @@ __global__ __launch_bounds__(kBlock) void k_keys(const DevScene* __restrict__ T,
 // (one block, before the scatter overwrites them).
 __device__ inline void density_error0(const DevScene& S) {
     __shared__ double sh[kWaves];
-    const double avg0 = scene_partial_sum((const double*)S.perm, S.nChunks, sh) / (double)S.n;
+    const double avg0 = (quad_sweep(S.nChunks) ? scene_group_sum(group_partial(S, 0), S.nChunks, sh)
+                                                       : scene_partial_sum(group_partial(S, 0), S.nChunks, sh)) / (double)S.n;
     if (threadIdx.x == 0) S.ss->avgErr0 = avg0;
 }
 // The first launch behind a DFSPH density loop whose end the position update
@@ -1418,16 +1512,14 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
     if (M == DFSPH) {
         __shared__ double sh[kWaves];
         const double bs = block_sum(e, sh);
-        if (threadIdx.x == 0) ((gptr<double>)S.perm)[c.begin / kBlock] = bs;
+        if (threadIdx.x == 0) group_partial(S, 0)[c.begin / kBlock] = bs;
         if (c.begin == 0 && threadIdx.x == 0) build_starts_divergence(S, fused);
     }
 }
 
-// The same build with 4 lanes a particle, for launches too small to fill the
-// chip.  A block of 4 wavefronts holds one list group: lane 4 q + u of
-// wavefront w works on particle 16 w + q of the group, on every 4th candidate
-// from u on.  The block stages its group's rows once, for the fluid and for
-// the boundary.  Where k_build's wavefront walks its 27 cells 4 candidates at
+// The same build with 4 lanes a particle (part_at), for launches too small to
+// fill the chip: a lane takes every 4th candidate.  The block stages its
+// group's rows once, for the fluid and for the boundary.  Where k_build's wavefront walks its 27 cells 4 candidates at
 // a time in ~50 passes, each waiting on LDS, its four stores and, later, ~10
 // passes over the survivors' data in memory, a quad has a quarter of the
 // instructions in each of them.  Survivors keep their order (their slots are
@@ -1439,36 +1531,22 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
 constexpr int kQuadStage = 816, kQuadPad = 8;    // fluid candidates staged (12 B each); reads past a row's end
 constexpr int kQuadBound = 512;                  // boundary candidates staged (16 B each)
 
-// x of lane V of the quad
-template <int V>
-__device__ inline int quad_lane(int x) {
-    return __builtin_amdgcn_update_dpp(0, x, V * 0x55, 0xf, 0xf, true);
-}
-template <int V>
-__device__ inline double quad_lane(double x) {
-    return __hiloint2double(quad_lane<V>(__double2hiint(x)), quad_lane<V>(__double2loint(x)));
-}
-
 template <int M>
 __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__ T, const Chunk* __restrict__ C, int nchunks,
                                                     int fused) {
-    // a chunk's groups run on one XCD, like the chunk
-    const int slot = ((int)(blockIdx.x >> 3) / kWaves) * 8 + (int)(blockIdx.x & 7), sub = (int)(blockIdx.x >> 3) % kWaves;
-    if (slot >= nchunks) return;
-    const Chunk c = chunk_at(C, kBlock, slot, nchunks);
+    Chunk c;
+    int g0, i;   // the group's first particle and the lane's
+    if (!part_at<4>(C, nchunks, c, g0, i)) return;
     const DevScene& S = T[c.scene];
     if (S.stall) return;
     __shared__ float2 sxy[kQuadStage + kQuadPad];
     __shared__ float sz[kQuadStage + kQuadPad];
     __shared__ float4 sb[kQuadBound];
-    __shared__ double se[kGroup];
     __shared__ int spad[4];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, u = lane & 3;
-    const int g0 = c.begin + sub * kGroup;   // the group's first particle
-    const int pl = w * 16 + (lane >> 2);     // the lane's particle in the group
-    const int i = g0 + pl;
+    const int pl = tid >> 2;                 // the lane's particle in the group
     if (g0 >= S.n) {
-        if (M == DFSPH && tid == 0) ((gptr<double>)S.perm)[g0 >> 6] = 0.0;
+        if (M == DFSPH && tid == 0) group_partial(S, 0)[g0 >> 6] = 0.0;
         return;
     }
     const bool valid = i < S.n;
@@ -1788,12 +1866,7 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
         }
     }
     if (M == DFSPH) {
-        if (u == 0) se[pl] = e;
-        __syncthreads();
-        if (w == 0) {
-            const double es = wave_sum(se[lane]);
-            if (lane == 0) ((gptr<double>)S.perm)[g0 >> 6] = es;
-        }
+        group_error(S, 0, g0, e);
         if (g0 == 0 && tid == 0) build_starts_divergence(S, fused);
     }
 }
@@ -1802,11 +1875,14 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
 
 // Akinci surface normals n_i = h sum_j (m/rho_j) gradW_ij
 // (src/SurfaceTensionAkinci.h:46-61).  nrm.w carries rho_i - rho0 for pass 2.
-__global__ __launch_bounds__(kBlock) void k_normals(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = chunk_at(C, kBlock);
+template <int Q>
+__global__ __launch_bounds__(kPartBlock<Q>) void k_normals(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                           int nchunks) {
+    Chunk c;
+    int i0, i;
+    if (!part_at<Q>(C, nchunks, c, i0, i)) return;
     const DevScene& S = T[c.scene];
     if (S.stall) return;
-    const int i = c.begin + threadIdx.x;
     // a batch may hold scenes without surface tension, which have no normals
     if (i >= S.n || !(S.flags & F_ST)) return;
     const KCoefD k = S.kd;
@@ -1814,14 +1890,17 @@ __global__ __launch_bounds__(kBlock) void k_normals(const DevScene* __restrict__
     const double xx = xi.x, xy = xi.y, xz = xi.z;
     const double m = S.mD, rho0 = S.rho0D;
     double nx = 0.0, ny = 0.0, nz = 0.0;
-    sweep4(S, i, [&](uint32_t j) { XV r; r.x = ld4(S.x, j); r.v.x = ldg(S.drho, j); return r; },
-           [&](uint32_t, const XV& d) {
-               const Pair p = pair_of(xx, xy, xz, d.x, k);
-               const double g = G_d(p, k) * (m / (rho0 + (double)d.v.x));
-               nx += g * p.dx;
-               ny += g * p.dy;
-               nz += g * p.dz;
-           });
+    sweep<Q>(S, i, [&](uint32_t j) { XV r; r.x = ld4(S.x, j); r.v.x = ldg(S.drho, j); return r; },
+             [&](const XV& d) {
+                 const Pair p = pair_of(xx, xy, xz, d.x, k);
+                 return Terms<4>{{G_d(p, k) * (m / (rho0 + (double)d.v.x)), p.dx, p.dy, p.dz}};
+             },
+             [&](const Terms<4>& t) {
+                 nx = fma(t.v[0], t.v[1], nx);
+                 ny = fma(t.v[0], t.v[2], ny);
+                 nz = fma(t.v[0], t.v[3], nz);
+             });
+    if (Q > 1 && (threadIdx.x & 3) != 0) return;
     const double h = k.h;
     st4(S.nrm, i, make_float4((float)(nx * h), (float)(ny * h), (float)(nz * h), ldg(S.drho, i)));
 }
@@ -1869,13 +1948,15 @@ __device__ inline bool time_in_last_kernel(const DevScene& S) { return !(S.cubeO
 // to 190 registers, 2 wavefronts a SIMD, with one of XSPH and cohesion 90 to
 // 118, with both 124 to 146.  XSPH alone, WCSPH, 599,169 particles: 99.8 ->
 // 78.4 us; XSPH and cohesion, DFSPH, 35,805 particles: 30.4 -> 15 us.
-template <int M, int FL>
-__global__ __launch_bounds__(kBlock) void k_forces(const DevScene* __restrict__ T, const Chunk* __restrict__ C) {
-    const Chunk c = chunk_at(C, kBlock);
+template <int M, int FL, int Q>
+__global__ __launch_bounds__(kPartBlock<Q>) void k_forces(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                          int nchunks) {
+    Chunk c;
+    int i0, i;
+    if (!part_at<Q>(C, nchunks, c, i0, i)) return;
     const DevScene& S = T[c.scene];
     if (S.stall) return;
-    const int i = c.begin + threadIdx.x;
-    if ((M == WCSPH) && c.begin == 0 && threadIdx.x == 0 && time_in_last_kernel(S)) advance_time(S);
+    if ((M == WCSPH) && i0 == 0 && threadIdx.x == 0 && time_in_last_kernel(S)) advance_time(S);
     if (i >= S.n) return;
     const KCoefD k = S.kd;
     const double dt = S.ss->dt;
@@ -1895,28 +1976,39 @@ __global__ __launch_bounds__(kBlock) void k_forces(const DevScene* __restrict__ 
     double vx = 0.0, vy = 0.0, vz = 0.0;   // XSPH part (before nu/dt)
     double sx = 0.0, sy = 0.0, sz = 0.0;   // surface tension part (before gamma)
     double wx = 0.0, wy = 0.0, wz = 0.0;   // standard / artificial viscosity part
-    sweep4(
-        S, i,
-        [&](uint32_t j) {
-            NbF r;
-            r.x = (M == WCSPH) ? ld4(S.xk, j) : ld4(S.x, j);
-            if (vel) r.v = (M == WCSPH) ? ld4(S.aux, j) : ld4(S.v, j);
-            // rho_j: XSPH under WCSPH takes m/rho_j from aux.w instead
-            if ((vel && M != WCSPH) || vstd || vart) r.d = ldg(S.drho, j);
-            if (st) r.n = ld4(S.nrm, j);
-            return r;
-        },
-        [&](uint32_t, const NbF& d) {
+    auto load = [&](uint32_t j) {
+        NbF r;
+        r.x = (M == WCSPH) ? ld4(S.xk, j) : ld4(S.x, j);
+        if (vel) r.v = (M == WCSPH) ? ld4(S.aux, j) : ld4(S.v, j);
+        // rho_j: XSPH under WCSPH takes m/rho_j from aux.w instead
+        if ((vel && M != WCSPH) || vstd || vart) r.d = ldg(S.drho, j);
+        if (st) r.n = ld4(S.nrm, j);
+        return r;
+    };
+    auto pressure_of = [&](const Pair& p, const NbF& d) { return G_d(p, k) * m * (pri + (double)d.x.w); };
+    auto xsph_of = [&](const Pair& p, const NbF& d) {
+        const double mj = (M == WCSPH) ? (double)d.v.w : m / (rho0 + (double)d.d);
+        return mj * W_d(p.q, k);
+    };
+    // list members satisfy |r| <= h exactly (FP64), the reference's test at
+    // src/SurfaceTensionAkinci.h:88
+    auto kij_of = [&](const NbF& d) { return 2.0 * rho0 / (rhoi + (rho0 + (double)d.n.w)); };
+    auto cohesion_of = [&](const Pair& p, const NbF& d) {
+        bool outer = 2.0 * p.rl > k.h;
+        if (fabs(2.0 * p.rl - k.h) < 1e-9 * k.h) outer = 2.0 * exact_q(xi, d.x, S.hD).rl > S.hD;
+        return -m * C_d(p.rl, outer, k) * p.inv;
+    };
+    if constexpr (Q == 1) {
+        sweep4(S, i, load, [&](uint32_t, const NbF& d) {
             const Pair p = pair_of(xx, xy, xz, d.x, k);
             if (M == WCSPH) {
-                const double g = G_d(p, k) * m * (pri + (double)d.x.w);
+                const double g = pressure_of(p, d);
                 px -= g * p.dx;
                 py -= g * p.dy;
                 pz -= g * p.dz;
             }
             if (xs) {
-                const double mj = (M == WCSPH) ? (double)d.v.w : m / (rho0 + (double)d.d);
-                const double w = mj * W_d(p.q, k);
+                const double w = xsph_of(p, d);
                 vx += w * ((double)d.v.x - vx0);
                 vy += w * ((double)d.v.y - vy0);
                 vz += w * ((double)d.v.z - vz0);
@@ -1938,17 +2030,62 @@ __global__ __launch_bounds__(kBlock) void k_forces(const DevScene* __restrict__ 
                 wz += f * p.dz;
             }
             if (st && p.r2 > 0.0) {
-                // list members satisfy |r| <= h exactly (FP64), the reference's
-                // test at src/SurfaceTensionAkinci.h:88
-                const double kij = 2.0 * rho0 / (rhoi + (rho0 + (double)d.n.w));
-                bool outer = 2.0 * p.rl > k.h;
-                if (fabs(2.0 * p.rl - k.h) < 1e-9 * k.h) outer = 2.0 * exact_q(xi, d.x, S.hD).rl > S.hD;
-                const double cs = -m * C_d(p.rl, outer, k) * p.inv;
+                const double kij = kij_of(d);
+                const double cs = cohesion_of(p, d);
                 sx += kij * (cs * p.dx - ((double)ni.x - (double)d.n.x));
                 sy += kij * (cs * p.dy - ((double)ni.y - (double)d.n.y));
                 sz += kij * (cs * p.dz - ((double)ni.z - (double)d.n.z));
             }
         });
+    } else {
+        // (pressure g, d), (XSPH w, v_j - v_i), (cohesion K_ij and its vector)
+        constexpr int kX = M == WCSPH ? 4 : 0, kS = kX + ((FL & F_XSPH) ? 4 : 0), kN = kS + ((FL & F_ST) ? 4 : 0);
+        if constexpr (kN > 0)
+            sweep<Q>(S, i, load,
+                     [&](const NbF& d) {
+                         const Pair p = pair_of(xx, xy, xz, d.x, k);
+                         Terms<kN> t;
+                         if constexpr (M == WCSPH) {
+                             t.v[0] = pressure_of(p, d);
+                             t.v[1] = p.dx;
+                             t.v[2] = p.dy;
+                             t.v[3] = p.dz;
+                         }
+                         if constexpr ((FL & F_XSPH) != 0) {
+                             t.v[kX] = xsph_of(p, d);
+                             t.v[kX + 1] = (double)d.v.x - vx0;
+                             t.v[kX + 2] = (double)d.v.y - vy0;
+                             t.v[kX + 3] = (double)d.v.z - vz0;
+                         }
+                         if constexpr ((FL & F_ST) != 0) {
+                             const bool on = p.r2 > 0.0;
+                             const double cs = cohesion_of(p, d);
+                             t.v[kS] = on ? kij_of(d) : 0.0;
+                             t.v[kS + 1] = on ? fma(cs, p.dx, -((double)ni.x - (double)d.n.x)) : 0.0;
+                             t.v[kS + 2] = on ? fma(cs, p.dy, -((double)ni.y - (double)d.n.y)) : 0.0;
+                             t.v[kS + 3] = on ? fma(cs, p.dz, -((double)ni.z - (double)d.n.z)) : 0.0;
+                         }
+                         return t;
+                     },
+                     [&](const Terms<kN>& t) {
+                         if constexpr (M == WCSPH) {
+                             px = fma(-t.v[0], t.v[1], px);
+                             py = fma(-t.v[0], t.v[2], py);
+                             pz = fma(-t.v[0], t.v[3], pz);
+                         }
+                         if constexpr ((FL & F_XSPH) != 0) {
+                             vx = fma(t.v[kX], t.v[kX + 1], vx);
+                             vy = fma(t.v[kX], t.v[kX + 2], vy);
+                             vz = fma(t.v[kX], t.v[kX + 3], vz);
+                         }
+                         if constexpr ((FL & F_ST) != 0) {
+                             sx = fma(t.v[kS], t.v[kS + 1], sx);
+                             sy = fma(t.v[kS], t.v[kS + 2], sy);
+                             sz = fma(t.v[kS], t.v[kS + 3], sz);
+                         }
+                     });
+        if ((threadIdx.x & 3) != 0) return;
+    }
     double ax = 0.0, ay = 0.0, az = 0.0;
     if (M == WCSPH) {
         const float4 gb = S.gb[i];
@@ -2146,29 +2283,30 @@ __global__ __launch_bounds__(kBlock) void k_df_predict(const DevScene* __restric
 // :349), 2 = divergence (kv_i += divErr_i alpha_i, :534).
 // `fused`: the sweep decides whether its iteration runs (loop_over); the warm
 // start makes the new time step dt and starts the density loop.
-template <int MODE>
-__global__ __launch_bounds__(kBlock) void k_df_vel(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
-                                                   int iter, int fused) {
-    const Chunk c = chunk_at(C, kBlock);
+template <int MODE, int Q>
+__global__ __launch_bounds__(kPartBlock<Q>) void k_df_vel(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                          int nchunks, int iter, int fused) {
+    Chunk c;
+    int i0, i;
+    if (!part_at<Q>(C, nchunks, c, i0, i)) return;
     const DevScene& S = T[c.scene];
     if (S.stall) return;
     Scalars* ss = S.ss;
     if (MODE == 1 && ended_before(ss->done, iter + 1)) return;
     if (MODE == 2 && ended_before(ss->doneV, iter + 1)) return;
-    const int i = c.begin + threadIdx.x;
     double dt = ss->dt;
     if (fused) {
         if (MODE == 0) {
             // (a large scene's finalize kernel has written dt itself)
             if (S.nChunks <= kFusedLoopChunks) dt = ss->dtNew;
-            if (c.begin == 0 && threadIdx.x == 0) {
+            if (i0 == 0 && threadIdx.x == 0) {
                 if (S.nChunks <= kFusedLoopChunks) ss->dt = dt;
                 ss->it = 0;
                 ss->done = loop_goes_on<LOOP_DENS>(S, ss, 0, 0.0) ? 0 : 1;
             }
         } else {
-            __shared__ double sh[kWaves];
-            if (loop_over<MODE == 1 ? LOOP_DENS : LOOP_DIV>(S, ss, c.begin == 0, iter + 1, sh)) return;
+            __shared__ double sh[kPartBlock<Q> / 64];
+            if (loop_over<MODE == 1 ? LOOP_DENS : LOOP_DIV, kPartBlock<Q>>(S, ss, i0 == 0, iter + 1, sh)) return;
         }
     }
     if (i >= S.n) return;
@@ -2179,15 +2317,18 @@ __global__ __launch_bounds__(kBlock) void k_df_vel(const DevScene* __restrict__ 
     const double si = xi.w;
     const double m = S.mD;
     double sx = 0.0, sy = 0.0, sz = 0.0;
-    sweep4(S, i, [&](uint32_t j) { return ld4o(S.xk, j); },
-           [&](uint32_t, const float4& xj) {
-               const double ks = si + (double)xj.w;
-               const PairG p = pairg_of(xx, xy, xz, xj, k);
-               const double g = sel(fabs(ks) > eps, m * ks * p.g, 0.0);
-               sx += g * p.dx;
-               sy += g * p.dy;
-               sz += g * p.dz;
-           });
+    sweep<Q>(S, i, [&](uint32_t j) { return ld4o(S.xk, j); },
+             [&](const float4& xj) {
+                 const double ks = si + (double)xj.w;
+                 const PairG p = pairg_of(xx, xy, xz, xj, k);
+                 return Terms<4>{{sel(fabs(ks) > eps, m * ks * p.g, 0.0), p.dx, p.dy, p.dz}};
+             },
+             [&](const Terms<4>& t) {
+                 sx = fma(t.v[0], t.v[1], sx);
+                 sy = fma(t.v[0], t.v[2], sy);
+                 sz = fma(t.v[0], t.v[3], sz);
+             });
+    if (Q > 1 && (threadIdx.x & 3) != 0) return;
     // every load of the epilogue is issued before its first store: a wait
     // for a load also waits for the stores issued before it
     const float4 gb = S.gb[i];
@@ -2239,10 +2380,12 @@ __global__ __launch_bounds__(kBlock) void k_df_vel(const DevScene* __restrict__ 
 // (:326, :511); 1/3 is the call at the end of an iteration.  Loop test
 // (:327, :512; the divergence loop is bounded by maxIterations):
 //   continue while (err > eta (eta_V/dt) or it < minIt) and it < maxIt.
-template <int MODE>
-__global__ __launch_bounds__(kBlock) void k_df_err(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
-                                                   int fused) {
-    const Chunk c = chunk_at(C, kBlock);
+template <int MODE, int Q>
+__global__ __launch_bounds__(kPartBlock<Q>) void k_df_err(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                          int nchunks, int fused) {
+    Chunk c;
+    int i0, i;
+    if (!part_at<Q>(C, nchunks, c, i0, i)) return;
     const DevScene& S = T[c.scene];
     if (S.stall) return;
     Scalars* ss = S.ss;
@@ -2250,12 +2393,10 @@ __global__ __launch_bounds__(kBlock) void k_df_err(const DevScene* __restrict__ 
     if (MODE == 1 && ss->done) return;
     if (MODE == 3 && ss->doneV) return;
     // `fused`: no finalize kernel counts the iteration
-    if (fused && MODE != 0 && c.begin == 0 && threadIdx.x == 0) {
+    if (fused && MODE != 0 && i0 == 0 && threadIdx.x == 0) {
         if (DENS) ss->it += 1;
         else ss->itV += 1;
     }
-    __shared__ double sh[kWaves];
-    const int i = c.begin + threadIdx.x;
     const KCoefD k = S.kd;
     const double dt = ss->dt;
     double e = 0.0;
@@ -2267,6 +2408,15 @@ __global__ __launch_bounds__(kBlock) void k_df_err(const DevScene* __restrict__ 
         // stores issued before it)
         const float drhof = S.drho[i], alf = S.alpha[i];
         const int ngr = DENS ? 20 : (int)S.ngrad[i];
+        // sum_j g_ij (u_i - u_j).(x_i - x_j), u_j in x.w and vyz
+        auto change = [&](double ux, double uy, double uz, double& sum) {
+            sweep<Q>(S, i, [&](uint32_t j) { XVP r; r.xv = ld4o(S.x, j); r.yz = ld2o(S.vyz, j); return r; },
+                     [&](const XVP& d) {
+                         const PairG p = pairg_of(xx, xy, xz, d.xv, k);
+                         return Terms<2>{{p.g, (ux - (double)d.xv.w) * p.dx + (uy - (double)d.yz.x) * p.dy + (uz - (double)d.yz.y) * p.dz}};
+                     },
+                     [&](const Terms<2>& t) { sum = fma(t.v[0], t.v[1], sum); });
+        };
         double dc;
         if (DENS) {
             // the density solve: x.w and vyz hold u, v holds v0 (see store_u)
@@ -2279,24 +2429,25 @@ __global__ __launch_bounds__(kBlock) void k_df_err(const DevScene* __restrict__ 
                 const float4 vi = ld4(S.v, i);
                 const double wx = vi.x, wy = vi.y, wz = vi.z;
                 double s0 = 0.0;
-                sweep4(S, i,
-                       [&](uint32_t j) { XVU r; r.x = ld4o(S.x, j); r.v = ld4o(S.v, j); r.yz = ld2o(S.vyz, j); return r; },
-                       [&](uint32_t, const XVU& d) {
-                           const PairG p = pairg_of(xx, xy, xz, d.x, k);
-                           s0 += p.g * ((wx - (double)d.v.x) * p.dx + (wy - (double)d.v.y) * p.dy + (wz - (double)d.v.z) * p.dz);
-                           su += p.g * ((ux - (double)d.x.w) * p.dx + (uy - (double)d.yz.x) * p.dy + (uz - (double)d.yz.y) * p.dz);
-                       });
+                sweep<Q>(S, i,
+                         [&](uint32_t j) { XVU r; r.x = ld4o(S.x, j); r.v = ld4o(S.v, j); r.yz = ld2o(S.vyz, j); return r; },
+                         [&](const XVU& d) {
+                             const PairG p = pairg_of(xx, xy, xz, d.x, k);
+                             return Terms<3>{{p.g,
+                                              (wx - (double)d.v.x) * p.dx + (wy - (double)d.v.y) * p.dy + (wz - (double)d.v.z) * p.dz,
+                                              (ux - (double)d.x.w) * p.dx + (uy - (double)d.yz.x) * p.dy + (uz - (double)d.yz.y) * p.dz}};
+                         },
+                         [&](const Terms<3>& t) {
+                             s0 = fma(t.v[0], t.v[1], s0);
+                             su = fma(t.v[0], t.v[2], su);
+                         });
                 const double d0 = S.mD * s0 + (wx * (double)gb.x + wy * (double)gb.y + wz * (double)gb.z);
-                ((gptr<double>)S.d0)[i] = d0;
+                if (Q == 1 || (threadIdx.x & 3) == 0) ((gptr<double>)S.d0)[i] = d0;
                 dc = d0;
                 // (d0Valid stays 0 until the next divergence sweep: other
                 // blocks of this launch test it)
             } else {
-                sweep4(S, i, [&](uint32_t j) { XVP r; r.xv = ld4o(S.x, j); r.yz = ld2o(S.vyz, j); return r; },
-                       [&](uint32_t, const XVP& d) {
-                           const PairG p = pairg_of(xx, xy, xz, d.xv, k);
-                           su += p.g * ((ux - (double)d.xv.w) * p.dx + (uy - (double)d.yz.x) * p.dy + (uz - (double)d.yz.y) * p.dz);
-                       });
+                change(ux, uy, uz, su);
                 dc = ((gptr<const double>)S.d0)[i];
             }
             dc += S.mD * su + (ux * (double)gb.x + uy * (double)gb.y + uz * (double)gb.z);
@@ -2305,37 +2456,40 @@ __global__ __launch_bounds__(kBlock) void k_df_err(const DevScene* __restrict__ 
             const double ux = vi.x, uy = vi.y, uz = vi.z;
             dc = 0.0;
             // the velocity sweep before this one wrote x.w and vyz
-            sweep4(S, i, [&](uint32_t j) { XVP r; r.xv = ld4o(S.x, j); r.yz = ld2o(S.vyz, j); return r; },
-                   [&](uint32_t, const XVP& d) {
-                       const PairG p = pairg_of(xx, xy, xz, d.xv, k);
-                       dc += p.g * ((ux - (double)d.xv.w) * p.dx + (uy - (double)d.yz.x) * p.dy + (uz - (double)d.yz.y) * p.dz);
-                   });
+            change(ux, uy, uz, dc);
             dc = S.mD * dc + (ux * (double)gb.x + uy * (double)gb.y + uz * (double)gb.z);
             // the divergence of the current velocities: the next step's D0
-            ((gptr<double>)S.d0)[i] = dc;
+            if (Q == 1 || (threadIdx.x & 3) == 0) ((gptr<double>)S.d0)[i] = dc;
         }
-        const double drho = (double)drhof;
-        const double rho = S.rho0D + drho;
-        const double al = alf;
-        double s;
-        if (DENS) {
-            const double drs = fmax(drho + dc * dt, 0.0);
-            S.drhoS[i] = (float)drs;
-            s = drs * al / (dt * dt * rho);
-            e = drs / S.rho0D;
-        } else {
-            const double de = (ngr < 20) ? 0.0 : fmax(dc, 0.0);
-            S.divErr[i] = (float)de;
-            s = de * al / (dt * rho);
-            e = de / S.rho0D;
+        if (Q == 1 || (threadIdx.x & 3) == 0) {
+            const double drho = (double)drhof;
+            const double rho = S.rho0D + drho;
+            const double al = alf;
+            double s;
+            if (DENS) {
+                const double drs = fmax(drho + dc * dt, 0.0);
+                S.drhoS[i] = (float)drs;
+                s = drs * al / (dt * dt * rho);
+                e = drs / S.rho0D;
+            } else {
+                const double de = (ngr < 20) ? 0.0 : fmax(dc, 0.0);
+                S.divErr[i] = (float)de;
+                s = de * al / (dt * rho);
+                e = de / S.rho0D;
+            }
+            S.xk[i] = make_float4(xi.x, xi.y, xi.z, (float)s);
         }
-        S.xk[i] = make_float4(xi.x, xi.y, xi.z, (float)s);
     }
-    const double bs = block_sum(e, sh);
     // `fused`: the error before the loop, which only the log has, waits in
     // the sort's scratch for the cell scan to add it up
-    double* const part = (fused && MODE == 0) ? (double*)S.perm : S.partial;
-    if (threadIdx.x == 0) part[c.begin / kBlock] = bs;
+    const bool log = fused && MODE == 0;
+    if constexpr (Q == 1) {
+        __shared__ double sh[kWaves];
+        const double bs = block_sum(e, sh);
+        if (threadIdx.x == 0) (log ? group_partial(S, 0) : S.partial)[i0 / kBlock] = bs;
+    } else {
+        group_error(S, log ? 0 : 1, i0, e);
+    }
 }
 
 // updatePositions (src/DFSPHSolver.cpp:216-236) fused with the cell key and
@@ -2530,17 +2684,15 @@ __device__ inline double quad_sum(double s, double t) {
 }
 __global__ __launch_bounds__(256) void k_pci_density_quad(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
                                                           int nchunks, int iter, int fused) {
-    const int slot = ((int)(blockIdx.x >> 3) / kWaves) * 8 + (int)(blockIdx.x & 7), sub = (int)(blockIdx.x >> 3) % kWaves;
-    if (slot >= nchunks) return;
-    const Chunk c = chunk_at(C, kBlock, slot, nchunks);
+    Chunk c;
+    int g0, i;
+    if (!part_at<4>(C, nchunks, c, g0, i)) return;
     const DevScene& S = T[c.scene];
     if (S.stall) return;
     Scalars* ss = S.ss;
     if (ended_before(ss->done, iter + 1)) return;
     __shared__ double sh[4];
     const int tid = threadIdx.x, lane = tid & 63, u = lane & 3;
-    const int g0 = c.begin + sub * kGroup;
-    const int i = g0 + (tid >> 2);
     if (fused && loop_over<LOOP_PCI, 256>(S, ss, g0 == 0, iter + 1, sh)) return;
     const int il = min(i, S.n - 1);
     const KCoefD k = S.kd;
@@ -2625,7 +2777,7 @@ __global__ __launch_bounds__(256) void k_pci_density_quad(const DevScene* __rest
     }
     __syncthreads();
     if (tid == 0) {
-        pci_wide_partial(S, fused ? ss->it : 0)[g0 >> 6] = fmax(fmax(sm[0], sm[1]), fmax(sm[2], sm[3]));
+        group_partial(S, fused ? ss->it & 1 : 0)[g0 >> 6] = fmax(fmax(sm[0], sm[1]), fmax(sm[2], sm[3]));
         if (S.pciShell) store_displacement(S, g0 >> 6, fmax(fmax(sm[4], sm[5]), fmax(sm[6], sm[7])), iter);
     }
 }
@@ -2634,9 +2786,12 @@ __global__ __launch_bounds__(256) void k_pci_density_quad(const DevScene* __rest
 // predicted densities (src/PCISPHSolver.cpp:297-358), then the prediction of
 // the next iteration (:122-149).  Runs after every k_pci_density, including
 // the one that ended the loop.
-__global__ __launch_bounds__(kBlock) void k_pci_pacc(const DevScene* __restrict__ T, const Chunk* __restrict__ C, int iter,
-                                                     int fused) {
-    const Chunk c = chunk_at(C, kBlock);
+template <int Q>
+__global__ __launch_bounds__(kPartBlock<Q>) void k_pci_pacc(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+                                                            int nchunks, int iter, int fused) {
+    Chunk c;
+    int i0, i;
+    if (!part_at<Q>(C, nchunks, c, i0, i)) return;
     const DevScene& S = T[c.scene];
     if (S.stall) return;
     Scalars* ss = S.ss;
@@ -2644,8 +2799,7 @@ __global__ __launch_bounds__(kBlock) void k_pci_pacc(const DevScene* __restrict_
     // the iteration; with `fused` the density sweep sets done instead, and the
     // iteration is counted here)
     if (fused ? ss->done : ss->it <= iter) return;
-    if (fused && c.begin == 0 && threadIdx.x == 0) ss->it += 1;
-    const int i = c.begin + threadIdx.x;
+    if (fused && i0 == 0 && threadIdx.x == 0) ss->it += 1;
     if (i >= S.n) return;
     const KCoefD k = S.kd;
     const double dt = ss->dt;
@@ -2654,14 +2808,17 @@ __global__ __launch_bounds__(kBlock) void k_pci_pacc(const DevScene* __restrict_
     const double pri = xi.w;
     const double m = S.mD;
     double ax = 0.0, ay = 0.0, az = 0.0;
-    sweep4(S, i, [&](uint32_t j) { return ld4(S.xk, j); },
-           [&](uint32_t, const float4& xj) {
-               const Pair p = pair_of(xx, xy, xz, xj, k);
-               const double g = m * (pri + (double)xj.w) * Gs_d(p, k);
-               ax -= g * p.dx;
-               ay -= g * p.dy;
-               az -= g * p.dz;
-           });
+    sweep<Q>(S, i, [&](uint32_t j) { return ld4(S.xk, j); },
+             [&](const float4& xj) {
+                 const Pair p = pair_of(xx, xy, xz, xj, k);
+                 return Terms<4>{{m * (pri + (double)xj.w) * Gs_d(p, k), p.dx, p.dy, p.dz}};
+             },
+             [&](const Terms<4>& t) {
+                 ax = fma(-t.v[0], t.v[1], ax);
+                 ay = fma(-t.v[0], t.v[2], ay);
+                 az = fma(-t.v[0], t.v[3], az);
+             });
+    if (Q > 1 && (threadIdx.x & 3) != 0) return;
     const float4 gs = S.gbs[i];
     ax -= pri * (double)gs.x;
     ay -= pri * (double)gs.y;
@@ -2734,8 +2891,8 @@ __global__ __launch_bounds__(kBlock) void k_pci_integrate(const DevScene* __rest
 // scenes still iterating, active[1] is the largest iteration count reached.
 enum FinKind { FIN_DT = 0, FIN_DENS0, FIN_DENS, FIN_DIV0, FIN_DIV, FIN_PCI };
 
-// wide: the partials of the PCISPH density sweep (k_pci_density_quad) or the
-// list build (k_build_quad) are one a group
+// wide: the kernel that wrote the partials gave a particle 4 lanes, so they are
+// one a group
 template <int KIND>
 __global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict__ T, int nscenes, int* active, int wide) {
     const int sc = blockIdx.x;
@@ -2746,10 +2903,11 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict_
     if ((KIND == FIN_DENS || KIND == FIN_PCI) && ss->done) return;
     if (KIND == FIN_DIV && ss->doneV) return;
     __shared__ double sh[kWaves];
-    const double red = (KIND == FIN_PCI && wide) ? scene_partial_max(pci_wide_partial(S, 0), S.nChunks * kWaves, sh)
-                       : (KIND == FIN_DT || KIND == FIN_PCI) ? scene_partial_max(S.partial, S.nChunks, sh)
-                       : KIND == FIN_DIV0 ? build_error_sum(S, wide, sh)
-                                          : scene_partial_sum(S.partial, S.nChunks, sh);
+    const double* const part = (KIND == FIN_PCI && wide) || KIND == FIN_DIV0 ? group_partial(S, 0)
+                               : wide ? group_partial(S, 1) : S.partial;
+    const double red = (KIND == FIN_DT || KIND == FIN_PCI) ? scene_partial_max(part, wide ? S.nChunks * kWaves : S.nChunks, sh)
+                       : wide ? scene_group_sum(part, S.nChunks, sh)
+                              : scene_partial_sum(part, S.nChunks, sh);
     if (threadIdx.x != 0) return;
     if (KIND == FIN_DT) {
         // the density solve's loop counters start here (counted by FIN_DENS0)
@@ -2833,7 +2991,8 @@ __global__ __launch_bounds__(kBlock) void k_loop_end(const DevScene* __restrict_
         // (the PCISPH integration has decided where the sweeps do)
         if (!over && !(END && KIND == LOOP_PCI)) over = loop_over<KIND>(S, ss, true, idx, sh, true);
         if (END && KIND == LOOP_DIV) {
-            const double avg0 = build_error_sum(S, S.nChunks <= kQuadChunks, sh) / (double)S.n;
+            const double avg0 = (S.nChunks <= kQuadChunks ? scene_group_sum(group_partial(S, 0), S.nChunks, sh)
+                                                          : scene_partial_sum(group_partial(S, 0), S.nChunks, sh)) / (double)S.n;
             if (threadIdx.x == 0) ss->avgErrV0 = avg0;
         }
         if (END && !over && tables.a) {
@@ -3201,6 +3360,9 @@ __global__ void k_load_state(const DevScene* __restrict__ T, int scene, const fl
 
 // ============================================================ launchers
 
+// a kernel with 4 lanes a particle over n chunks
+#define LAUNCH_QUAD(kern, n, stream, ...) \
+    hipLaunchKernelGGL(kern, dim3((n + 7) / 8 * 8 * kWaves), dim3(256), 0, stream, __VA_ARGS__)
 #define LAUNCH(kern, grid, stream, ...) hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), 0, stream, __VA_ARGS__)
 
 void launch_keys(hipStream_t st, const DevScene* T, const Chunk* C, int n, int* begin_active) {
@@ -3238,28 +3400,47 @@ void launch_build(hipStream_t st, int method, const DevScene* T, const Chunk* C,
     // PCISPH 64k 200.8 / 191.3, 97k 223.3 / 222.6, 125k 240.0 / 247.6; DFSPH 64k
     // 161.7 / 157.2, 97k 200.9 / 199.4, 125k 210.2 / 218.8.
     if (n <= (method == WCSPH ? kQuadChunksWcsph : kQuadChunks)) {
-        const int blocks = (n + 7) / 8 * 8 * kWaves;
-        if (method == DFSPH) hipLaunchKernelGGL(k_build_quad<DFSPH>, dim3(blocks), dim3(256), 0, st, T, C, n, fused);
-        else if (method == WCSPH) hipLaunchKernelGGL(k_build_quad<WCSPH>, dim3(blocks), dim3(256), 0, st, T, C, n, 0);
-        else hipLaunchKernelGGL(k_build_quad<PCISPH>, dim3(blocks), dim3(256), 0, st, T, C, n, 0);
+        if (method == DFSPH) LAUNCH_QUAD(k_build_quad<DFSPH>, n, st, T, C, n, fused);
+        else if (method == WCSPH) LAUNCH_QUAD(k_build_quad<WCSPH>, n, st, T, C, n, 0);
+        else LAUNCH_QUAD(k_build_quad<PCISPH>, n, st, T, C, n, 0);
         return;
     }
     if (method == DFSPH) LAUNCH(k_build<DFSPH>, n, st, T, C, fused);
     else if (method == WCSPH) LAUNCH(k_build<WCSPH>, n, st, T, C, 0);
     else LAUNCH(k_build<PCISPH>, n, st, T, C, 0);
 }
-void launch_normals(hipStream_t st, const DevScene* T, const Chunk* C, int n) { if (n) LAUNCH(k_normals, n, st, T, C); }
+// The sweeps with 4 lanes a particle where a launch leaves SIMDs without a
+// wavefront (us per step, one lane -> 4).  DFSPH without forces: 16 chunks 122
+// -> 102, 128: 136 -> 123, 183: 144 -> 138, 198: 149 -> 152, 250: 158 -> 160,
+// 290: 188 -> 177, 381: 203 -> 199, 432: 206 -> 212; the cohesion of DFSPH and
+// PCISPH has its lines in the same places (154: 221 -> 219, 198: 253 -> 254,
+// 333: 347 -> 346, 489: 398 -> 404).  Forces without cohesion, WCSPH: 16: 52
+// -> 42, 128: 55 -> 49, 333: 81 -> 79, 489: 94 -> 94; with it 16: 57 -> 50,
+// 128: 60 -> 58, 154: 68 -> 71 (128 registers and ~100 FP64 instructions a
+// pair, 12 terms to exchange).  PCISPH pressure force: 16: 118.9 -> 114.7,
+// 128: 125 -> 123, 141: 139 -> 140, 198: 152 -> 159.
+void launch_normals(hipStream_t st, const DevScene* T, const Chunk* C, int n) {
+    if (!n) return;
+    if (quad_sweep(n)) LAUNCH_QUAD(k_normals<4>, n, st, T, C, n);
+    else LAUNCH(k_normals<1>, n, st, T, C, n);
+}
 // The combinations of XSPH and cohesion get a kernel of their own; the two
 // viscosity forces that read rho_j as well, and batches whose scenes differ,
 // take the general one.
+template <int M, int FL>
+void launch_forces_f(hipStream_t st, const DevScene* T, const Chunk* C, int n) {
+    const bool quad = !(FL & F_ST) ? n <= kQuadForcesChunks : M == WCSPH ? n <= kQuadTensionChunks : quad_sweep(n);
+    if (quad) LAUNCH_QUAD((k_forces<M, FL, 4>), n, st, T, C, n);
+    else LAUNCH((k_forces<M, FL, 1>), n, st, T, C, n);
+}
 template <int M>
 void launch_forces_m(hipStream_t st, int flags, const DevScene* T, const Chunk* C, int n) {
     switch (flags < 0 ? -1 : flags & ~F_ADH) {
-        case 0: LAUNCH((k_forces<M, 0>), n, st, T, C); break;
-        case F_XSPH: LAUNCH((k_forces<M, F_XSPH>), n, st, T, C); break;
-        case F_ST: LAUNCH((k_forces<M, F_ST>), n, st, T, C); break;
-        case F_XSPH | F_ST: LAUNCH((k_forces<M, F_XSPH | F_ST>), n, st, T, C); break;
-        default: LAUNCH((k_forces<M, -1>), n, st, T, C);
+        case 0: launch_forces_f<M, 0>(st, T, C, n); break;
+        case F_XSPH: launch_forces_f<M, F_XSPH>(st, T, C, n); break;
+        case F_ST: launch_forces_f<M, F_ST>(st, T, C, n); break;
+        case F_XSPH | F_ST: launch_forces_f<M, F_XSPH | F_ST>(st, T, C, n); break;
+        default: LAUNCH((k_forces<M, -1, 1>), n, st, T, C, n);
     }
 }
 void launch_forces(hipStream_t st, int method, int flags, const DevScene* T, const Chunk* C, int n) {
@@ -3272,26 +3453,36 @@ void launch_dt(hipStream_t st, const DevScene* T, const Chunk* C, int n) { if (n
 void launch_df_predict(hipStream_t st, const DevScene* T, const Chunk* C, int n, int fused) {
     if (n) LAUNCH(k_df_predict, n, st, T, C, fused);
 }
+template <int MODE>
+void launch_df_vel_m(hipStream_t st, const DevScene* T, const Chunk* C, int n, int iter, int fused) {
+    if (quad_sweep(n)) LAUNCH_QUAD((k_df_vel<MODE, 4>), n, st, T, C, n, iter, fused);
+    else LAUNCH((k_df_vel<MODE, 1>), n, st, T, C, n, iter, fused);
+}
 void launch_df_vel(hipStream_t st, int mode, const DevScene* T, const Chunk* C, int n, int iter, int fused) {
     if (!n) return;
-    if (mode == 0) LAUNCH(k_df_vel<0>, n, st, T, C, iter, fused);
-    else if (mode == 1) LAUNCH(k_df_vel<1>, n, st, T, C, iter, fused);
-    else LAUNCH(k_df_vel<2>, n, st, T, C, iter, fused);
+    if (mode == 0) launch_df_vel_m<0>(st, T, C, n, iter, fused);
+    else if (mode == 1) launch_df_vel_m<1>(st, T, C, n, iter, fused);
+    else launch_df_vel_m<2>(st, T, C, n, iter, fused);
+}
+template <int MODE>
+void launch_df_err_m(hipStream_t st, const DevScene* T, const Chunk* C, int n, int fused) {
+    if (quad_sweep(n)) LAUNCH_QUAD((k_df_err<MODE, 4>), n, st, T, C, n, fused);
+    else LAUNCH((k_df_err<MODE, 1>), n, st, T, C, n, fused);
 }
 void launch_df_err(hipStream_t st, int mode, const DevScene* T, const Chunk* C, int n, int fused) {
     if (!n) return;
-    if (mode == 0) LAUNCH(k_df_err<0>, n, st, T, C, fused);
-    else if (mode == 1) LAUNCH(k_df_err<1>, n, st, T, C, fused);
-    else LAUNCH(k_df_err<3>, n, st, T, C, fused);
+    if (mode == 0) launch_df_err_m<0>(st, T, C, n, fused);
+    else if (mode == 1) launch_df_err_m<1>(st, T, C, n, fused);
+    else launch_df_err_m<3>(st, T, C, n, fused);
 }
 void launch_finalize(hipStream_t st, int kind, const DevScene* T, int nscenes, int* active, int nchunks) {
     if (!nscenes) return;
     switch (kind) {
         case FIN_DT: LAUNCH(k_finalize<FIN_DT>, nscenes, st, T, nscenes, active, 0); break;
-        case FIN_DENS0: LAUNCH(k_finalize<FIN_DENS0>, nscenes, st, T, nscenes, active, 0); break;
-        case FIN_DENS: LAUNCH(k_finalize<FIN_DENS>, nscenes, st, T, nscenes, active, 0); break;
+        case FIN_DENS0: LAUNCH(k_finalize<FIN_DENS0>, nscenes, st, T, nscenes, active, quad_sweep(nchunks)); break;
+        case FIN_DENS: LAUNCH(k_finalize<FIN_DENS>, nscenes, st, T, nscenes, active, quad_sweep(nchunks)); break;
         case FIN_DIV0: LAUNCH(k_finalize<FIN_DIV0>, nscenes, st, T, nscenes, active, nchunks <= kQuadChunks ? 1 : 0); break;
-        case FIN_DIV: LAUNCH(k_finalize<FIN_DIV>, nscenes, st, T, nscenes, active, 0); break;
+        case FIN_DIV: LAUNCH(k_finalize<FIN_DIV>, nscenes, st, T, nscenes, active, quad_sweep(nchunks)); break;
         default: LAUNCH(k_finalize<FIN_PCI>, nscenes, st, T, nscenes, active, nchunks <= kQuadPciChunks ? 1 : 0); break;
     }
 }
@@ -3303,11 +3494,13 @@ void launch_pci_density(hipStream_t st, const DevScene* T, const Chunk* C, int n
     // (us a step, one lane / four: 64,000 particles 191 / 156, 97k 221 / 199, 195k
     // 283 / 281, 373k 427 / 453)
     if (n <= kQuadPciChunks)
-        hipLaunchKernelGGL(k_pci_density_quad, dim3((n + 7) / 8 * 8 * kWaves), dim3(256), 0, st, T, C, n, iter, fused);
+        LAUNCH_QUAD(k_pci_density_quad, n, st, T, C, n, iter, fused);
     else LAUNCH(k_pci_density, n, st, T, C, iter, fused);
 }
 void launch_pci_pacc(hipStream_t st, const DevScene* T, const Chunk* C, int n, int iter, int fused) {
-    if (n) LAUNCH(k_pci_pacc, n, st, T, C, iter, fused);
+    if (!n) return;
+    if (n <= kQuadPaccChunks) LAUNCH_QUAD(k_pci_pacc<4>, n, st, T, C, n, iter, fused);
+    else LAUNCH(k_pci_pacc<1>, n, st, T, C, n, iter, fused);
 }
 void launch_pci_integrate(hipStream_t st, const DevScene* T, const Chunk* C, int n, int ahead) {
     if (n) LAUNCH(k_pci_integrate, n, st, T, C, ahead);

@@ -252,3 +252,39 @@ def test_four_lane_build_with_overflow_and_nan(ctx, crowd, method):
     assert np.isfinite(np.delete(alone.get(sphg.FIELD_X), 77, 0)).all()
     alone.close()
     mixed.close()
+
+
+@pytest.mark.parametrize("method", METHODS)
+@pytest.mark.parametrize("forces", ["none", "xsph", "cohesion", "xsph_cohesion"])
+@pytest.mark.parametrize("n", [1, 63, 65, 257, 3000])
+def test_sweeps_with_four_lanes_a_particle(ctx, crowd, method, forces, n):
+    """The sweeps of a small launch, of one scene and of a batch, give a
+    particle 4 lanes, those of a large one give it one: the same sums."""
+    r = 0.01
+    p = configs.small_scene(method, n_side=2, spacing=2 * r, **FORCES[forces]).params
+    x = block_of(n, 2 * r, 0.3, 7)
+    v = np.random.default_rng(8).uniform(-0.5, 0.5, x.shape).astype(np.float32)
+    b = sphg.sample_box((0.02, 0.02, 0.02), (0.6, 0.4, 0.45), 4 * r)
+    alone, pair, twin, mixed = [sphg.Scene(ctx, p, x, b, v) for _ in range(4)]
+    for _ in range(4):
+        alone.step(1)
+        ctx.batch_step([pair, twin], 1)
+        ctx.batch_step([mixed, crowd[method]], 1)
+        assert scalars(alone) == scalars(pair) == scalars(twin) == scalars(mixed)
+        assert same(alone, pair) and same(alone, twin) and same(alone, mixed)
+    for s in (alone, pair, twin, mixed):
+        s.close()
+
+
+@pytest.mark.parametrize("method", METHODS)
+@pytest.mark.parametrize("side", [32, 33, 36, 37, 40, 41, 46, 47])
+def test_lines_of_the_four_lane_sweeps(ctx, crowd, method, side):
+    """Both sides of 128, 192, 256 and 384 chunks of 256 particles."""
+    spec = configs.small_scene(method, n_side=side, spacing=0.02, **FORCES["xsph_cohesion"])
+    v = moving(spec, speed=0.3)
+    alone, mixed = [sphg.Scene(ctx, spec.params, spec.fluid, spec.boundary, v) for _ in range(2)]
+    alone.step(3)
+    ctx.batch_step([mixed, crowd[method]], 3)
+    assert scalars(alone) == scalars(mixed) and same(alone, mixed)
+    alone.close()
+    mixed.close()
