@@ -1016,28 +1016,32 @@ __global__ __launch_bounds__(kBlock) void k_bvolume_pack(const DevScene* __restr
 // the adhesion sum (src/AdhesionForce.h:46-59).
 // Fluid neighbors of particle i in two passes.  Pass 1 walks the 27 cells
 // with an FP32 distance test whose bound is 1e-5 above h^2 (FP32 rounding of
-// |x_i - x_j|^2 is ~1e-7 relative) and writes the survivors to the list.
-// Pass 2 runs the FP64 test and sums over those survivors only, compacting
-// the list in place.  Pass 2 thus iterates ~1.1x the neighbor count on
+// |x_i - x_j|^2 is ~1e-7 relative) and keeps the survivors in the list's
+// memory.  Pass 2 runs the FP64 test and sums over those survivors only and
+// writes the list in place.  Pass 2 thus iterates ~1.1x the neighbor count on
 // every lane of a wavefront, instead of running the FP64 path for every
 // candidate that any lane of the wavefront accepts.  A particle with more
 // survivors than list slots takes the one-pass walk over all candidates.
 //
-// Pass 1 reads its candidates from LDS.  The 64 particles of a wavefront are
-// sorted by cell, so they span one cell range [cF, cL], and each of a lane's
-// 9 candidate rows (cells c-1..c+1 of row (dy, dz)) lies inside that row's
-// range cF-1..cL+1 for the whole wavefront.  The wavefront copies those 9
-// particle ranges (~800 positions in a dense fluid, 12 B each) into LDS
-// once, instead of every lane loading its ~216 candidates from memory.  A
-// wavefront whose ranges exceed the stage reads global memory.
-#ifndef SPHG_BUILD_STAGE
-#define SPHG_BUILD_STAGE 1
-#endif
-constexpr int kWaveStage = SPHG_BUILD_STAGE ? 816 : 1;   // candidates per wavefront: 4 x 9.8 KB per block
-// Pass 1 reads a staged row 4 candidates at a time from one LDS address (the
-// 4 reads take immediate offsets); the last pass of a lane's row may read up
-// to 3 entries past the staged ones, so the stage has 3 more.
-constexpr int kWaveStagePad = kWaveStage + 3;
+// Both passes read positions from LDS.  The particles of a block are sorted by
+// cell, so they span one cell range [cF, cL], and each of a lane's 9 candidate
+// rows (cells c-1..c+1 of row (dy, dz)) lies inside that row's range
+// cF-1..cL+1 for the whole block.  The block copies those 9 particle ranges
+// (~2,450 positions in a dense fluid, 12 B each) into LDS once; rows past the
+// stage are read from global memory.
+//
+// FP64 math (~45 instructions a survivor, half of the vector instructions) and
+// pass 1's FP32 tests bound it, with 4 wavefronts a SIMD to cover LDS and the
+// velocity gathers.  With a stage a wavefront, a store for every candidate
+// step that some lane accepted (28 M write requests to L2 in a scene of 1M
+// particles, now 18 M) and pass 2's positions gathered from memory, it took
+// 255 us for 1M DFSPH particles, 166 for 600k WCSPH and 111 for 350k PCISPH;
+// now 207, 123 and 91.  5 wavefronts a SIMD (96 registers) spill in DFSPH: +85.
+// Candidates staged by a block: 9 rows of its own particles and two cells on
+// each side.  With 256 particles 31.9 KB, which leaves room for 5 blocks a
+// compute unit.  A row is read 8 candidates at a time, so up to 7 entries past
+// its end.
+constexpr int kBuildStage = 9 * (kBlock + 38), kBuildPad = 7;
 
 // FP64 test of a candidate: whether the reference's sums hold it, its W and
 // gradient factor, and whether its gradient is nonzero.
@@ -1145,8 +1149,9 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
     const Chunk c = chunk_at(C, kBlock);
     const DevScene& S = T[c.scene];
     if (S.stall) return;
-    __shared__ float2 sxy[kBlock / 64][kWaveStagePad];
-    __shared__ float sz[kBlock / 64][kWaveStagePad];
+    __shared__ float2 sxy[kBuildStage + kBuildPad];
+    __shared__ float sz[kBuildStage + kBuildPad];
+    __shared__ int sd[9];
     const int i = c.begin + threadIdx.x;
     const bool valid = i < S.n;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -1157,12 +1162,10 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
     const int ci = valid ? ldg(S.cell, (size_t)i) : 0;
     const int nx = S.nx, nxny = S.nx * S.ny;
 
-    // the wavefront's 9 row ranges: first particle and offset in the stage
-    const int wb = c.begin + (w << 6);
-    const bool live = wb < S.n;
+    // the block's 9 row ranges: first particle and offset in the stage
     int rfirst = 0, rcnt = 0;
-    if (live && lane < 9) {
-        const int cF = ldg(S.cell, (size_t)wb), cL = ldg(S.cell, (size_t)min(wb + 63, S.n - 1));
+    if (lane < 9) {
+        const int cF = ldg(S.cell, (size_t)c.begin), cL = ldg(S.cell, (size_t)min(c.begin + kBlock - 1, S.n - 1));
         const int off = (lane % 3 - 1) * nx + (lane / 3 - 1) * nxny;
         rfirst = ldg(S.cellStart, (size_t)(cF - 1 + off));
         rcnt = ldg(S.cellStart, (size_t)(cL + 2 + off)) - rfirst;
@@ -1181,33 +1184,32 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
         base[r + 1] = __builtin_amdgcn_readlane(incl, r);
     }
     // the leading rows that fit are staged (all 9 in a dense fluid); the
-    // rest of an oversized wavefront's rows are read from global memory
+    // others are read from global memory
     int nStaged = 0;
-    if (SPHG_BUILD_STAGE && live) {
 #pragma unroll
-        for (int r = 0; r < 9; ++r)
-            if (base[r + 1] <= kWaveStage) nStaged = r + 1;
-    }
+    for (int r = 0; r < 9; ++r)
+        if (base[r + 1] <= kBuildStage) nStaged = r + 1;
+    if (lane < 9 && w == 0) sd[lane] = incl - rcnt - rfirst;
     {
         // 4 loads per lane in flight before the first is written to LDS
         const int tot = base[nStaged];
-        for (int t0 = lane; t0 < tot; t0 += 256) {
+        for (int t0 = threadIdx.x; t0 < tot; t0 += 4 * kBlock) {
             float4 p[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const int t = t0 + 64 * u;
-                int f = first[0], b0 = 0;
+                const int t = t0 + kBlock * u;
+                int o = first[0];
 #pragma unroll
                 for (int q = 1; q < 9; ++q)
-                    if (t >= base[q]) { f = first[q]; b0 = base[q]; }
-                p[u] = (t < tot) ? ld4(S.x, (size_t)(f + (t - b0))) : make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (t >= base[q]) o = first[q] - base[q];
+                if (t < tot) p[u] = ld3o(S.x, (uint32_t)(o + t));
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const int t = t0 + 64 * u;
+                const int t = t0 + kBlock * u;
                 if (t < tot) {
-                    sxy[w][t] = make_float2(p[u].x, p[u].y);
-                    sz[w][t] = p[u].z;
+                    sxy[t] = make_float2(p[u].x, p[u].y);
+                    sz[t] = p[u].z;
                 }
             }
         }
@@ -1216,27 +1218,20 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
 
     uint32_t* L = list_of_w(S, valid ? i : (i & ~63));
     const int maxN = S.maxNbr;
-    // Pass 1 stores at byte offsets from the wavefront's group list (a
-    // uniform base, so each store takes the base + 32-bit offset form; a
-    // group's list is maxN KB).  The cursor is the offset of the lane's
-    // next slot with the lane field (bits 4..9) held at all ones: + 4 then
-    // carries from the last slot of a 4-slot block straight into the next
-    // block (bits 10 up), and the store address is the cursor with the lane
-    // field put back.  Its bits 2..3 and 10 up count the survivors.
+    // Pass 1's survivors go to the group's list memory (a uniform base, so
+    // each store takes the base + 32-bit offset form; a group's list is maxN
+    // KB): slot by slot, 64 lanes' entries in a row, so a store touches a few
+    // 64 B lines, until pass 2, which has read a block of 4 slots in all lanes
+    // before it writes that KB as 16 B a lane.  PCISPH has the shells of other
+    // lanes there and stores where the list has its slots.
     char* const Lw = (char*)(S.nbr + (size_t)__builtin_amdgcn_readfirstlane(i >> 6) * (size_t)maxN * kGroup);
-    constexpr uint32_t kLaneBits = 0x3F0u;
-    const uint32_t lane16 = (uint32_t)lane << 4;
-    uint32_t cur = kLaneBits;
-    const uint32_t curMax = kLaneBits | (slot_of(maxN - 1) << 2);
-    // past the last slot the particle takes the one-pass walk, which
-    // rewrites its list: the store is clamped to the last slot
-    auto put = [&](uint32_t j) {
-        const uint32_t a = (min(cur, curMax) & ~kLaneBits) | lane16;
-        cur = (cur + 4u) | kLaneBits;
-        *(gptr<uint32_t>)((gptr<char>)Lw + a) = j;
-    };
-    auto putSlot = [&](int s, uint32_t j) { *(gptr<uint32_t>)((gptr<char>)Lw + ((slot_of(s) << 2) | lane16)) = j; };
-    auto curCount = [&]() { return (int)(((cur >> 10) << 2) | ((cur >> 2) & 3u)); };
+    constexpr bool kRows = M != PCISPH;
+    // where all rows are staged a survivor is kept as its place in the stage
+    // and its row, and pass 2 reads its position there
+    const bool codes = nStaged == 9;
+    const uint32_t lane4 = (uint32_t)lane << 2, lane16 = (uint32_t)lane << 4;
+    auto putAt = [&](uint32_t at, uint32_t j) { *(gptr<uint32_t>)((gptr<char>)Lw + at) = j; };
+    auto putSlot = [&](int s, uint32_t j) { putAt((slot_of(s) << 2) | lane16, j); };
     // PCISPH: the shell, candidates within h + skin that are not in the
     // list, fills the slots from the last one down; it stands in for the
     // 27-cell walk of the predicted densities while it fits beside the list
@@ -1252,7 +1247,7 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
     const float4 vi = (M == DFSPH && valid) ? ld4(S.v, i) : make_float4(0.f, 0.f, 0.f, 0.f);
     const double ux = vi.x, uy = vi.y, uz = vi.z;
     // FP64 test and sums of one candidate that passed the FP32 test
-    int nc = 0;   // FP32 survivors of pass 1 (slots [0, nc) while pass 2 reads them)
+    int nc = 0;   // FP32 survivors of pass 1
     // a survivor the FP64 test rejects goes to the shell (PCISPH)
     auto toShell = [&](uint32_t j) {
         if (M != PCISPH) return;
@@ -1260,17 +1255,14 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
         else shellLost = true;
         ++ns;
     };
-    // pos: the slot the candidate was read from (-1: from the walk); an
-    // entry is written only where the compaction moves it
-    auto visit = [&](uint32_t j, const float4& xj, const float4& vj, int pos) {
+    auto visit = [&](uint32_t j, const float4& xj, const float4& vj) {
         const Pair p = pair_of(xx, xy, xz, xj, k);
         double g, wq;
         bool gnz;
         if (!member_of(p, xi, xj, S.hD, k, g, wq, gnz)) {
             toShell(j);
-            return;
+            return false;
         }
-        if (cnt < maxN && cnt != pos) stg(L, (size_t)slot_of(cnt), j);
         ++cnt;
         ngr += gnz ? 1 : 0;
         b.ws += wq;
@@ -1279,87 +1271,75 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
         b.sgz += g * p.dz;
         b.ssq += g * g * p.r2;
         if (M == DFSPH) b.dv += g * ((ux - (double)vj.x) * p.dx + (uy - (double)vj.y) * p.dy + (uz - (double)vj.z) * p.dz);
+        return true;
     };
     auto vel = [&](uint32_t j) { return (M == DFSPH) ? ld3o(S.v, j) : make_float4(0.f, 0.f, 0.f, 0.f); };
-    // pass 1 over the 27 cells as 9 rows (walk27 order), candidate positions
-    // from `fetch(j, row)`
-    // (4 candidates per pass: their loads are issued before the first test)
-    auto scanRow = [&](int r, int s0, int e0, int& nc, auto&& fetch) {
-        for (int j0 = s0; j0 < e0; j0 += 4) {
-            float3 q[4];
+    // Pass 1 over the 27 cells as 9 rows (walk27 order), up to 32 candidates
+    // of a row at a time: their tests go to the bits of a mask, 4 candidates'
+    // loads before the first test, and the survivors are then taken from it.
+    // Candidates past the row's end are read (staged rows: at most 3, inside
+    // the padded stage) and dropped with the mask's last bits.
+    // fetch(j): position of candidate j; self: the row may hold particle i;
+    // survivor j is kept as j + code
+    auto scanRow = [&](int s0, int e0, bool self, int code, auto&& fetch) {
+        for (int c0 = s0; c0 < e0; c0 += 32) {
+            const int nv = min(e0 - c0, 32);
+            uint32_t mo = 0, ms = 0;
+            int k0 = 0;
+            for (; k0 < nv; k0 += 8) {
+                float3 p[8];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) q[u] = fetch(min(j0 + u, e0 - 1), r);
-            bool ok[4], sh[4];
+                for (int u = 0; u < 8; ++u) p[u] = fetch(c0 + k0 + u);
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int j = j0 + u;
-                const float fx = xi.x - q[u].x, fy = xi.y - q[u].y, fz = xi.z - q[u].z;
-                const float d2 = fx * fx + fy * fy + fz * fz;
-                // evaluated without short-circuit: one exec-mask section
-                ok[u] = (j < e0) & (j != i) & (d2 <= hh);
-                sh[u] = (M == PCISPH) & (j < e0) & (j != i) & (d2 > hh) & (d2 <= hsk);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (ok[u]) {
-                    put((uint32_t)(j0 + u));
-                    if (M == PCISPH) ++nc;
+                for (int u = 0; u < 8; ++u) {
+                    const float fx = xi.x - p[u].x, fy = xi.y - p[u].y, fz = xi.z - p[u].z;
+                    if (M == PCISPH) {
+                        const float d2 = fx * fx + fy * fy + fz * fz;
+                        mo = mo + mo + (d2 <= hh ? 1u : 0u);
+                        ms = ms + ms + (d2 <= hsk ? 1u : 0u);
+                    } else {
+                        // the sign of d2 - hh
+                        mo = __builtin_amdgcn_alignbit(mo, __float_as_uint(fmaf(fz, fz, fmaf(fy, fy, fmaf(fx, fx, -hh)))), 31);
+                    }
                 }
-                if (M == PCISPH && sh[u]) {
+            }
+            // bit b: candidate jb + b
+            const int jb = c0 + nv - 32;
+            mo = __builtin_bitreverse32(mo >> (k0 - nv));
+            if (self && (uint32_t)(i - c0) < (uint32_t)nv) mo &= ~(1u << (i - jb));
+            if (M == PCISPH) {
+                ms = __builtin_bitreverse32(ms >> (k0 - nv)) & ~mo;
+                if (self && (uint32_t)(i - c0) < (uint32_t)nv) ms &= ~(1u << (i - jb));
+            }
+            // past the last slot the particle takes the one-pass walk
+            if (nc + __popc(mo) > maxN) {
+                nc = maxN + 1;
+                mo = 0;
+            }
+            uint32_t at = lane4 + (uint32_t)nc * 256u;
+            nc += __popc(mo);
+            int s = nc - __popc(mo);
+            while (mo) {
+                const uint32_t j = (uint32_t)(jb + code + __builtin_ctz(mo));
+                mo &= mo - 1u;
+                if (kRows) {
+                    putAt(at, j);
+                    at += 256u;
+                } else {
+                    putSlot(s++, j);
+                }
+            }
+            if (M == PCISPH)
+                while (ms) {
+                    const uint32_t j = (uint32_t)(jb + __builtin_ctz(ms));
+                    ms &= ms - 1u;
                     // below the list's slots only (list writes that later
                     // reach the shell are caught by nc + ns > maxN)
-                    if (nc + ns < maxN) putSlot(maxN - 1 - ns, (uint32_t)(j0 + u));
+                    if (nc + ns < maxN) putSlot(maxN - 1 - ns, j);
                     else shellLost = true;
                     ++ns;
                 }
-            }
         }
-    };
-    // pass 1 over a staged row: candidate j sits at stage entry
-    // j + base[r] - first[r], and one LDS address per row advances by 4
-    // entries a pass, so the candidates need no per-read index arithmetic.
-    // Entries past the lane's row end (at most 3, inside the padded stage)
-    // are read and fail the u < e0 - j0 test.  Particle i itself can only
-    // lie in row 4 (cells ci-1..ci+1): the other rows are offset by at
-    // least nx >= 3 cells, so only that row tests j != i.
-    auto scanRowLds = [&](auto rc, int s0, int e0, int& nc) {
-        constexpr int r = decltype(rc)::value;
-        const int t0 = s0 + (base[r] - first[r]);
-        const float2* pxy = &sxy[w][t0];
-        const float* pz = &sz[w][t0];
-        for (int j0 = s0; j0 < e0; j0 += 4, pxy += 4, pz += 4) {
-            float d2[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const float2 a = pxy[u];
-                const float fx = xi.x - a.x, fy = xi.y - a.y, fz = xi.z - pz[u];
-                d2[u] = fx * fx + fy * fy + fz * fz;
-            }
-            const int rem = e0 - j0;
-            bool ok[4], sh[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const bool in = (u == 0 || u < rem) & (r != 4 || j0 + u != i);
-                ok[u] = in & (d2[u] <= hh);
-                sh[u] = (M == PCISPH) & in & (d2[u] > hh) & (d2[u] <= hsk);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (ok[u]) {
-                    put((uint32_t)(j0 + u));
-                    if (M == PCISPH) ++nc;
-                }
-                if (M == PCISPH && sh[u]) {
-                    if (nc + ns < maxN) putSlot(maxN - 1 - ns, (uint32_t)(j0 + u));
-                    else shellLost = true;
-                    ++ns;
-                }
-            }
-        }
-    };
-    auto gblFetch = [&](int j, int) {
-        const float4 p = ld4(S.x, (size_t)j);
-        return make_float3(p.x, p.y, p.z);
     };
     if (valid) {
         // the 9 rows' ranges are loaded before pass 1's first list store:
@@ -1373,45 +1353,91 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
         }
         static_for<9>([&](auto rc) {
             constexpr int r = decltype(rc)::value;
-            if (r < nStaged) scanRowLds(rc, rs[r], re[r], nc);
-            else scanRow(r, rs[r], re[r], nc, gblFetch);
+            // particle i can only lie in row 4 (cells ci-1..ci+1): the other
+            // rows are offset by at least nx >= 3 cells
+            if (r < nStaged) {
+                const int d = base[r] - first[r];
+                scanRow(rs[r], re[r], r == 4, codes ? d + (r << 16) : 0, [&](int j) {
+                    const float2 a = sxy[j + d];
+                    return make_float3(a.x, a.y, sz[j + d]);
+                });
+            } else {
+                const int last = re[r] - 1;
+                scanRow(rs[r], re[r], r == 4, 0, [&](int j) {
+                    const float4 p = ld4(S.x, (size_t)min(j, last));
+                    return make_float3(p.x, p.y, p.z);
+                });
+            }
         });
-        nc = curCount();
         if (M == PCISPH && nc + ns > maxN) shellLost = true;
         if (nc <= maxN) {
             // 4 survivors per pass, their list entries and positions loaded
             // first; visit writes slots <= the one it reads, so entries
             // already loaded are not overwritten before use, and the next
             // block of entries is requested before this pass's data is used
-            v4u bn = ld_block(L, 0);
+            auto entries = [&](int q0) {
+                if (!kRows) return ld_block(L, q0 >> 2);
+                v4u e;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) e[u] = *(gptr<const uint32_t>)((gptr<char>)Lw + (lane4 + (uint32_t)(q0 + u) * 256u));
+                return e;
+            };
+            const uint32_t own0 = (uint32_t)i + (codes ? (uint32_t)(base[4] - first[4] + (4 << 16)) : 0u);
+            v4u bn = entries(0);
             for (int q0 = 0; q0 < nc; q0 += 4) {
                 // one block of 4 slots; those past the last survivor hold
-                // stale values and are replaced by the first (a valid index)
-                const v4u blk = bn;
-                const uint32_t jj[4] = {blk.x, q0 + 1 < nc ? blk.y : blk.x, q0 + 2 < nc ? blk.z : blk.x,
-                                        q0 + 3 < nc ? blk.w : blk.x};
+                // stale values and are replaced by the particle itself
+                v4u jj = bn;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) jj[u] = q0 + u < nc ? jj[u] : own0;
                 float4 xj[4], vj[4];
+                if (codes) {
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    xj[u] = ld3o(S.x, jj[u]);
-                    vj[u] = vel(jj[u]);
+                    for (int u = 0; u < 4; ++u) {
+                        const uint32_t t = jj[u] & 0xFFFFu;
+                        const float2 a = sxy[t];
+                        xj[u] = make_float4(a.x, a.y, sz[t], 0.f);
+                        jj[u] = t - (uint32_t)sd[jj[u] >> 16];
+                    }
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) xj[u] = ld3o(S.x, jj[u]);
                 }
-                bn = ld_block(L, (q0 + 4 < nc ? q0 + 4 : q0) >> 2);
-                asm volatile("" ::: "memory");
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (q0 + u < nc) visit(jj[u], xj[u], vj[u], q0 + u);
+                for (int u = 0; u < 4; ++u) vj[u] = vel(jj[u]);
+                bn = entries(q0 + 4 < nc ? q0 + 4 : q0);
+                asm volatile("" ::: "memory");
+                const int c0 = cnt;
+                bool in[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) in[u] = q0 + u < nc && visit(jj[u], xj[u], vj[u]);
+                // where the FP64 test has rejected none so far the whole block
+                // goes out, past the last survivor the particle itself
+                if (c0 == q0 && cnt - c0 == min(4, nc - q0)) {
+                    *(gptr<v4u>)((gptr<char>)Lw + ((uint32_t)q0 * 256u + lane16)) = jj;
+                } else {
+                    int to = c0;
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (in[u]) putSlot(to++, jj[u]);
+                }
             }
-        } else {
-            shellLost = true;
-            ns = maxN;   // toShell writes nothing from here on
-            walk27(S.cellStart, ci, nx, nxny, [&](int j) {
-                const float4 xj = ld4(S.x, j);
-                const float fx = xi.x - xj.x, fy = xi.y - xj.y, fz = xi.z - xj.z;
-                if (!(fx * fx + fy * fy + fz * fz <= hh) || j == i) return;
-                visit((uint32_t)j, xj, vel((uint32_t)j), -1);
-            });
         }
+    }
+    // (after every lane's pass 2: a walk writes its list where the others'
+    // survivors were)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const bool walk = valid && nc > maxN;
+    if (walk) {
+        shellLost = true;
+        ns = maxN;   // toShell writes nothing from here on
+        walk27(S.cellStart, ci, nx, nxny, [&](int j) {
+            const float4 xj = ld4(S.x, j);
+            const float fx = xi.x - xj.x, fy = xi.y - xj.y, fz = xi.z - xj.z;
+            if (!(fx * fx + fy * fy + fz * fz <= hh) || j == i) return;
+            if (visit((uint32_t)j, xj, vel((uint32_t)j)) && cnt <= maxN) putSlot(cnt - 1, (uint32_t)j);
+        });
     }
     // pad the list with the particle itself up to the group's longest list
     // rounded to 4 (a self term is exactly zero in every sweep)
@@ -1447,8 +1473,10 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
             b.az += sa * p.dz;
         }
     };
-    // the boundary survivors use the free slots between the list and the shell
-    const int room = max(0, maxN - own - ((M == PCISPH && !shellLost) ? ns : 0));
+    // the boundary survivors use the free slots between the list's blocks and
+    // the shell
+    const int free0 = (own + 3) & ~3;
+    const int room = max(0, maxN - free0 - ((M == PCISPH && !shellLost) ? ns : 0));
     int nbc = 0;
     bool nearBound = false;
     {
@@ -1475,7 +1503,7 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
                 for (int u = 0; u < 4; ++u) {
                     const float fx = xi.x - y[u].x, fy = xi.y - y[u].y, fz = xi.z - y[u].z;
                     if ((b0 + u < be[r]) & (fx * fx + fy * fy + fz * fz <= hh)) {
-                        if (nbc < room) putSlot(own + nbc, (uint32_t)(b0 + u));
+                        if (nbc < room) putSlot(free0 + nbc, (uint32_t)(b0 + u));
                         ++nbc;
                     }
                 }
@@ -1487,7 +1515,7 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
             float4 yb[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u)
-                yb[u] = ld4(S.xb, ldg((const uint32_t*)L, (size_t)slot_of(own + min(q0 + u, nbc - 1))));
+                yb[u] = ld4(S.xb, ldg((const uint32_t*)L, (size_t)slot_of(free0 + min(q0 + u, nbc - 1))));
 #pragma unroll
             for (int u = 0; u < 4; ++u)
                 if (q0 + u < nbc) bvisit(yb[u]);
@@ -1500,8 +1528,12 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
         });
     }
     // pad the list with the particle itself up to the group's longest list
-    // (overwrites the boundary survivors' slots)
-    for (int q = own; q < pad; ++q) stg(L, (size_t)slot_of(q), (uint32_t)i);
+    // (overwrites the boundary survivors' slots); pass 2 has filled the last
+    // block unless the FP64 test rejected a survivor
+    if (cnt != nc)
+        for (int q = own; q < free0; ++q) putSlot(q, (uint32_t)i);
+    const uint32_t self = (uint32_t)i;
+    for (int q = free0; q < pad; q += 4) *(gptr<v4u>)((gptr<char>)Lw + ((uint32_t)q * 256u + lane16)) = v4u{self, self, self, self};
     if (M == PCISPH) {
         if (pad + ns > maxN) shellLost = true;   // the padding reached the shell
         stg(S.nsh, (size_t)i, (uint16_t)(shellLost ? 0xFFFF : ns));
@@ -1519,10 +1551,9 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
 
 // The same build with 4 lanes a particle (part_at), for launches too small to
 // fill the chip: a lane takes every 4th candidate.  The block stages its
-// group's rows once, for the fluid and for the boundary.  Where k_build's wavefront walks its 27 cells 4 candidates at
-// a time in ~50 passes, each waiting on LDS, its four stores and, later, ~10
-// passes over the survivors' data in memory, a quad has a quarter of the
-// instructions in each of them.  Survivors keep their order (their slots are
+// group's rows once, for the fluid and for the boundary.  Where a lone
+// wavefront waits for LDS, list memory and gathers in each of k_build's ~50
+// steps, a quad has a quarter of the steps.  Survivors keep their order (their slots are
 // counted within the quad), and the four lanes' FP64 terms are added one after
 // the other in list order, in every lane alike, so the sums are k_build's bit
 // for bit. A step (most of the difference is this kernel): WCSPH 2,197
