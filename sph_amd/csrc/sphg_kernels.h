@@ -22,7 +22,7 @@ enum LoopKind { LOOP_DENS, LOOP_DIV, LOOP_PCI };
 constexpr int kFusedLoopChunks = 2048;
 // Launches of up to so many chunks give a particle 4 lanes (figures at the
 // launchers).
-constexpr int kQuadChunks = 320, kQuadChunksWcsph = 512;    // list build
+constexpr int kQuadChunks = 320;                            // list build
 constexpr int kQuadPciChunks = 768, kQuadPaccChunks = 128;  // PCISPH loop
 constexpr int kQuadForcesChunks = 384;                      // forces without cohesion
 constexpr int kQuadTensionChunks = 128;                     // WCSPH forces with cohesion

@@ -285,11 +285,11 @@ __device__ inline bool loop_over(const DevScene& S, Scalars* ss, bool firstChunk
     return true;
 }
 
-// A group's sum of e (in the first lane of each quad), formed as a wavefront
+// A group's sum of e (in the first lane of each of 64 quads), formed as a wavefront
 // that holds the 64 particles forms it.
 __device__ inline void group_error(const DevScene& S, int buffer, int i0, double e) {
     __shared__ double se[kGroup];
-    if ((threadIdx.x & 3) == 0) se[threadIdx.x >> 2] = e;
+    if (threadIdx.x < 256 && (threadIdx.x & 3) == 0) se[threadIdx.x >> 2] = e;
     __syncthreads();
     if (threadIdx.x < 64) {
         const double es = wave_sum(se[threadIdx.x]);
@@ -1549,21 +1549,39 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
     }
 }
 
-// The same build with 4 lanes a particle (part_at), for launches too small to
-// fill the chip: a lane takes every 4th candidate.  The block stages its
-// group's rows once, for the fluid and for the boundary.  Where a lone
-// wavefront waits for LDS, list memory and gathers in each of k_build's ~50
-// steps, a quad has a quarter of the steps.  Survivors keep their order (their slots are
-// counted within the quad), and the four lanes' FP64 terms are added one after
-// the other in list order, in every lane alike, so the sums are k_build's bit
-// for bit. A step (most of the difference is this kernel): WCSPH 2,197
-// particles 83 -> 55 us, 32,768 71 -> 54, PCISPH 4,845 239 -> 204, DFSPH 4,096
-// 149 -> 122, 35,805 184 -> 164.
-constexpr int kQuadStage = 816, kQuadPad = 8;    // fluid candidates staged (12 B each); reads past a row's end
-constexpr int kQuadBound = 512;                  // boundary candidates staged (16 B each)
+// The same build with 4 lanes a particle, for launches too small to fill the
+// chip.  A block of 8 wavefronts holds one list group (part_at): in wavefronts
+// 0-3 lane 4 q + u of wavefront w works on the fluid candidates 4 k + u of
+// particle 16 w + q, in 4-7 likewise on the boundary's.  The tests' signs are
+// shifted into a mask a lane, the quad's masks joined, so that every lane knows
+// the place of its survivors in the list; up to 126 of a particle wait in LDS,
+// as their place in the stage and their row.  The four lanes' FP64 terms are
+// added one after the other in list order, in every lane alike, so the sums are
+// k_build's bit for bit.
+//
+// A lone wavefront a SIMD bounds it: ~2,000 instructions of ~10 cycles for the
+// fluid, as many for the boundary of a particle in a corner, which ran one
+// after the other (23 us for 2,197 particles, 13 of them in the slowest block's
+// boundary, read from memory where the group's row ranges, with the walls
+// between two rows of fluid, exceeded the stage).  Side by side 14 us.  A step:
+// WCSPH 2,197 particles 83 -> 37 us (one lane 64), 32,768 71 -> 42, PCISPH
+// 4,845 154 -> 122, DFSPH 4,032 131 -> 94, 9,000 125 -> 100 (one lane -> 4).
+// DFSPH takes one survivor a lane at a time: two at once need 184 registers,
+// which leaves one block a compute unit (35,805 particles 164 us, now 152).
+constexpr int kQuadStage = 816;    // fluid candidates staged (12 B each)
+constexpr int kQuadBound = 512;    // boundary candidates staged (16 B each)
+constexpr int kQuadPad = 32;       // reads past a row's end
+// survivors of a particle kept in LDS, of the fluid (2 B each) and of the
+// boundary (4 B); odd numbers of dwords a particle
+constexpr int kQuadList = 126, kQuadBoundList = 45;
+// a particle's boundary sums (see BuildSums) from the wavefronts that form them
+struct BoundSums {
+    double bw, gx, gy, gz, sx, sy, sz, ax, ay, az;
+    int near;
+};
 
 template <int M>
-__global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__ T, const Chunk* __restrict__ C, int nchunks,
+__global__ __launch_bounds__(512, 4) void k_build_quad(const DevScene* __restrict__ T, const Chunk* __restrict__ C, int nchunks,
                                                     int fused) {
     Chunk c;
     int g0, i;   // the group's first particle and the lane's
@@ -1572,10 +1590,16 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
     if (S.stall) return;
     __shared__ float2 sxy[kQuadStage + kQuadPad];
     __shared__ float sz[kQuadStage + kQuadPad];
-    __shared__ float4 sb[kQuadBound];
+    __shared__ float4 sb[kQuadBound + kQuadPad];
+    __shared__ uint16_t sl[kGroup * kQuadList];
+    __shared__ uint32_t sbl[kGroup * kQuadBoundList];
+    __shared__ BoundSums sbs[kGroup];
+    __shared__ int sd[9];
     __shared__ int spad[4];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, u = lane & 3;
-    const int pl = tid >> 2;                 // the lane's particle in the group
+    const bool fluid = w < 4;                // wavefronts 0-3: the fluid, 4-7: the boundary
+    const int pl = (tid & 255) >> 2;         // the lane's particle in the group
+    i = g0 + pl;
     if (g0 >= S.n) {
         if (M == DFSPH && tid == 0) group_partial(S, 0)[g0 >> 6] = 0.0;
         return;
@@ -1591,14 +1615,15 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
     const double xx = xi.x, xy = xi.y, xz = xi.z;
     const double ux = vi.x, uy = vi.y, uz = vi.z;
     const int nx = S.nx, nxny = S.nx * S.ny;
-    // the particle's 9 rows, and the group's 9 fluid (lanes 0..8) and boundary
-    // (lanes 16..24) rows with their offsets in the stages
+    // the particle's 9 fluid or boundary rows, and the group's 9 fluid (lanes
+    // 0..8) and boundary (lanes 16..24) rows with their offsets in the stages
+    const int* const rows = fluid ? S.cellStart : S.bCellStart;
     int rs[9], re[9];
 #pragma unroll
     for (int r = 0; r < 9; ++r) {
         const int off = (r % 3 - 1) * nx + (r / 3 - 1) * nxny;
-        rs[r] = ldg(S.cellStart, (size_t)(ci - 1 + off));
-        re[r] = ldg(S.cellStart, (size_t)(ci + 2 + off));
+        rs[r] = ldg(rows, (size_t)(ci - 1 + off));
+        re[r] = ldg(rows, (size_t)(ci + 2 + off));
     }
     int rfirst = 0, rcnt = 0;
     const int lr = lane & 15;
@@ -1630,6 +1655,8 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
     for (int r = 0; r < 9; ++r)
         if (base[r + 1] <= kQuadStage) nStaged = r + 1;
     const int tot = base[nStaged];
+    const bool staged = nStaged == 9;
+    if (tid < 9) sd[tid] = incl - rcnt - rfirst;
     const bool bStaged = bbase[9] <= kQuadBound;
     const int btot = bStaged ? bbase[9] : 0;
     {
@@ -1640,22 +1667,18 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
                 if (t >= bs[q]) o = f[q] - bs[q];
             return o + t;
         };
-        float4 p[4], y[2];
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (tid + 256 * q < tot) p[q] = ld3o(S.x, (uint32_t)at(tid + 256 * q, first, base));
+        float4 p[2], y;
 #pragma unroll
         for (int q = 0; q < 2; ++q)
-            if (tid + 256 * q < btot) y[q] = ld4o(S.xb, (uint32_t)at(tid + 256 * q, bfirst, bbase));
+            if (tid + 512 * q < tot) p[q] = ld3o(S.x, (uint32_t)at(tid + 512 * q, first, base));
+        if (tid < btot) y = ld4o(S.xb, (uint32_t)at(tid, bfirst, bbase));
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (tid + 256 * q < tot) {
-                sxy[tid + 256 * q] = make_float2(p[q].x, p[q].y);
-                sz[tid + 256 * q] = p[q].z;
+        for (int q = 0; q < 2; ++q)
+            if (tid + 512 * q < tot) {
+                sxy[tid + 512 * q] = make_float2(p[q].x, p[q].y);
+                sz[tid + 512 * q] = p[q].z;
             }
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-            if (tid + 256 * q < btot) sb[tid + 256 * q] = y[q];
+        if (tid < btot) sb[tid] = y;
     }
     __syncthreads();
 
@@ -1672,6 +1695,29 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
     }
     int nc = 0, ns = 0;
     bool shellLost = false;
+    // up to 32 candidates c0.. of a row, every 4th of them a lane's: the sign
+    // of each test is shifted into bits 31, 27, .. of m.  Makes bit b stand for
+    // candidate c0 + b, of nv; m: the lane's own, returns the quad's
+    auto joined = [&](uint32_t& m, int nv) {
+        m = __builtin_bitreverse32((m & 0x88888888u) >> u);
+        if (nv < 32) m &= (1u << nv) - 1u;
+        uint32_t f = m | (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xF, 0xF, true);
+        return f | (uint32_t)__builtin_amdgcn_mov_dpp((int)f, 0x4E, 0xF, 0xF, true);
+    };
+    auto test = [&](float fx, float fy, float fz, float bound) {
+        return __float_as_uint(fmaf(fz, fz, fmaf(fy, fy, fmaf(fx, fx, -bound))));
+    };
+    uint16_t* const mine = sl + pl * kQuadList;
+    uint32_t* const bmine = sbl + pl * kQuadBoundList;
+    // the lane's survivors m of f, kept as code + bit from place n of the list on
+    auto keep = [&](uint32_t m, uint32_t f, int n, uint32_t code, auto* list, int most) {
+        while (m) {
+            const int b = __builtin_ctz(m);
+            m &= m - 1u;
+            const int to = n + __popc(f & ((1u << b) - 1u));
+            if (to < most) list[to] = (std::remove_pointer_t<decltype(list)>)(code + b);
+        }
+    };
     // pass 1: this lane's candidate j at squared distance d2 (in: it is one)
     auto scan = [&](bool in, uint32_t j, float d2) {
         const bool ok = in & (d2 <= hh);
@@ -1693,7 +1739,76 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
         if (ok) stg(L, (size_t)slot_of(min(nc + __popc(okb & below), maxN - 1)), j);
         nc += __popc(okb);
     };
-    if (valid) {
+    bool lds = staged;
+    if (fluid && valid && lds) {
+        static_for<9>([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
+            const int d = base[r] - first[r];
+            for (int c0 = rs[r]; c0 < re[r]; c0 += 32) {
+                const int nv = min(re[r] - c0, 32);
+                const float2* const pxy = sxy + c0 + d + u;
+                const float* const pz = sz + c0 + d + u;
+                uint32_t m = 0, ms = 0;
+                auto half = [&](int k0) {
+                    float2 a[4];
+                    float z[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        a[k] = pxy[k0 + 4 * k];
+                        z[k] = pz[k0 + 4 * k];
+                    }
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const float fx = xi.x - a[k].x, fy = xi.y - a[k].y, fz = xi.z - z[k];
+                        if (M == PCISPH) {
+                            const float d2 = fx * fx + fy * fy + fz * fz;
+                            m = (m << 4) | (d2 <= hh ? 8u : 0u);
+                            ms = (ms << 4) | (d2 <= hsk ? 8u : 0u);
+                        } else {
+                            m = __builtin_amdgcn_alignbit(m, test(fx, fy, fz, hh), 28);
+                        }
+                    }
+                };
+                half(0);
+                if (nv > 16) {
+                    half(16);
+                } else {
+                    m <<= 16;
+                    ms <<= 16;
+                }
+                uint32_t f = joined(m, nv);
+                // particle i itself can only lie in row 4
+                const uint32_t other = (r == 4 && (uint32_t)(i - c0) < 32u) ? ~(1u << (i - c0)) : ~0u;
+                f &= other;
+                m &= other;
+                keep(m, f, nc, (uint32_t)(c0 + d + (r << 12)), mine, kQuadList);
+                nc += __popc(f);
+                if (M == PCISPH) {
+                    uint32_t fs = joined(ms, nv);
+                    fs &= other & ~f;
+                    ms &= fs;
+                    while (ms) {
+                        const int b = __builtin_ctz(ms);
+                        ms &= ms - 1u;
+                        const int sn = ns + __popc(fs & ((1u << b) - 1u));
+                        // below the list's slots only (list writes that later
+                        // reach the shell are caught by nc + ns > maxN)
+                        if (nc + sn < maxN) stg(L, (size_t)slot_of(maxN - 1 - sn), (uint32_t)(c0 + b));
+                        else shellLost = true;
+                    }
+                    ns += __popc(fs);
+                }
+            }
+        });
+    }
+    // survivors that LDS does not hold, like those of rows that are not
+    // staged, go through the list's memory
+    if (fluid && lds && __any(nc > kQuadList && nc <= maxN)) {
+        lds = false;
+        nc = ns = 0;
+        shellLost = false;
+    }
+    if (fluid && valid && !lds) {
         static_for<9>([&](auto rc) {
             constexpr int r = decltype(rc)::value;
             const int s0 = rs[r], e0 = re[r];
@@ -1728,27 +1843,12 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
     int cnt = 0, ngr = 0;
     BuildSums b;
     if (M == PCISPH && nc + ns > maxN) shellLost = true;
-    if (valid && nc <= maxN) {
-        // pass 2, 8 survivors at a time
-        const uint32_t* const Lu = L + u;
-        uint32_t jn[2];
+    if (fluid && valid && nc <= maxN) {
+        // pass 2, kH survivors a lane at a time
+        constexpr int kH = M == DFSPH ? 1 : 2;
+        auto sums = [&](int q0, const uint32_t* j, const float4* xj, const float4* vj) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) jn[h] = ldg(Lu, (size_t)slot_of(min(4 * h, maxN - 4)));
-        for (int q0 = 0; q0 < nc; q0 += 8) {
-            uint32_t j[2];
-            float4 xj[2], vj[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                j[h] = (q0 + 4 * h + u < nc) ? jn[h] : (uint32_t)i;   // past the last: a valid index
-                xj[h] = ld3o(S.x, j[h]);
-                vj[h] = (M == DFSPH) ? ld3o(S.v, j[h]) : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-            // maxN is a multiple of 4: the block after the last is re-read
-#pragma unroll
-            for (int h = 0; h < 2; ++h) jn[h] = ldg(Lu, (size_t)slot_of(q0 + 8 + 4 * h < nc ? q0 + 8 + 4 * h : q0));
-            asm volatile("" ::: "memory");
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
+            for (int h = 0; h < kH; ++h) {
                 const int pos = q0 + 4 * h + u;
                 const Pair p = pair_of(xx, xy, xz, xj[h], k);
                 double g = 0.0, wq = 0.0;
@@ -1768,7 +1868,7 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
                 }
                 // an entry is written only where the compaction moves it
                 const int to = cnt + __popc(inb & below);
-                if (in && to != pos) stg(L, (size_t)slot_of(to), j[h]);
+                if (in && (lds || to != pos)) stg(L, (size_t)slot_of(to), j[h]);
                 cnt += __popc(inb);
                 ngr += __popc(quad_bits(in && gnz));
                 // in list order; a lane without a member adds zeros, which
@@ -1791,8 +1891,60 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
                     }
                 });
             }
+        };
+        if (lds) {
+            // the next survivors' velocities are requested before the current
+            // ones' sums; past the last survivor the particle itself
+            const uint32_t own0 = (uint32_t)(i + base[4] - first[4] + (4 << 12));
+            uint32_t e[kH], jn[kH];
+            float4 vn[kH];
+            auto next = [&](int q0) {
+#pragma unroll
+                for (int h = 0; h < kH; ++h) {
+                    const int pos = q0 + 4 * h + u;
+                    e[h] = pos < nc ? (uint32_t)mine[pos] : own0;
+                    jn[h] = (e[h] & 0xFFFu) - (uint32_t)sd[e[h] >> 12];
+                    vn[h] = (M == DFSPH) ? ld3o(S.v, jn[h]) : make_float4(0.f, 0.f, 0.f, 0.f);
+                }
+            };
+            next(0);
+            for (int q0 = 0; q0 < nc; q0 += 4 * kH) {
+                float4 xj[kH], vj[kH];
+                uint32_t j[kH];
+#pragma unroll
+                for (int h = 0; h < kH; ++h) {
+                    const uint32_t t = e[h] & 0xFFFu;
+                    const float2 a = sxy[t];
+                    xj[h] = make_float4(a.x, a.y, sz[t], 0.f);
+                    vj[h] = vn[h];
+                    j[h] = jn[h];
+                }
+                next(q0 + 4 * kH);
+                asm volatile("" ::: "memory");
+                sums(q0, j, xj, vj);
+            }
+        } else {
+            const uint32_t* const Lu = L + u;
+            uint32_t jn[kH];
+#pragma unroll
+            for (int h = 0; h < kH; ++h) jn[h] = ldg(Lu, (size_t)slot_of(min(4 * h, maxN - 4)));
+            for (int q0 = 0; q0 < nc; q0 += 4 * kH) {
+                uint32_t j[kH];
+                float4 xj[kH], vj[kH];
+#pragma unroll
+                for (int h = 0; h < kH; ++h) {
+                    j[h] = (q0 + 4 * h + u < nc) ? jn[h] : (uint32_t)i;   // past the last: a valid index
+                    xj[h] = ld3o(S.x, j[h]);
+                    vj[h] = (M == DFSPH) ? ld3o(S.v, j[h]) : make_float4(0.f, 0.f, 0.f, 0.f);
+                }
+                // maxN is a multiple of 4: the block after the last is re-read
+#pragma unroll
+                for (int h = 0; h < kH; ++h) jn[h] = ldg(Lu, (size_t)slot_of(q0 + 4 * kH + 4 * h < nc ? q0 + 4 * kH + 4 * h : q0));
+                asm volatile("" ::: "memory");
+                sums(q0, j, xj, vj);
+            }
         }
-    } else if (valid) {
+    } else if (fluid && valid) {
         // more survivors than slots: all candidates one after the other, the
         // four lanes alike
         shellLost = true;
@@ -1818,81 +1970,126 @@ __global__ __launch_bounds__(256) void k_build_quad(const DevScene* __restrict__
             }
         });
     }
+    const bool wantAdh = (S.flags & F_ADH) != 0;
+    const double rho0 = S.rho0D;
+    // boundary sums, 4 survivors of the FP32 test at a time
+    bool nearBound = false;
+    if (!fluid && bbase[9] > 0 && valid) {
+#pragma unroll
+        for (int r = 0; r < 9; ++r) nearBound |= re[r] > rs[r];
+        // one boundary candidate a lane
+        auto bsums = [&](bool ok, const float4& y) {
+            const Pair p = pair_of(xx, xy, xz, y, k);
+            const bool in = ok && p.q <= 1.0;
+            const double cb = in ? rho0 * (double)y.w : 0.0;
+            const double wq = in ? W_d(p.q, k) : 0.0;
+            const double g = in ? cb * G_d(p, k) : 0.0;
+            const double gs = (M == PCISPH && in) ? cb * Gs_d(p, k) : 0.0;
+            const double sa = (wantAdh && in && p.r2 > 0.0) ? cb * A_d(p.rl, k) * p.inv : 0.0;
+            static_for<4>([&](auto vc) {
+                constexpr int v = decltype(vc)::value;
+                const double dx = quad_lane<v>(p.dx), dy = quad_lane<v>(p.dy), dz = quad_lane<v>(p.dz);
+                b.bw = fma(quad_lane<v>(cb), quad_lane<v>(wq), b.bw);
+                const double gv = quad_lane<v>(g);
+                b.bgx = fma(gv, dx, b.bgx);
+                b.bgy = fma(gv, dy, b.bgy);
+                b.bgz = fma(gv, dz, b.bgz);
+                if (M == PCISPH) {
+                    const double gsv = quad_lane<v>(gs);
+                    b.sx2 = fma(gsv, dx, b.sx2);
+                    b.sy2 = fma(gsv, dy, b.sy2);
+                    b.sz2 = fma(gsv, dz, b.sz2);
+                }
+                if (wantAdh) {
+                    const double sav = quad_lane<v>(sa);
+                    b.ax = fma(sav, dx, b.ax);
+                    b.ay = fma(sav, dy, b.ay);
+                    b.az = fma(sav, dz, b.az);
+                }
+            });
+        };
+        int nb = 0;
+        // (survivors as places in the stage or in the boundary table)
+        static_for<9>([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
+            const int d = bStaged ? bbase[r] - bfirst[r] : 0;
+            for (int c0 = rs[r]; c0 < re[r]; c0 += 32) {
+                const int nv = min(re[r] - c0, 32);
+                uint32_t m = 0;
+                auto half = [&](int k0) {
+                    float4 y[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int t = c0 + u + k0 + 4 * k;
+                        if (bStaged) y[k] = sb[t + d];
+                        else y[k] = ld4(S.xb, (size_t)min(t, re[r] - 1));
+                    }
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        m = __builtin_amdgcn_alignbit(m, test(xi.x - y[k].x, xi.y - y[k].y, xi.z - y[k].z, hh), 28);
+                };
+                half(0);
+                if (nv > 16) half(16);
+                else m <<= 16;
+                const uint32_t f = joined(m, nv);
+                keep(m, f, nb, (uint32_t)(c0 + d), bmine, kQuadBoundList);
+                nb += __popc(f);
+            }
+        });
+        if (!__any(nb > kQuadBoundList)) {
+            for (int q0 = 0; q0 < nb; q0 += 4) {
+                const int pos = q0 + u;
+                const uint32_t t = bmine[min(pos, nb - 1)];
+                float4 y;
+                if (bStaged) y = sb[t];
+                else y = ld4(S.xb, (size_t)t);
+                bsums(pos < nb, y);
+            }
+        } else {
+            static_for<9>([&](auto rc) {
+                constexpr int r = decltype(rc)::value;
+                for (int b0 = rs[r]; b0 < re[r]; b0 += 4) {
+                    const int t = min(b0 + u, re[r] - 1);
+                    const float4 y = ld4(S.xb, (size_t)t);
+                    const float fx = xi.x - y.x, fy = xi.y - y.y, fz = xi.z - y.z;
+                    const bool ok = (b0 + u < re[r]) & (fx * fx + fy * fy + fz * fz <= hh);
+                    if (__any(ok)) bsums(ok, y);
+                }
+            });
+        }
+    }
+    if (!fluid && u == 0) sbs[pl] = BoundSums{b.bw, b.bgx, b.bgy, b.bgz, b.sx2, b.sy2, b.sz2, b.ax, b.ay, b.az, nearBound ? 1 : 0};
     // the list is padded with the particle itself up to the group's longest
     // list rounded to 4
     const int own = min(cnt, maxN);
     int pad = min((own + 3) & ~3, maxN);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) pad = max(pad, __shfl_xor(pad, o));
-    if (lane == 0) spad[w] = pad;
+    if (lane == 0 && fluid) spad[w] = pad;
     __syncthreads();
     pad = max(max(spad[0], spad[1]), max(spad[2], spad[3]));
-    const bool wantAdh = (S.flags & F_ADH) != 0;
-    const double rho0 = S.rho0D;
-    // boundary sums, 4 candidates at a time
-    bool nearBound = false;
-    if (bbase[9] > 0 && valid) {
-        int bs[9], be[9];
-#pragma unroll
-        for (int r = 0; r < 9; ++r) {
-            const int off = (r % 3 - 1) * nx + (r / 3 - 1) * nxny;
-            bs[r] = be[r] = 0;
-            if (bbase[r + 1] > bbase[r]) {
-                bs[r] = ldg(S.bCellStart, (size_t)(ci - 1 + off));
-                be[r] = ldg(S.bCellStart, (size_t)(ci + 2 + off));
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 9; ++r) nearBound |= be[r] > bs[r];
-        static_for<9>([&](auto rc) {
-            constexpr int r = decltype(rc)::value;
-            for (int b0 = bs[r]; b0 < be[r]; b0 += 4) {
-                const int t = min(b0 + u, be[r] - 1);
-                const float4 y = bStaged ? sb[t - bfirst[r] + bbase[r]] : ld4(S.xb, (size_t)t);
-                const float fx = xi.x - y.x, fy = xi.y - y.y, fz = xi.z - y.z;
-                const bool ok = (b0 + u < be[r]) & (fx * fx + fy * fy + fz * fz <= hh);
-                if (!__any(ok)) continue;
-                const Pair p = pair_of(xx, xy, xz, y, k);
-                const bool in = ok && p.q <= 1.0;
-                const double cb = in ? rho0 * (double)y.w : 0.0;
-                const double wq = in ? W_d(p.q, k) : 0.0;
-                const double g = in ? cb * G_d(p, k) : 0.0;
-                const double gs = (M == PCISPH && in) ? cb * Gs_d(p, k) : 0.0;
-                const double sa = (wantAdh && in && p.r2 > 0.0) ? cb * A_d(p.rl, k) * p.inv : 0.0;
-                static_for<4>([&](auto vc) {
-                    constexpr int v = decltype(vc)::value;
-                    const double dx = quad_lane<v>(p.dx), dy = quad_lane<v>(p.dy), dz = quad_lane<v>(p.dz);
-                    b.bw = fma(quad_lane<v>(cb), quad_lane<v>(wq), b.bw);
-                    const double gv = quad_lane<v>(g);
-                    b.bgx = fma(gv, dx, b.bgx);
-                    b.bgy = fma(gv, dy, b.bgy);
-                    b.bgz = fma(gv, dz, b.bgz);
-                    if (M == PCISPH) {
-                        const double gsv = quad_lane<v>(gs);
-                        b.sx2 = fma(gsv, dx, b.sx2);
-                        b.sy2 = fma(gsv, dy, b.sy2);
-                        b.sz2 = fma(gsv, dz, b.sz2);
-                    }
-                    if (wantAdh) {
-                        const double sav = quad_lane<v>(sa);
-                        b.ax = fma(sav, dx, b.ax);
-                        b.ay = fma(sav, dy, b.ay);
-                        b.az = fma(sav, dz, b.az);
-                    }
-                });
-            }
-        });
-    }
     double e = 0.0;
     if (M == PCISPH) {
         if (pad + ns > maxN) shellLost = true;   // the padding reached the shell
         shellLost = quad_bits(shellLost) != 0u;
     }
-    if (valid) {
+    if (fluid && valid) {
         for (int q = own + u; q < pad; q += 4) stg(L, (size_t)slot_of(q), (uint32_t)i);
         if (u == 0) {
             if (M == PCISPH) stg(S.nsh, (size_t)i, (uint16_t)(shellLost ? 0xFFFF : ns));
             if (pl == 0) stg(S.gcnt, (size_t)(i >> 6), (uint16_t)pad);
+            const BoundSums& f = sbs[pl];
+            b.bw = f.bw;
+            b.bgx = f.gx;
+            b.bgy = f.gy;
+            b.bgz = f.gz;
+            b.sx2 = f.sx;
+            b.sy2 = f.sy;
+            b.sz2 = f.sz;
+            b.ax = f.ax;
+            b.ay = f.ay;
+            b.az = f.az;
+            nearBound = f.near != 0;
             e = build_finish<M>(S, k, i, xi, vi, b, cnt, own, ngr, nearBound);
         }
     }
@@ -3391,9 +3588,11 @@ __global__ void k_load_state(const DevScene* __restrict__ T, int scene, const fl
 
 // ============================================================ launchers
 
-// a kernel with 4 lanes a particle over n chunks
-#define LAUNCH_QUAD(kern, n, stream, ...) \
-    hipLaunchKernelGGL(kern, dim3((n + 7) / 8 * 8 * kWaves), dim3(256), 0, stream, __VA_ARGS__)
+// a kernel with 4 lanes a particle over n chunks, with 4 wavefronts or BT
+// threads a block
+#define LAUNCH_QUAD_BT(kern, BT, n, stream, ...) \
+    hipLaunchKernelGGL(kern, dim3((n + 7) / 8 * 8 * kWaves), dim3(BT), 0, stream, __VA_ARGS__)
+#define LAUNCH_QUAD(kern, n, stream, ...) LAUNCH_QUAD_BT(kern, 256, n, stream, __VA_ARGS__)
 #define LAUNCH(kern, grid, stream, ...) hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), 0, stream, __VA_ARGS__)
 
 void launch_keys(hipStream_t st, const DevScene* T, const Chunk* C, int n, int* begin_active) {
@@ -3427,13 +3626,13 @@ void launch_bvolume(hipStream_t st, const DevScene* T, int scene, int nb, float*
 void launch_build(hipStream_t st, int method, const DevScene* T, const Chunk* C, int n, int fused) {
     if (!n) return;
     // Up to where 4 lanes a particle are faster (us a step; one lane / four):
-    // WCSPH 125k particles 97.2 / 93.9, 157k 110.6 / 109.0, 195k 115.4 / 119.5;
-    // PCISPH 64k 200.8 / 191.3, 97k 223.3 / 222.6, 125k 240.0 / 247.6; DFSPH 64k
-    // 161.7 / 157.2, 97k 200.9 / 199.4, 125k 210.2 / 218.8.
-    if (n <= (method == WCSPH ? kQuadChunksWcsph : kQuadChunks)) {
-        if (method == DFSPH) LAUNCH_QUAD(k_build_quad<DFSPH>, n, st, T, C, n, fused);
-        else if (method == WCSPH) LAUNCH_QUAD(k_build_quad<WCSPH>, n, st, T, C, n, 0);
-        else LAUNCH_QUAD(k_build_quad<PCISPH>, n, st, T, C, n, 0);
+    // WCSPH 16 chunks 64 / 36, 128 62 / 42, 232 71 / 63, 311 78 / 76, 381 83 /
+    // 87; PCISPH 16 136 / 105, 232 160 / 154, 311 180 / 180; DFSPH 16 123 / 94,
+    // 232 157 / 152, 311 178 / 178.
+    if (n <= kQuadChunks) {
+        if (method == DFSPH) LAUNCH_QUAD_BT(k_build_quad<DFSPH>, 512, n, st, T, C, n, fused);
+        else if (method == WCSPH) LAUNCH_QUAD_BT(k_build_quad<WCSPH>, 512, n, st, T, C, n, 0);
+        else LAUNCH_QUAD_BT(k_build_quad<PCISPH>, 512, n, st, T, C, n, 0);
         return;
     }
     if (method == DFSPH) LAUNCH(k_build<DFSPH>, n, st, T, C, fused);
