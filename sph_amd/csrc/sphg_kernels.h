@@ -23,7 +23,7 @@ constexpr int kFusedLoopChunks = 2048;
 // Launches of up to so many chunks give a particle 4 lanes (figures at the
 // launchers).
 constexpr int kQuadChunks = 320;                            // list build
-constexpr int kQuadPciChunks = 768, kQuadPaccChunks = 128;  // PCISPH loop
+constexpr int kQuadPciChunks = 768, kQuadSideChunks = 208, kQuadPaccChunks = 128;   // PCISPH loop
 constexpr int kQuadForcesChunks = 384;                      // forces without cohesion
 constexpr int kQuadTensionChunks = 128;                     // WCSPH forces with cohesion
 // The DFSPH sweeps, normals, cohesion: 4 lanes a particle take a block of 64

@@ -2903,14 +2903,17 @@ __global__ __launch_bounds__(kBlock) void k_pci_density(const DevScene* __restri
 // The same with 4 lanes a particle, a block per list group, for small
 // launches (see k_build_quad): a lane takes every 4th entry and the terms are
 // added in list order.  PCISPH, 4,845 particles: 28 -> 13 us a launch, the step
-// 204 -> 144.
+// 204 -> 144; then with a conservative FP32 test before the FP64 terms of the
+// boundary's candidates, most of which lie beyond h, and in the smallest
+// launches the boundary in 4 more wavefronts, the step 122 -> 110.
 template <int V>
 __device__ inline double quad_sum(double s, double t) {
     s += quad_lane<V>(t);
     if constexpr (V < 3) return quad_sum<V + 1>(s, t);
     else return s;
 }
-__global__ __launch_bounds__(256) void k_pci_density_quad(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+template <bool SIDE>
+__global__ __launch_bounds__(SIDE ? 512 : 256) void k_pci_density_quad(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
                                                           int nchunks, int iter, int fused) {
     Chunk c;
     int g0, i;
@@ -2919,24 +2922,52 @@ __global__ __launch_bounds__(256) void k_pci_density_quad(const DevScene* __rest
     if (S.stall) return;
     Scalars* ss = S.ss;
     if (ended_before(ss->done, iter + 1)) return;
-    __shared__ double sh[4];
+    constexpr int kBT = SIDE ? 512 : 256;
+    __shared__ double sh[kBT / 64], sbw[kGroup];
     const int tid = threadIdx.x, lane = tid & 63, u = lane & 3;
-    if (fused && loop_over<LOOP_PCI, 256>(S, ss, g0 == 0, iter + 1, sh)) return;
+    // SIDE: wavefronts 0-3 work on the fluid, 4-7 on the boundary
+    const bool fluid = !SIDE || tid < 256, bound = !SIDE || tid >= 256;
+    const int pl = (tid & 255) >> 2;
+    i = g0 + pl;
+    if (fused && loop_over<LOOP_PCI, kBT>(S, ss, g0 == 0, iter + 1, sh)) return;
     const int il = min(i, S.n - 1);
     const KCoefD k = S.kd;
+    const float hh = S.kc.hhi2 * (1.0f + 1e-5f);   // conservative FP32 test
     const bool useShell = S.pciShell && ss->shellBad == 0u;
-    double e = 0.0, dd = 0.0;
+    double e = 0.0, dd = 0.0, ws = 0.0;
+    const float4 xi = ld4(S.x, (size_t)il);
     if (i < S.n) {
-        const float4 xi = ld4(S.x, (size_t)il);
         const float4 di = ld4(S.xs, (size_t)il);
         const int ci = ldg(S.cell, (size_t)il);
         const int nx = S.nx, nxny = S.nx * S.ny;
-        const Rows br = rows_of(S.bCellStart, ci, nx, nxny);
         dd = (double)(di.x * di.x + di.y * di.y + di.z * di.z);
         const Predicted a{xi.x, xi.y, xi.z, di.x, di.y, di.z};
-        const int nsi = useShell ? (int)ldg(S.nsh, (size_t)i) : 0xFFFF;
-        double ws = 0.0;
-        if (nsi != 0xFFFF) {
+        const int nsi = useShell && fluid ? (int)ldg(S.nsh, (size_t)i) : 0xFFFF;
+        if (bound) {
+            const Rows br = rows_of(S.bCellStart, ci, nx, nxny);
+            double bw = 0.0;
+            static_for<9>([&](auto rc) {
+                constexpr int r = decltype(rc)::value;
+                for (int b0 = br.s[r]; b0 < br.e[r]; b0 += 8) {
+                    float4 y[2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) y[h] = ld4(S.xb, (size_t)min(b0 + 4 * h + u, br.e[r] - 1));
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const float fx = (xi.x - y[h].x) + di.x, fy = (xi.y - y[h].y) + di.y, fz = (xi.z - y[h].z) + di.z;
+                        const bool ok = (b0 + 4 * h + u < br.e[r]) & (fx * fx + fy * fy + fz * fz <= hh);
+                        if (!__any(ok)) continue;
+                        const double w = ok ? predicted_wb(a, y[h], k) : 0.0, vb = y[h].w;
+                        static_for<4>([&](auto vc) {
+                            constexpr int v = decltype(vc)::value;
+                            bw = fma(quad_lane<v>(vb), quad_lane<v>(w), bw);
+                        });
+                    }
+                }
+            });
+            if (u == 0) sbw[pl] = bw;
+        }
+        if (fluid && nsi != 0xFFFF) {
             ws = W_d(0.0, k);
             const uint32_t* const L = list_of(S, i);
             const int maxN = S.maxNbr;
@@ -2965,7 +2996,7 @@ __global__ __launch_bounds__(256) void k_pci_density_quad(const DevScene* __rest
             };
             run((int)ldg(S.nnb, (size_t)i), false);
             run(nsi, true);
-        } else {
+        } else if (fluid) {
             const Rows fr = rows_of(S.cellStart, ci, nx, nxny);
             static_for<9>([&](auto rc) {
                 constexpr int r = decltype(rc)::value;
@@ -2976,30 +3007,14 @@ __global__ __launch_bounds__(256) void k_pci_density_quad(const DevScene* __rest
                 }
             });
         }
-        double bw = 0.0;
-        static_for<9>([&](auto rc) {
-            constexpr int r = decltype(rc)::value;
-            for (int b0 = br.s[r]; b0 < br.e[r]; b0 += 8) {
-                float4 y[2];
-#pragma unroll
-                for (int h = 0; h < 2; ++h) y[h] = ld4(S.xb, (size_t)min(b0 + 4 * h + u, br.e[r] - 1));
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const double w = b0 + 4 * h + u < br.e[r] ? predicted_wb(a, y[h], k) : 0.0, vb = y[h].w;
-                    static_for<4>([&](auto vc) {
-                        constexpr int v = decltype(vc)::value;
-                        bw = fma(quad_lane<v>(vb), quad_lane<v>(w), bw);
-                    });
-                }
-            }
-        });
-        if (u == 0) e = pci_pressure(S, i, xi, ws, bw);
     }
+    __syncthreads();
+    if (fluid && i < S.n && u == 0) e = pci_pressure(S, i, xi, ws, sbw[pl]);
     // one partial a group
     e = wave_max(e);
     dd = wave_max(dd);
     __shared__ double sm[8];
-    if (lane == 0) {
+    if (lane == 0 && fluid) {
         sm[tid >> 6] = e;
         sm[4 + (tid >> 6)] = dd;
     }
@@ -3721,10 +3736,12 @@ void launch_df_positions(hipStream_t st, const DevScene* T, const Chunk* C, int 
 }
 void launch_pci_density(hipStream_t st, const DevScene* T, const Chunk* C, int n, int iter, int fused) {
     if (!n) return;
-    // (us a step, one lane / four: 64,000 particles 191 / 156, 97k 221 / 199, 195k
-    // 283 / 281, 373k 427 / 453)
-    if (n <= kQuadPciChunks)
-        LAUNCH_QUAD(k_pci_density_quad, n, st, T, C, n, iter, fused);
+    // (us a step, one lane / four: 64,000 particles 191 / 142, 97k 221 / 187, 195k
+    // 283 / 269, 287k 308 / 308, 351k spheres 412 / 440; four lanes, boundary after
+    // the fluid / beside it: 4,096 101 / 93, 51k 144 / 141, 59k 148.6 / 149.2, 64k
+    // 142 / 149)
+    if (n <= kQuadSideChunks) LAUNCH_QUAD_BT(k_pci_density_quad<true>, 512, n, st, T, C, n, iter, fused);
+    else if (n <= kQuadPciChunks) LAUNCH_QUAD(k_pci_density_quad<false>, n, st, T, C, n, iter, fused);
     else LAUNCH(k_pci_density, n, st, T, C, iter, fused);
 }
 void launch_pci_pacc(hipStream_t st, const DevScene* T, const Chunk* C, int n, int iter, int fused) {
