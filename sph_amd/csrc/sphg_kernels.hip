@@ -1568,7 +1568,7 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
 // 4,845 154 -> 122, DFSPH 4,032 131 -> 94, 9,000 125 -> 100 (one lane -> 4).
 // DFSPH takes one survivor a lane at a time: two at once need 184 registers,
 // which leaves one block a compute unit (35,805 particles 164 us, now 152).
-constexpr int kQuadStage = 816;    // fluid candidates staged (12 B each)
+constexpr int kQuadStage = 1024;   // fluid candidates staged (12 B each); ~800 are usual, more where a group goes on to the next row
 constexpr int kQuadBound = 512;    // boundary candidates staged (16 B each)
 constexpr int kQuadPad = 32;       // reads past a row's end
 // survivors of a particle kept in LDS, of the fluid (2 B each) and of the
