@@ -801,7 +801,8 @@ int lone_step(sphg_ctx* ctx, Batch& B, int from, int it, bool ask, uint32_t seq,
         const bool resumed = it > 0;
         auto run = [&] {
             iterate(it++);
-            if (large && !ask && it >= least) launch_loop_end(st, kind, 0, Tl, none, nullptr, 0, it);
+            // (where the host is about to ask, that launch decides)
+            if (large && it >= least && (!ask || it < ahead)) launch_loop_end(st, kind, 0, Tl, none, nullptr, 0, it);
         };
         if (resumed) run();
         else

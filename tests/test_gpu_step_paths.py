@@ -288,3 +288,20 @@ def test_lines_of_the_four_lane_sweeps(ctx, crowd, method, side):
     assert scalars(alone) == scalars(mixed) and same(alone, mixed)
     alone.close()
     mixed.close()
+
+
+@pytest.mark.parametrize("method", [sphg.DFSPH, sphg.PCISPH])
+def test_large_lone_scene_with_kernel_timing(ctx, method):
+    """While kernels are timed the host asks after the predicted iterations;
+    in a large scene those are decided one by one as well, so that a step
+    ends where its loop does."""
+    spec = configs.small_scene(method, n_side=(129, 64, 64), spacing=0.02, box=tuple(0.02 * (s + 4) for s in (129, 64, 64)))
+    v = moving(spec, speed=0.3)
+    plain, timed = [sphg.Scene(ctx, spec.params, spec.fluid, spec.boundary, v) for _ in range(2)]
+    plain.step(8)
+    ctx.kernel_timing(True)
+    timed.step(8)
+    ctx.kernel_timing(False)
+    assert scalars(plain) == scalars(timed) and same(plain, timed)
+    plain.close()
+    timed.close()
