@@ -498,7 +498,7 @@ __device__ inline void sweep4(const DevScene& S, int i, Load&& load, Body&& body
 // order (add).  Q = 1 is sweep4.  With 4 lanes a lane takes every 4th entry,
 // two at a time, and every lane adds the quad's terms one after the other, so
 // the sums are the same bit for bit.  A small launch has a wavefront or so a
-// SIMD, whose chain of gathers and FP64 math bounds it: a DFSPH sweep of 4,032
+// SIMD, whose chain of gathers and FP64 math bounds it: a DFSPH sweep of 4,096
 // particles 8 -> 5.3 us, the WCSPH forces of 2,197 15.8 -> 6.3.
 template <int Q, class Load, class Term, class Add>
 __device__ inline void sweep(const DevScene& S, int i, Load&& load, Term&& term, Add&& add) {
@@ -1567,7 +1567,7 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
 // boundary, read from memory where the group's row ranges, with the walls
 // between two rows of fluid, exceeded the stage).  Side by side 14 us.  A step:
 // WCSPH 2,197 particles 83 -> 37 us (one lane 64), 32,768 71 -> 42, PCISPH
-// 4,845 154 -> 122, DFSPH 4,032 131 -> 94, 9,000 125 -> 100 (one lane -> 4).
+// 4,845 154 -> 122, DFSPH 4,096 131 -> 94, 9,261 125 -> 100 (one lane -> 4).
 // DFSPH takes one survivor a lane at a time: two at once need 184 registers,
 // which leaves one block a compute unit (35,805 particles 164 us, now 152).
 constexpr int kQuadStage = 1024;   // fluid candidates staged (12 B each); ~800 are usual, more where a group goes on to the next row
@@ -2515,7 +2515,7 @@ __global__ __launch_bounds__(kBlock) void k_df_predict(const DevScene* __restric
 // start makes the new time step dt and starts the density loop.  FP64 math, 36
 // instructions a neighbor, bounds it (1M particles 50 us at 1.9-2.1 GHz); one
 // zeroing for both conditions on a term, of its size and of the distance, is 2
-// fewer (a step of 1M 918 -> 914 us, a batch of 825k 1222 -> 1215, 4,032 94 -> 92).
+// fewer (a step of 1M 918 -> 914 us, a batch of 825k 1222 -> 1215, 4,096 94 -> 92).
 template <int MODE, int Q>
 __global__ __launch_bounds__(kPartBlock<Q>) void k_df_vel(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
                                                           int nchunks, int iter, int fused) {
