@@ -797,7 +797,7 @@ int lone_step(sphg_ctx* ctx, Batch& B, int from, int it, bool ask, uint32_t seq,
     // launches iterations: the `ahead` predicted ones, then one at a time
     // while the scene's record says that the loop goes on
     auto loop = [&](int kind, int end, const DevScene* Tl, int ahead, int& reached, auto&& iterate) -> int {
-        const int least = kind == LOOP_DIV ? V.minItV : V.minIt;
+        const int least = std::min(kind == LOOP_DIV ? V.minItV : V.minIt, V.maxIt);
         const bool resumed = it > 0;
         auto run = [&] {
             iterate(it++);

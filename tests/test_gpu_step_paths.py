@@ -305,3 +305,23 @@ def test_large_lone_scene_with_kernel_timing(ctx, method):
     assert scalars(plain) == scalars(timed) and same(plain, timed)
     plain.close()
     timed.close()
+
+
+@pytest.mark.parametrize("method", [sphg.DFSPH, sphg.PCISPH])
+@pytest.mark.parametrize("loops", sorted(LOOPS))
+def test_large_lone_scene_loop_limits(ctx, method, loops):
+    """The loop limits of test_lone_scene_steps_like_one_of_a_batch where a
+    kernel of its own decides the loops."""
+    spec = configs.small_scene(method, n_side=(129, 64, 64), spacing=0.02, box=tuple(0.02 * (s + 4) for s in (129, 64, 64)),
+                               **LOOPS[loops])
+    other = configs.small_scene(method, n_side=5)
+    v = moving(spec, speed=0.3)
+    alone, mixed = [sphg.Scene(ctx, spec.params, spec.fluid, spec.boundary, v) for _ in range(2)]
+    extra = sphg.Scene(ctx, other.params, other.fluid, other.boundary)
+    for steps in (1, 5, 2):
+        alone.step(steps)
+        ctx.batch_step([mixed, extra], steps)
+        assert scalars(alone) == scalars(mixed)
+    assert same(alone, mixed)
+    for s in (alone, mixed, extra):
+        s.close()
