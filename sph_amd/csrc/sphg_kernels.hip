@@ -2959,6 +2959,16 @@ __global__ __launch_bounds__(SIDE ? 512 : 256) void k_pci_density_quad(const Dev
     const int pl = (tid & 255) >> 2;
     i = g0 + pl;
     if (fused && loop_over<LOOP_PCI, kBT>(S, ss, g0 == 0, iter + 1, sh)) return;
+    double* const part = group_partial(S, fused ? ss->it & 1 : 0);
+    if (g0 >= S.n) {
+        // past the active particles, of which a scene with emitters may have
+        // none: there is no particle to read
+        if (tid == 0) {
+            part[g0 >> 6] = 0.0;
+            if (S.pciShell) store_displacement(S, g0 >> 6, 0.0, iter);
+        }
+        return;
+    }
     const int il = min(i, S.n - 1);
     const KCoefD k = S.kd;
     const float hh = S.kc.hhi2 * (1.0f + 1e-5f);   // conservative FP32 test
@@ -3049,7 +3059,7 @@ __global__ __launch_bounds__(SIDE ? 512 : 256) void k_pci_density_quad(const Dev
     }
     __syncthreads();
     if (tid == 0) {
-        group_partial(S, fused ? ss->it & 1 : 0)[g0 >> 6] = fmax(fmax(sm[0], sm[1]), fmax(sm[2], sm[3]));
+        part[g0 >> 6] = fmax(fmax(sm[0], sm[1]), fmax(sm[2], sm[3]));
         if (S.pciShell) store_displacement(S, g0 >> 6, fmax(fmax(sm[4], sm[5]), fmax(sm[6], sm[7])), iter);
     }
 }

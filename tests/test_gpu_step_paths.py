@@ -325,3 +325,34 @@ def test_large_lone_scene_loop_limits(ctx, method, loops):
     assert same(alone, mixed)
     for s in (alone, mixed, extra):
         s.close()
+
+
+def inflow(method, budget, fluid=None, start=3.5, **kw):
+    """A scene with room for `budget` more particles, the first of which enter
+    after `start` steps; without `fluid` it begins empty."""
+    spec = configs.small_scene(method, n_side=4, **kw)
+    em = sphg.Emitter(type=sphg.EMITTER_CIRCLE, num_particles=budget, position=(0.5, 0.26, 0.5), velocity=5.0,
+                      rotation=(0.0, 1.0, 0.0, 0.0), start_time=start * spec.params.time_step, width=0.1, spacing=1.0)
+    return spec.params, np.zeros((0, 3), np.float32) if fluid is None else fluid, spec.boundary, [em]
+
+
+def test_pcisph_densities_without_active_particles(ctx):
+    """A group without an active particle, among them those of a scene that is
+    still empty, reads none and has an error of zero: the loop takes its
+    minimum of iterations."""
+    p, x, b, em = inflow(sphg.PCISPH, 600)
+    other = configs.small_scene(sphg.PCISPH, n_side=5)
+    alone, mixed = [sphg.Scene(ctx, p, x, b, emitters=em) for _ in range(2)]
+    extra = sphg.Scene(ctx, other.params, other.fluid, other.boundary)
+    empty = 0
+    for _ in range(30):
+        before = alone.n
+        alone.step(1)
+        ctx.batch_step([mixed, extra], 1)
+        assert alone.n == mixed.n and scalars(alone) == scalars(mixed) and same(alone, mixed)
+        if before == 0:
+            empty += 1
+            assert alone.scalars().iterations == p.min_iterations and alone.scalars().max_density_error == 0.0
+    assert empty >= 3 and alone.n > 7 and np.isfinite(alone.get(sphg.FIELD_X)).all()
+    for s in (alone, mixed, extra):
+        s.close()
