@@ -1179,6 +1179,15 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
     __shared__ float sz[kBuildStage + kBuildPad];
     __shared__ int sd[9];
     const int i = c.begin + threadIdx.x;
+    if (c.begin >= S.n) {
+        // past the active particles, of which a scene with emitters may have
+        // none: there is no cell to take the row ranges from
+        if (M == DFSPH && threadIdx.x == 0) {
+            group_partial(S, 0)[c.begin / kBlock] = 0.0;
+            if (c.begin == 0) build_starts_divergence(S, fused);
+        }
+        return;
+    }
     const bool valid = i < S.n;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const KCoefD k = S.kd;

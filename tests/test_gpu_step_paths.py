@@ -356,3 +356,24 @@ def test_pcisph_densities_without_active_particles(ctx):
     assert empty >= 3 and alone.n > 7 and np.isfinite(alone.get(sphg.FIELD_X)).all()
     for s in (alone, mixed, extra):
         s.close()
+
+
+@pytest.mark.parametrize("method", METHODS)
+@pytest.mark.parametrize("start", ["empty", "few"])
+def test_list_build_of_an_inflow_in_a_large_launch(ctx, crowd, method, start):
+    """Chunks cover a scene's capacity: those past its active particles, the
+    first one of an empty scene among them, have no cell to start from.  Alone
+    the lists are built with 4 lanes a particle, beside the crowd with one."""
+    fluid = None if start == "empty" else block_of(40, 0.05, 0.1, 9, at=0.1)
+    p, x, b, em = inflow(method, 1500, fluid)
+    alone, mixed = [sphg.Scene(ctx, p, x, b, emitters=em) for _ in range(2)]
+    first = alone.n
+    for _ in range(25):
+        alone.step(1)
+        ctx.batch_step([mixed, crowd[method]], 1)
+        assert alone.n == mixed.n and scalars(alone) == scalars(mixed)
+        if alone.n:
+            assert all(np.array_equal(a, m, equal_nan=True) for a, m in zip(build_fields(alone), build_fields(mixed)))
+    assert alone.n >= first + 7 and alone.capacity > 5 * 256 and np.isfinite(alone.get(sphg.FIELD_X)).all()
+    alone.close()
+    mixed.close()
