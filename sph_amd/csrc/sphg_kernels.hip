@@ -1907,21 +1907,24 @@ __global__ __launch_bounds__(512, 4) void k_build_quad(const DevScene* __restric
                 cnt += __popc(inb);
                 ngr += __popc(quad_bits(in && gnz));
                 // in list order; a lane without a member adds zeros, which
-                // change no sum
+                // change no sum (all factors: a rejected candidate's position
+                // or velocity may be infinite or NaN)
                 if (!in) g = wq = 0.0;
                 const double gg = g * g;
-                const double dot = (M == DFSPH) ? (ux - (double)vj[h].x) * p.dx + (uy - (double)vj[h].y) * p.dy +
-                                                      (uz - (double)vj[h].z) * p.dz
-                                                : 0.0;
+                double dx = p.dx, dy = p.dy, dz = p.dz, r2 = p.r2;
+                double dot = (M == DFSPH) ? (ux - (double)vj[h].x) * p.dx + (uy - (double)vj[h].y) * p.dy +
+                                                (uz - (double)vj[h].z) * p.dz
+                                          : 0.0;
+                if (!in) dx = dy = dz = r2 = dot = 0.0;
                 static_for<4>([&](auto vc) {
                     constexpr int v = decltype(vc)::value;
                     b.ws += quad_lane<v>(wq);
                     if (M == DFSPH) {
                         const double gv = quad_lane<v>(g);
-                        b.sgx = fma(gv, quad_lane<v>(p.dx), b.sgx);
-                        b.sgy = fma(gv, quad_lane<v>(p.dy), b.sgy);
-                        b.sgz = fma(gv, quad_lane<v>(p.dz), b.sgz);
-                        b.ssq = fma(quad_lane<v>(gg), quad_lane<v>(p.r2), b.ssq);
+                        b.sgx = fma(gv, quad_lane<v>(dx), b.sgx);
+                        b.sgy = fma(gv, quad_lane<v>(dy), b.sgy);
+                        b.sgz = fma(gv, quad_lane<v>(dz), b.sgz);
+                        b.ssq = fma(quad_lane<v>(gg), quad_lane<v>(r2), b.ssq);
                         b.dv = fma(gv, quad_lane<v>(dot), b.dv);
                     }
                 });
@@ -2021,9 +2024,11 @@ __global__ __launch_bounds__(512, 4) void k_build_quad(const DevScene* __restric
             const double g = in ? cb * G_d(p, k) : 0.0;
             const double gs = (M == PCISPH && in) ? cb * Gs_d(p, k) : 0.0;
             const double sa = (wantAdh && in && p.r2 > 0.0) ? cb * A_d(p.rl, k) * p.inv : 0.0;
+            // (every factor of a candidate that is none is zero)
+            const double px = in ? p.dx : 0.0, py = in ? p.dy : 0.0, pz = in ? p.dz : 0.0;
             static_for<4>([&](auto vc) {
                 constexpr int v = decltype(vc)::value;
-                const double dx = quad_lane<v>(p.dx), dy = quad_lane<v>(p.dy), dz = quad_lane<v>(p.dz);
+                const double dx = quad_lane<v>(px), dy = quad_lane<v>(py), dz = quad_lane<v>(pz);
                 b.bw = fma(quad_lane<v>(cb), quad_lane<v>(wq), b.bw);
                 const double gv = quad_lane<v>(g);
                 b.bgx = fma(gv, dx, b.bgx);
@@ -3005,7 +3010,7 @@ __global__ __launch_bounds__(SIDE ? 512 : 256) void k_pci_density_quad(const Dev
                         const float fx = (xi.x - y[h].x) + di.x, fy = (xi.y - y[h].y) + di.y, fz = (xi.z - y[h].z) + di.z;
                         const bool ok = (b0 + 4 * h + u < br.e[r]) & (fx * fx + fy * fy + fz * fz <= hh);
                         if (!__any(ok)) continue;
-                        const double w = ok ? predicted_wb(a, y[h], k) : 0.0, vb = y[h].w;
+                        const double w = ok ? predicted_wb(a, y[h], k) : 0.0, vb = ok ? (double)y[h].w : 0.0;
                         static_for<4>([&](auto vc) {
                             constexpr int v = decltype(vc)::value;
                             bw = fma(quad_lane<v>(vb), quad_lane<v>(w), bw);

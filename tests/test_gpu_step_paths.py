@@ -377,3 +377,52 @@ def test_list_build_of_an_inflow_in_a_large_launch(ctx, crowd, method, start):
     assert alone.n >= first + 7 and alone.capacity > 5 * 256 and np.isfinite(alone.get(sphg.FIELD_X)).all()
     alone.close()
     mixed.close()
+
+
+@pytest.mark.parametrize("method", METHODS)
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_nan_position_of_either_sign_stays_its_own_particles(ctx, crowd, method, sign):
+    """The list build's FP32 test by the sign of d^2 - h^2 lets a NaN with its
+    sign bit set through to the FP64 test, which rejects it: no other
+    particle's sums hold a trace of it, with 4 lanes a particle or one."""
+    r = 0.01
+    p = configs.small_scene(method, n_side=2, spacing=2 * r).params
+    b = sphg.sample_box((0.0, 0.0, 0.0), (0.4, 0.4, 0.4), 4 * r)
+    x = block_of(300, 2 * r, 0.1, 4, at=0.02)
+    v = np.random.default_rng(6).uniform(-0.3, 0.3, x.shape).astype(np.float32)
+    alone, mixed = [sphg.Scene(ctx, p, x, b) for _ in range(2)]
+    x = x.copy()
+    # the grid clamps it to the cells of the domain's corner, where the block is
+    x[77] = np.copysign(np.float32(np.nan), np.float32(sign))
+    for s in (alone, mixed):
+        s.set_state(x, v)
+    for _ in range(3):
+        alone.step(1)
+        ctx.batch_step([mixed, crowd[method]], 1)
+        assert all(np.array_equal(a, m, equal_nan=True) for a, m in zip(build_fields(alone), build_fields(mixed)))
+        assert all(np.isfinite(np.delete(f, 77, 0)).all() for f in fields(alone))
+    alone.close()
+    mixed.close()
+
+
+@pytest.mark.parametrize("speed", [np.inf, -np.nan])
+def test_velocity_of_a_rejected_candidate(ctx, speed):
+    """A candidate just past h passes the FP32 test and not the FP64 one: its
+    velocity, which may be anything, is in no divergence."""
+    r, side = 0.01, 10
+    p = configs.small_scene(sphg.DFSPH, n_side=2, spacing=2 * r).params
+    b = sphg.sample_box((0.0, 0.0, 0.0), (0.4, 0.4, 0.4), 4 * r)
+    x = block_of(side ** 3, 0.8, 0.0, 4, at=0.0) * 2 * r + np.float32(0.06)
+    face = ((side - 1) * side + side // 2) * side + side // 2
+    past = x[face] + np.array([p.support_radius * (1 + 2e-5), 0, 0])
+    x = np.concatenate([x, past[None]]).astype(np.float32)
+    v = np.random.default_rng(6).uniform(-0.3, 0.3, x.shape).astype(np.float32)
+    v[face] = (-1.0, 0.0, 0.0)   # into its neighbors
+    s = sphg.Scene(ctx, p, x, b)
+    out = []
+    for u in (0.0, speed):
+        v[-1] = u
+        s.set_state(x, v)
+        out.append([s.get(f)[:-1] for f in (sphg.FIELD_ALPHA, sphg.FIELD_DIVERR)])
+    assert out[0][1][face] > 0.0 and all(np.array_equal(a, c) for a, c in zip(*out))
+    s.close()
