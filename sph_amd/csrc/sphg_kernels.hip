@@ -108,6 +108,13 @@ __device__ inline bool part_at(const Chunk* C, int nchunks, Chunk& c, int& i0, i
 }
 template <int Q> constexpr int kPartBlock = Q == 1 ? kBlock : 256;
 
+// What the wavefront's lanes wrote before it is there for all of them, and none
+// goes on before the others have come here.
+__device__ inline void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // x of lane V of the quad
 template <int V>
 __device__ inline int quad_lane(int x) {
@@ -1404,65 +1411,69 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
                 });
             }
         });
-        if (M == PCISPH && nc + ns > maxN) shellLost = true;
-        if (nc <= maxN) {
-            // 4 survivors per pass, their list entries and positions loaded
-            // first; visit writes slots <= the one it reads, so entries
-            // already loaded are not overwritten before use, and the next
-            // block of entries is requested before this pass's data is used
-            auto entries = [&](int q0) {
-                if (!kRows) return ld_block(L, q0 >> 2);
-                v4u e;
+    }
+    if (M == PCISPH && nc + ns > maxN) shellLost = true;
+    // the lanes' survivors lie in common rows, and pass 2 writes lists over
+    // them: it starts after every lane's pass 1
+    wave_sync();
+    if (valid && nc <= maxN) {
+        // 4 survivors per pass, their list entries and positions loaded
+        // first; visit writes slots <= the one it reads, so entries
+        // already loaded are not overwritten before use, and the next
+        // block of entries is requested before this pass's data is used
+        auto entries = [&](int q0) {
+            if (!kRows) return ld_block(L, q0 >> 2);
+            v4u e;
 #pragma unroll
-                for (int u = 0; u < 4; ++u) e[u] = *(gptr<const uint32_t>)((gptr<char>)Lw + (lane4 + (uint32_t)(q0 + u) * 256u));
-                return e;
-            };
-            const uint32_t own0 = (uint32_t)i + (codes ? (uint32_t)(base[4] - first[4] + (4 << 16)) : 0u);
-            v4u bn = entries(0);
-            for (int q0 = 0; q0 < nc; q0 += 4) {
-                // one block of 4 slots; those past the last survivor hold
-                // stale values and are replaced by the particle itself
-                v4u jj = bn;
+            for (int u = 0; u < 4; ++u) e[u] = *(gptr<const uint32_t>)((gptr<char>)Lw + (lane4 + (uint32_t)(q0 + u) * 256u));
+            return e;
+        };
+        const uint32_t own0 = (uint32_t)i + (codes ? (uint32_t)(base[4] - first[4] + (4 << 16)) : 0u);
+        v4u bn = entries(0);
+        for (int q0 = 0; q0 < nc; q0 += 4) {
+            // one block of 4 slots; those past the last survivor hold
+            // stale values and are replaced by the particle itself
+            v4u jj = bn;
 #pragma unroll
-                for (int u = 0; u < 4; ++u) jj[u] = q0 + u < nc ? jj[u] : own0;
-                float4 xj[4], vj[4];
-                if (codes) {
+            for (int u = 0; u < 4; ++u) jj[u] = q0 + u < nc ? jj[u] : own0;
+            float4 xj[4], vj[4];
+            if (codes) {
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const uint32_t t = jj[u] & 0xFFFFu;
-                        const float2 a = sxy[t];
-                        xj[u] = make_float4(a.x, a.y, sz[t], 0.f);
-                        jj[u] = t - (uint32_t)sd[jj[u] >> 16];
-                    }
-                } else {
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) xj[u] = ld3o(S.x, jj[u]);
+                for (int u = 0; u < 4; ++u) {
+                    const uint32_t t = jj[u] & 0xFFFFu;
+                    const float2 a = sxy[t];
+                    xj[u] = make_float4(a.x, a.y, sz[t], 0.f);
+                    jj[u] = t - (uint32_t)sd[jj[u] >> 16];
                 }
+            } else {
 #pragma unroll
-                for (int u = 0; u < 4; ++u) vj[u] = vel(jj[u]);
-                bn = entries(q0 + 4 < nc ? q0 + 4 : q0);
-                asm volatile("" ::: "memory");
-                const int c0 = cnt;
-                bool in[4];
+                for (int u = 0; u < 4; ++u) xj[u] = ld3o(S.x, jj[u]);
+            }
 #pragma unroll
-                for (int u = 0; u < 4; ++u) in[u] = q0 + u < nc && visit(jj[u], xj[u], vj[u]);
-                // where the FP64 test has rejected none so far the whole block
-                // goes out, past the last survivor the particle itself
-                if (c0 == q0 && cnt - c0 == min(4, nc - q0)) {
-                    *(gptr<v4u>)((gptr<char>)Lw + ((uint32_t)q0 * 256u + lane16)) = jj;
-                } else {
-                    int to = c0;
+            for (int u = 0; u < 4; ++u) vj[u] = vel(jj[u]);
+            bn = entries(q0 + 4 < nc ? q0 + 4 : q0);
+            asm volatile("" ::: "memory");
+            // every lane has read this block's rows before one writes there
+            __builtin_amdgcn_wave_barrier();
+            const int c0 = cnt;
+            bool in[4];
 #pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        if (in[u]) putSlot(to++, jj[u]);
-                }
+            for (int u = 0; u < 4; ++u) in[u] = q0 + u < nc && visit(jj[u], xj[u], vj[u]);
+            // where the FP64 test has rejected none so far the whole block
+            // goes out, past the last survivor the particle itself
+            if (c0 == q0 && cnt - c0 == min(4, nc - q0)) {
+                *(gptr<v4u>)((gptr<char>)Lw + ((uint32_t)q0 * 256u + lane16)) = jj;
+            } else {
+                int to = c0;
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (in[u]) putSlot(to++, jj[u]);
             }
         }
     }
     // (after every lane's pass 2: a walk writes its list where the others'
     // survivors were)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     const bool walk = valid && nc > maxN;
     if (walk) {
         shellLost = true;
