@@ -3021,7 +3021,7 @@ __global__ __launch_bounds__(SIDE ? 512 : 256) void k_pci_density_quad(const Dev
                         const float fx = (xi.x - y[h].x) + di.x, fy = (xi.y - y[h].y) + di.y, fz = (xi.z - y[h].z) + di.z;
                         const bool ok = (b0 + 4 * h + u < br.e[r]) & (fx * fx + fy * fy + fz * fz <= hh);
                         if (!__any(ok)) continue;
-                        const double w = ok ? predicted_wb(a, y[h], k) : 0.0, vb = ok ? (double)y[h].w : 0.0;
+                        const double w = predicted_wb(a, y[h], k), vb = ok ? y[h].w : 0.f;   // (w is finite)
                         static_for<4>([&](auto vc) {
                             constexpr int v = decltype(vc)::value;
                             bw = fma(quad_lane<v>(vb), quad_lane<v>(w), bw);
