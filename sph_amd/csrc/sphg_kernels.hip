@@ -815,6 +815,8 @@ __device__ inline void density_error0(const DevScene& S) {
 // The first launch behind a DFSPH density loop whose end the position update
 // has decided (`tables` not null: a lone scene whose iterations were launched
 // ahead): whether it had ended.  If not, nothing behind this launch runs.
+// (`tables` are the tables that the kernel reads as T: its T is not restrict,
+// and what it needs of the scene it reads before its own stores.)
 __device__ inline bool sort_runs(const DevScene& S, const Chunk& c, const Tables& tables, int fused) {
     if (tables.a && !S.ss->done) {
         if (c.begin == 0 && threadIdx.x == 0) tables.a->stall = tables.b->stall = 1;
@@ -825,10 +827,12 @@ __device__ inline bool sort_runs(const DevScene& S, const Chunk& c, const Tables
 }
 
 // Per cell chunk: total count.
-__global__ __launch_bounds__(kBlock) void k_scan_sum(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+__global__ __launch_bounds__(kBlock) void k_scan_sum(const DevScene* T, const Chunk* __restrict__ C,
                                                      Tables tables, int fused) {
     const Chunk c = chunk_at(C, kCellChunk);
     const DevScene& S = T[c.scene];
+    const int ncells = S.ncells;
+    int *const cellCount = S.cellCount, *const cellChunkSum = S.cellChunkSum;
     if (S.stall || !sort_runs(S, c, tables, fused)) return;
     __shared__ double sh[kWaves];
     int acc = 0;
@@ -836,10 +840,10 @@ __global__ __launch_bounds__(kBlock) void k_scan_sum(const DevScene* __restrict_
 #pragma unroll
     for (int u = 0; u < kCellPerThread; ++u) {
         const int cc = c0 + u;
-        if (cc < S.ncells) acc += ldg(S.cellCount, (size_t)cc);
+        if (cc < ncells) acc += ldg(cellCount, (size_t)cc);
     }
     const double tot = block_sum((double)acc, sh);
-    if (threadIdx.x == 0) G(S.cellChunkSum)[c.begin / kCellChunk] = (int)tot;
+    if (threadIdx.x == 0) G(cellChunkSum)[c.begin / kCellChunk] = (int)tot;
 }
 
 __device__ inline int wave_incl_scan(int v) {
@@ -891,10 +895,12 @@ __global__ __launch_bounds__(kBlock) void k_scan_offsets(const DevScene* __restr
 // Integer sums, so all give the same offsets.
 enum ScanKind { SCAN_ONE, SCAN_TOTALS, SCAN_OFFSETS };
 template <int KIND>
-__global__ __launch_bounds__(kBlock) void k_scan_final(const DevScene* __restrict__ T, const Chunk* __restrict__ C,
+__global__ __launch_bounds__(kBlock) void k_scan_final(const DevScene* T, const Chunk* __restrict__ C,
                                                        Tables tables, int fused) {
     const Chunk c = chunk_at(C, kCellChunk);
     const DevScene& S = T[c.scene];
+    const int ncells = S.ncells, n = S.n;
+    int *const cellCount = S.cellCount, *const cellChunkSum = S.cellChunkSum, *const cellStart = S.cellStart;
     if (S.stall || !sort_runs(S, c, tables, fused)) return;
     __shared__ int wsum[kWaves];
     __shared__ int base;
@@ -904,7 +910,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_final(const DevScene* __restric
         if (KIND == SCAN_ONE) {
             constexpr int kU = 8;
             typedef int v4i __attribute__((ext_vector_type(4)));
-            const gptr<const v4i> cnt = (gptr<const v4i>)S.cellCount;
+            const gptr<const v4i> cnt = (gptr<const v4i>)cellCount;
             for (int t = threadIdx.x; t < c.begin / 4; t += kBlock * kU) {
                 v4i q[kU];
 #pragma unroll
@@ -913,7 +919,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_final(const DevScene* __restric
                 for (int u = 0; u < kU; ++u) acc += q[u].x + q[u].y + q[u].z + q[u].w;
             }
         } else {
-            for (int t = threadIdx.x; t < chunk; t += kBlock) acc += ldg(S.cellChunkSum, (size_t)t);
+            for (int t = threadIdx.x; t < chunk; t += kBlock) acc += ldg(cellChunkSum, (size_t)t);
         }
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o);
@@ -933,7 +939,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_final(const DevScene* __restric
 #pragma unroll
     for (int u = 0; u < kCellPerThread; ++u) {
         const int cc = c0 + u;
-        vals[u] = (cc < S.ncells) ? ldg(S.cellCount, (size_t)cc) : 0;
+        vals[u] = (cc < ncells) ? ldg(cellCount, (size_t)cc) : 0;
         local += vals[u];
     }
     const int incl = wave_incl_scan(local);
@@ -942,15 +948,15 @@ __global__ __launch_bounds__(kBlock) void k_scan_final(const DevScene* __restric
     __syncthreads();
     int woff = 0;
     for (int q = 0; q < w; ++q) woff += wsum[q];
-    int run = (KIND != SCAN_OFFSETS ? base : ldg(S.cellChunkSum, (size_t)chunk)) + woff + incl - local;
+    int run = (KIND != SCAN_OFFSETS ? base : ldg(cellChunkSum, (size_t)chunk)) + woff + incl - local;
 #pragma unroll
     for (int u = 0; u < kCellPerThread; ++u) {
         const int cc = c0 + u;
-        if (cc < S.ncells) G(S.cellStart)[cc] = run;
+        if (cc < ncells) G(cellStart)[cc] = run;
         run += vals[u];
     }
     // the chunk table covers ncells + 1 entries: the last one is the end
-    if (c0 <= S.ncells && S.ncells < c0 + kCellPerThread) G(S.cellStart)[S.ncells] = S.n;
+    if (c0 <= ncells && ncells < c0 + kCellPerThread) G(cellStart)[ncells] = n;
 }
 
 // Scatter the particle ids into their cells' slots (arrival order).  Each
@@ -3286,7 +3292,7 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const DevScene* __restrict_
 // Without `rec` it only decides, for a scene whose sweeps leave that to it;
 // idx: see loop_over.
 template <int KIND, bool END>
-__global__ __launch_bounds__(kBlock) void k_loop_end(const DevScene* __restrict__ T, Tables tables, StepRec* rec,
+__global__ __launch_bounds__(kBlock) void k_loop_end(const DevScene* T, Tables tables, StepRec* rec,
                                                      unsigned seq, int idx) {
     const DevScene& S = T[0];
     Scalars* ss = S.ss;
