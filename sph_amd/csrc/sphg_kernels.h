@@ -20,17 +20,21 @@ enum LoopKind { LOOP_DENS, LOOP_DIV, LOOP_PCI };
 // that may be the last (1M particles: 973 -> 960 us a step against finalize
 // kernels before the loops and after every iteration).
 constexpr int kFusedLoopChunks = 2048;
-// Launches of up to so many chunks give a particle 4 lanes (figures at the
-// launchers).
+// Launches of up to so many chunks of 256 particles give a particle 4 lanes
+// (figures at the launchers).
 constexpr int kQuadChunks = 320;                            // list build
 constexpr int kQuadPciChunks = 768, kQuadSideChunks = 208, kQuadPaccChunks = 128;   // PCISPH loop
 constexpr int kQuadForcesChunks = 384;                      // forces without cohesion
 constexpr int kQuadTensionChunks = 128;                     // WCSPH forces with cohesion
+constexpr int kQuadSweepChunks = 384;                       // the DFSPH sweeps, normals, cohesion
+// `nchunks` chunks, of kBlock particles, are at most `chunks256` of 256
+constexpr bool up_to(int chunks256, int nchunks) { return nchunks * kWaves <= chunks256 * 4; }
 // The DFSPH sweeps, normals, cohesion: 4 lanes a particle take a block of 64
 // particles ~1/3 of the time, and a sweep lasts as long as the compute units
 // (256) with the most blocks.
 constexpr bool quad_sweep(int nchunks) {
-    return nchunks <= 384 && (nchunks * kWaves + 255) / 256 <= 3 * ((nchunks + 255) / 256);
+    const int chunks = (nchunks * kWaves + 3) / 4;   // of 256
+    return up_to(kQuadSweepChunks, nchunks) && (chunks * 4 + 255) / 256 <= 3 * ((chunks + 255) / 256);
 }
 
 // begin_active: also the start of a WCSPH or PCISPH step, counting the

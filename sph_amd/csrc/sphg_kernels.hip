@@ -179,17 +179,25 @@ __device__ inline double block_max(double v, double* sh) {
 // loads of 4096 / kBlock of them are issued before the first is used, so
 // the loop waits on memory once for up to 4096 partials (a 1M-particle
 // scene's chunks) instead of once per partial.
+// Every kernel that forms a scene's sum adds in the same order, so a block of
+// more than kBlock threads leaves it to the first kBlock.  (One of fewer has at
+// most one partial a thread, which is that order: in the builds with blocks of
+// 512 the launches with 4 lanes a particle have up to 192 chunks.)
 constexpr int kPartU = 4096 / kBlock;
+template <int BT> constexpr int kSumThreads = BT < kBlock ? BT : kBlock;
+static_assert(kBlock <= 256 || kQuadSweepChunks <= kBlock, "at most 256 chunks, one partial a thread");
 template <int BT = kBlock>
 __device__ inline double scene_partial_sum(const double* partial, int n, double* sh) {
+    constexpr int kT = kSumThreads<BT>;
     double acc = 0.0;
-    for (int b = threadIdx.x; b < n; b += BT * kPartU) {
-        double v[kPartU];
+    if (kT == BT || threadIdx.x < kT)
+        for (int b = threadIdx.x; b < n; b += kT * kPartU) {
+            double v[kPartU];
 #pragma unroll
-        for (int u = 0; u < kPartU; ++u) v[u] = (b + u * BT < n) ? ldg(partial, (size_t)(b + u * BT)) : 0.0;
+            for (int u = 0; u < kPartU; ++u) v[u] = (b + u * kT < n) ? ldg(partial, (size_t)(b + u * kT)) : 0.0;
 #pragma unroll
-        for (int u = 0; u < kPartU; ++u) acc += v[u];
-    }
+            for (int u = 0; u < kPartU; ++u) acc += v[u];
+        }
     return block_sum<BT>(acc, sh);
 }
 // The same over n chunks whose 64-particle groups have a partial each (the
@@ -197,16 +205,18 @@ __device__ inline double scene_partial_sum(const double* partial, int n, double*
 // it.
 template <int BT = kBlock>
 __device__ inline double scene_group_sum(const double* partial, int n, double* sh) {
+    constexpr int kT = kSumThreads<BT>;
     double acc = 0.0;
-    for (int b = threadIdx.x; b < n; b += BT) {
-        double v[kWaves];
+    if (kT == BT || threadIdx.x < kT)
+        for (int b = threadIdx.x; b < n; b += kT) {
+            double v[kWaves];
 #pragma unroll
-        for (int k = 0; k < kWaves; ++k) v[k] = ldg(partial, (size_t)b * kWaves + k);
-        double r = v[0];
+            for (int k = 0; k < kWaves; ++k) v[k] = ldg(partial, (size_t)b * kWaves + k);
+            double r = v[0];
 #pragma unroll
-        for (int k = 1; k < kWaves; ++k) r += v[k];
-        acc += r;
-    }
+            for (int k = 1; k < kWaves; ++k) r += v[k];
+            acc += r;
+        }
     return block_sum<BT>(acc, sh);
 }
 template <int BT = kBlock>
@@ -285,7 +295,7 @@ __device__ inline bool loop_over(const DevScene& S, Scalars* ss, bool firstChunk
     if (KIND != LOOP_PCI)
         err = (quad_sweep(S.nChunks) ? scene_group_sum<BT>(group_partial(S, 1), S.nChunks, sh)
                                              : scene_partial_sum<BT>(S.partial, S.nChunks, sh)) / (double)S.n;
-    else if (S.nChunks <= kQuadPciChunks) err = scene_partial_max<BT>(group_partial(S, (it - 1) & 1), S.nChunks * kWaves, sh);
+    else if (up_to(kQuadPciChunks, S.nChunks)) err = scene_partial_max<BT>(group_partial(S, (it - 1) & 1), S.nChunks * kWaves, sh);
     else err = scene_partial_max<BT>(pci_partial(S, it - 1), S.nChunks, sh);
     if (loop_goes_on<KIND>(S, ss, it, err)) return false;
     if (firstChunk && threadIdx.x == 0) loop_ended<KIND>(ss, it, err, idx);
@@ -3304,7 +3314,7 @@ __global__ __launch_bounds__(kBlock) void k_loop_end(const DevScene* T, Tables t
         // (the PCISPH integration has decided where the sweeps do)
         if (!over && !(END && KIND == LOOP_PCI)) over = loop_over<KIND>(S, ss, true, idx, sh, true);
         if (END && KIND == LOOP_DIV) {
-            const double avg0 = (S.nChunks <= kQuadChunks ? scene_group_sum(group_partial(S, 0), S.nChunks, sh)
+            const double avg0 = (up_to(kQuadChunks, S.nChunks) ? scene_group_sum(group_partial(S, 0), S.nChunks, sh)
                                                           : scene_partial_sum(group_partial(S, 0), S.nChunks, sh)) / (double)S.n;
             if (threadIdx.x == 0) ss->avgErrV0 = avg0;
         }
@@ -3714,7 +3724,7 @@ void launch_build(hipStream_t st, int method, const DevScene* T, const Chunk* C,
     // WCSPH 16 chunks 64 / 36, 128 62 / 42, 232 71 / 63, 311 78 / 76, 381 83 /
     // 87; PCISPH 16 136 / 105, 232 160 / 154, 311 180 / 180; DFSPH 16 123 / 94,
     // 232 157 / 152, 311 178 / 178.
-    if (n <= kQuadChunks) {
+    if (up_to(kQuadChunks, n)) {
         if (method == DFSPH) LAUNCH_QUAD_BT(k_build_quad<DFSPH>, 512, n, st, T, C, n, fused);
         else if (method == WCSPH) LAUNCH_QUAD_BT(k_build_quad<WCSPH>, 512, n, st, T, C, n, 0);
         else LAUNCH_QUAD_BT(k_build_quad<PCISPH>, 512, n, st, T, C, n, 0);
@@ -3744,7 +3754,7 @@ void launch_normals(hipStream_t st, const DevScene* T, const Chunk* C, int n) {
 // take the general one.
 template <int M, int FL>
 void launch_forces_f(hipStream_t st, const DevScene* T, const Chunk* C, int n) {
-    const bool quad = !(FL & F_ST) ? n <= kQuadForcesChunks : M == WCSPH ? n <= kQuadTensionChunks : quad_sweep(n);
+    const bool quad = !(FL & F_ST) ? up_to(kQuadForcesChunks, n) : M == WCSPH ? up_to(kQuadTensionChunks, n) : quad_sweep(n);
     if (quad) LAUNCH_QUAD((k_forces<M, FL, 4>), n, st, T, C, n);
     else LAUNCH((k_forces<M, FL, 1>), n, st, T, C, n);
 }
@@ -3796,9 +3806,9 @@ void launch_finalize(hipStream_t st, int kind, const DevScene* T, int nscenes, i
         case FIN_DT: LAUNCH(k_finalize<FIN_DT>, nscenes, st, T, nscenes, active, 0); break;
         case FIN_DENS0: LAUNCH(k_finalize<FIN_DENS0>, nscenes, st, T, nscenes, active, quad_sweep(nchunks)); break;
         case FIN_DENS: LAUNCH(k_finalize<FIN_DENS>, nscenes, st, T, nscenes, active, quad_sweep(nchunks)); break;
-        case FIN_DIV0: LAUNCH(k_finalize<FIN_DIV0>, nscenes, st, T, nscenes, active, nchunks <= kQuadChunks ? 1 : 0); break;
+        case FIN_DIV0: LAUNCH(k_finalize<FIN_DIV0>, nscenes, st, T, nscenes, active, up_to(kQuadChunks, nchunks) ? 1 : 0); break;
         case FIN_DIV: LAUNCH(k_finalize<FIN_DIV>, nscenes, st, T, nscenes, active, quad_sweep(nchunks)); break;
-        default: LAUNCH(k_finalize<FIN_PCI>, nscenes, st, T, nscenes, active, nchunks <= kQuadPciChunks ? 1 : 0); break;
+        default: LAUNCH(k_finalize<FIN_PCI>, nscenes, st, T, nscenes, active, up_to(kQuadPciChunks, nchunks) ? 1 : 0); break;
     }
 }
 void launch_df_positions(hipStream_t st, const DevScene* T, const Chunk* C, int n, int* active, int ahead) {
@@ -3810,13 +3820,13 @@ void launch_pci_density(hipStream_t st, const DevScene* T, const Chunk* C, int n
     // 283 / 269, 287k 308 / 308, 351k spheres 412 / 440; four lanes, boundary after
     // the fluid / beside it: 4,096 101 / 93, 51k 144 / 141, 59k 148.6 / 149.2, 64k
     // 142 / 149)
-    if (n <= kQuadSideChunks) LAUNCH_QUAD_BT(k_pci_density_quad<true>, 512, n, st, T, C, n, iter, fused);
-    else if (n <= kQuadPciChunks) LAUNCH_QUAD(k_pci_density_quad<false>, n, st, T, C, n, iter, fused);
+    if (up_to(kQuadSideChunks, n)) LAUNCH_QUAD_BT(k_pci_density_quad<true>, 512, n, st, T, C, n, iter, fused);
+    else if (up_to(kQuadPciChunks, n)) LAUNCH_QUAD(k_pci_density_quad<false>, n, st, T, C, n, iter, fused);
     else LAUNCH(k_pci_density, n, st, T, C, iter, fused);
 }
 void launch_pci_pacc(hipStream_t st, const DevScene* T, const Chunk* C, int n, int iter, int fused) {
     if (!n) return;
-    if (n <= kQuadPaccChunks) LAUNCH_QUAD(k_pci_pacc<4>, n, st, T, C, n, iter, fused);
+    if (up_to(kQuadPaccChunks, n)) LAUNCH_QUAD(k_pci_pacc<4>, n, st, T, C, n, iter, fused);
     else LAUNCH(k_pci_pacc<1>, n, st, T, C, n, iter, fused);
 }
 void launch_pci_integrate(hipStream_t st, const DevScene* T, const Chunk* C, int n, int ahead) {
