@@ -14,6 +14,7 @@
 
 #include "sphg_internal.h"
 #include "sphg_kernels.h"
+#include "sphg_roots.h"
 
 #include <type_traits>
 
@@ -350,30 +351,6 @@ __device__ inline double rsqrt_d(double r2) {
     return (r2 > 1e-30) ? z : 0.0;
 }
 __device__ inline double sel(bool c, double a, double b) { return c ? a : b; }
-
-// sqrt(x) and a / b for arguments and results well inside the normal range: the
-// correctly rounded iterations (Markstein) without the scaling and the special
-// cases that the general forms add, 7 and 3 FP64 instructions a pair (PCISPH,
-// 351k particles with cohesion: 414 -> 407 us a step).  Equal to sqrt and / in
-// every bit for 1e9 random arguments of exponents -60 .. 60.  A zero x is taken
-// as 1e-290, whose root is as good as zero beside 1.
-__device__ inline double sqrt_n(double x) {
-    x = fmax(x, 1e-290);
-    const double y = __builtin_amdgcn_rsq(x);
-    double h = y * 0.5, s = x * y;
-    const double r = fma(-h, s, 0.5);
-    s = fma(s, r, s);
-    h = fma(h, r, h);
-    s = fma(fma(-s, s, x), h, s);
-    return fma(fma(-s, s, x), h, s);
-}
-__device__ inline double div_n(double a, double b) {
-    double r = __builtin_amdgcn_rcp(b);
-    r = fma(fma(-b, r, 1.0), r, r);
-    r = fma(fma(-b, r, 1.0), r, r);
-    const double q = a * r;
-    return fma(fma(-b, q, a), r, q);
-}
 
 struct Pair {
     double dx, dy, dz, r2, rl, inv, q;
