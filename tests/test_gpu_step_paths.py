@@ -426,3 +426,55 @@ def test_velocity_of_a_rejected_candidate(ctx, speed):
         out.append([s.get(f)[:-1] for f in (sphg.FIELD_ALPHA, sphg.FIELD_DIVERR)])
     assert out[0][1][face] > 0.0 and all(np.array_equal(a, c) for a, c in zip(*out))
     s.close()
+
+
+STALLS = {
+    # the loop that needs more iterations than were launched ahead; the other one stays at its minimum
+    "density": (sphg.DFSPH, dict(eta_v=1e9)),
+    "divergence": (sphg.DFSPH, dict(eta=1e3)),
+    "pressure": (sphg.PCISPH, {}),
+}
+
+
+@pytest.mark.parametrize("loop", sorted(STALLS))
+@pytest.mark.parametrize("where", ["small", "replayed", "large"])
+def test_lone_scene_that_needs_more_iterations_than_predicted(ctx, loop, where):
+    """At rest a loop takes a few iterations; with velocities that compress the
+    fluid it takes more, so that the steps launched ahead stop behind it and
+    the host adds iterations (the only waits that host_syncs counts once there
+    is a prediction): the same steps as in a batch."""
+    method, more = STALLS[loop]
+    if where == "large":
+        size = (129, 64, 64)
+        spec = configs.small_scene(method, n_side=size, spacing=0.02, box=tuple(0.02 * (s + 4) for s in size), **more)
+    else:
+        spec = configs.small_scene(method, n_side=(12, 9, 8), box=(0.9, 0.65, 0.6), **more)
+    other = configs.small_scene(method, n_side=5)
+    center = spec.fluid.mean(0)
+    speed = 300.0 * spec.params.particle_radius   # the same strain in both sizes
+    inward = ((center - spec.fluid) / np.abs(center - spec.fluid).max() * speed).astype(np.float32)
+    alone, mixed = [sphg.Scene(ctx, spec.params, spec.fluid, spec.boundary) for _ in range(2)]
+    extra = sphg.Scene(ctx, other.params, other.fluid, other.boundary)
+    ctx.set_graphs(where == "replayed")
+    try:
+        for steps in (1, 4):
+            alone.step(steps)
+        before = alone.scalars()
+        ctx.batch_step([mixed, extra], 5)
+        for s in (alone, mixed):
+            s.set_state(spec.fluid, inward)
+        stats = alone.step(4)
+        ctx.batch_step([mixed, extra], 4)
+    finally:
+        ctx.set_graphs(False)
+    after = alone.scalars()
+    assert stats.host_syncs > 0
+    if loop == "divergence":
+        assert after.sum_iterations_v - before.sum_iterations_v > 4 * spec.params.min_iterations_v
+        assert after.sum_iterations - before.sum_iterations == 4 * spec.params.min_iterations
+    else:
+        assert after.sum_iterations - before.sum_iterations > 4 * spec.params.min_iterations
+        assert after.sum_iterations_v - before.sum_iterations_v == (4 if method == sphg.DFSPH else 0)
+    assert scalars(alone) == scalars(mixed) and same(alone, mixed)
+    for s in (alone, mixed, extra):
+        s.close()
