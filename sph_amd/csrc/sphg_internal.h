@@ -95,6 +95,8 @@ struct Scalars {
     unsigned shellBad;          // PCISPH: this step's shell lists cannot stand in for the 27-cell walk
     unsigned maxD2Prev;         // PCISPH: largest squared predicted displacement (FP32 bits) of the
                                 // previous step, which sizes this step's shell
+    unsigned moved;             // PCISPH: an iteration of the step leaves the groups' displacements for it
+                                // (not `it`, which set_state writes)
     unsigned shellSteps, walkSteps;  // PCISPH: steps whose predicted densities used the shell lists /
                                      // took the 27-cell walk for every particle
     unsigned d0Valid;           // DFSPH: d0 holds the divergence of the current velocities (written by

@@ -744,7 +744,9 @@ __device__ inline void step_begin(const DevScene& S, const Chunk& c, int i, int*
     // the previous step's largest predicted displacement (none if no
     // iteration of it ran)
     double d2 = 0.0;
-    if (S.pciShell && ss->it > 0) {
+    const bool moved = S.pciShell && ss->moved;
+    __syncthreads();   // every thread has read the flag before it is set
+    if (moved) {
         __shared__ double sh[kWaves];
         float m = 0.f;
         const float* const disp = pci_displacements(S);
@@ -764,6 +766,7 @@ __device__ inline void step_begin(const DevScene& S, const Chunk& c, int i, int*
         if (S.method == PCISPH) {
             ss->it = 0;
             const bool run = (ss->maxDensErr > S.eta || 0 < S.minIt) && 0 < S.maxIt;
+            ss->moved = run ? 1u : 0u;
             ss->done = run ? 0 : 1;
             if (run) atomicAdd(active, 1);
         }

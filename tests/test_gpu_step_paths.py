@@ -478,3 +478,24 @@ def test_lone_scene_that_needs_more_iterations_than_predicted(ctx, loop, where):
     assert scalars(alone) == scalars(mixed) and same(alone, mixed)
     for s in (alone, mixed, extra):
         s.close()
+
+
+def test_shell_width_after_a_new_state(ctx):
+    """The shell of a PCISPH step is as wide as the previous step's predicted
+    displacements ask for, also where a new state (with its iteration count at
+    zero) came between: no step of a fluid at speed falls back to the walk
+    over 27 cells for it."""
+    spec = configs.small_scene(sphg.PCISPH, n_side=(9, 7, 8), box=(2.0, 0.55, 0.8))
+    v = np.zeros_like(spec.fluid)
+    v[:, 0] = 0.08 * spec.params.support_radius / spec.params.time_step
+    s = sphg.Scene(ctx, spec.params, spec.fluid, spec.boundary, v)
+    s.step(3)
+    before = s.scalars()
+    assert before.pcisph_walk_steps == 1 and before.pcisph_shell_steps == 2
+    s.set_state(spec.fluid, v)
+    s.step(1)
+    s.set_state(spec.fluid, v, last_iterations=3)
+    s.step(2)
+    after = s.scalars()
+    assert after.pcisph_walk_steps == 1 and after.pcisph_shell_steps == 5
+    s.close()
