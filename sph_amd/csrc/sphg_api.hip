@@ -771,8 +771,8 @@ int batch_one_step(sphg_ctx* ctx, Batch& B, uint32_t& syncs) {
 // asking after each, and goes on from there.  Which launches run does not
 // depend on any of that, so the results are those of waiting.
 //
-// Not for scenes whose step has more launches between the loops (cube clamp,
-// PCISPH boundary, emitters).
+// Not for scenes with a cube clamp, the PCISPH boundary method or emitters,
+// whose kernels do not look at the stall flag.
 bool lone_scene(const Batch& B) {
     if (B.scenes.size() != 1) return false;
     const DevScene& V = B.scenes[0]->view[0];

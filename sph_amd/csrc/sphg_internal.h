@@ -3,8 +3,9 @@
 //
 // One scene = one fluid model + one Akinci boundary model (the reference's
 // own constraint, src/Simulation.h:24-29 and src/AkinciBoundayModel.cpp:32).
-// Every kernel walks a chunk table: each 256-thread block owns one chunk of
-// one scene, so a launch covers any number of scenes of uneven size
+// Every kernel walks a chunk table: a block owns one chunk of 256 particles of
+// one scene, or a 64-particle group of it (small launches, 4 lanes a
+// particle), so a launch covers any number of scenes of uneven size
 // (batching).  A launch over one scene needs no table: its blocks' chunks
 // follow from their numbers.
 //
@@ -82,7 +83,7 @@ struct KCoefD {
 };
 
 // Device-resident control state of one scene (one writer at a time: the
-// last block of a reduction, or the first block of a scene).
+// scene's block of a finalize kernel, or the block of its first chunk).
 struct Scalars {
     double dt, time, maxVel, cflTs;
     double avgErr, avgErr0, avgErrV, avgErrV0, maxDensErr;

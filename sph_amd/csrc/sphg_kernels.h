@@ -54,8 +54,8 @@ void launch_rank_reorder(hipStream_t st, const DevScene* T, const Chunk* C, int 
 void launch_bvolume(hipStream_t st, const DevScene* T, int scene, int nb, float* tmp);
 void launch_build(hipStream_t st, int method, const DevScene* T, const Chunk* C, int nchunks, int fused = 0);
 void launch_normals(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks);
-// flags: the non-pressure forces (Flags) of every scene of the launch, or -1
-// where they differ
+// flags: the non-pressure forces (Flags, adhesion among them) of every scene of
+// the launch, or -1 where they differ
 void launch_forces(hipStream_t st, int method, int flags, const DevScene* T, const Chunk* C, int nchunks);
 void launch_dt(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks);
 void launch_df_predict(hipStream_t st, const DevScene* T, const Chunk* C, int nchunks, int fused);

@@ -1,11 +1,14 @@
 // sphg_kernels.hip -- gfx950 kernels of the SPH solver step.
 //
-// Every kernel takes a scene table and a chunk table; block b works on
-// chunk b (kBlock = 256 particles or kCellChunk = 1024 cells of one
-// scene).  Sums of a scene are formed in a fixed order: a butterfly inside
-// each wavefront, wave results combined in index order, one partial per
-// chunk, and then the partials added in chunk order by k_finalize (one
-// block per scene, launched after the sweep).  Results therefore do not
+// Every kernel takes a scene table and a chunk table; a block works on one
+// chunk (kBlock = 256 particles or kCellChunk = 1024 cells of one scene) or,
+// with 4 lanes a particle, on one 64-particle group of a chunk; which one
+// follows from the table, or without one from the block's number (chunk_at,
+// part_at).  Sums of a scene are formed in a fixed order: a butterfly inside
+// each wavefront, wave results combined in index order, one partial per chunk
+// or group, and then the partials added in chunk order, by k_finalize (one
+// block per scene, launched after the sweep) or, for a lone scene, by every
+// block of the next sweep (loop_over) or k_loop_end.  Results therefore do not
 // depend on scheduling.
 //
 // Reference algorithm: josemanuel28v/SPH src/SPHSolver.cpp,
@@ -248,7 +251,7 @@ __device__ inline double scene_partial_max(const double* partial, int n, double*
 // launches wrote (ended_before) and forms its own decision otherwise, so all
 // wavefronts of a block take the same branch, whenever they read the flag.
 
-// The decision after `it` iterations with error err; SUM: of an average.
+// The decision after `it` iterations with error err.
 template <int KIND>
 __device__ inline bool loop_goes_on(const DevScene& S, const Scalars* ss, int it, double err) {
     const double eta = KIND == LOOP_DIV ? S.etaV / ss->dt : S.eta;
@@ -1068,9 +1071,11 @@ __global__ __launch_bounds__(kBlock) void k_bvolume_pack(const DevScene* __restr
 // now 207, 123 and 91.  5 wavefronts a SIMD (96 registers) spill in DFSPH: +85.
 // Candidates staged by a block: 9 rows of its own particles and two cells on
 // each side.  With 256 particles 31.9 KB, which leaves room for 5 blocks a
-// compute unit.  A row is read 8 candidates at a time, so up to 7 entries past
-// its end.
-constexpr int kBuildStage = 9 * (kBlock + 38), kBuildPad = 7;
+// compute unit.  A row is read kScan candidates at a time, so up to kScan - 1
+// entries past its end.
+constexpr int kScan = 8;   // 32 a multiple of it: a row's tests fill a mask
+constexpr int kBuildStage = 9 * (kBlock + 38), kBuildPad = kScan - 1;
+static_assert(32 % kScan == 0, "whole masks");
 
 // FP64 test of a candidate: whether the reference's sums hold it, its W and
 // gradient factor, and whether its gradient is nonzero.
@@ -1313,10 +1318,10 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
     };
     auto vel = [&](uint32_t j) { return (M == DFSPH) ? ld3o(S.v, j) : make_float4(0.f, 0.f, 0.f, 0.f); };
     // Pass 1 over the 27 cells as 9 rows (walk27 order), up to 32 candidates
-    // of a row at a time: their tests go to the bits of a mask, 4 candidates'
-    // loads before the first test, and the survivors are then taken from it.
-    // Candidates past the row's end are read (staged rows: at most 3, inside
-    // the padded stage) and dropped with the mask's last bits.
+    // of a row at a time: their tests go to the bits of a mask, kScan
+    // candidates' loads before the first test, and the survivors are then taken
+    // from it.  Candidates past the row's end are read (staged rows: at most
+    // kScan - 1, inside the padded stage) and dropped with the mask's last bits.
     // fetch(j): position of candidate j; self: the row may hold particle i;
     // survivor j is kept as j + code
     auto scanRow = [&](int s0, int e0, bool self, int code, auto&& fetch) {
@@ -1324,12 +1329,12 @@ __global__ __launch_bounds__(kBlock) void k_build(const DevScene* __restrict__ T
             const int nv = min(e0 - c0, 32);
             uint32_t mo = 0, ms = 0;
             int k0 = 0;
-            for (; k0 < nv; k0 += 8) {
-                float3 p[8];
+            for (; k0 < nv; k0 += kScan) {
+                float3 p[kScan];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) p[u] = fetch(c0 + k0 + u);
+                for (int u = 0; u < kScan; ++u) p[u] = fetch(c0 + k0 + u);
 #pragma unroll
-                for (int u = 0; u < 8; ++u) {
+                for (int u = 0; u < kScan; ++u) {
                     const float fx = xi.x - p[u].x, fy = xi.y - p[u].y, fz = xi.z - p[u].z;
                     if (M == PCISPH) {
                         const float d2 = fx * fx + fy * fy + fz * fz;
@@ -2447,10 +2452,6 @@ __global__ __launch_bounds__(kPartBlock<Q>) void k_forces(const DevScene* __rest
         shell_guard(S, wx * dt, wy * dt, wz * dt);
     }
 }
-
-// WCSPH/PCISPH step-time bookkeeping: steps++ (one thread per scene) and,
-// for PCISPH, the entry test of the pressure loop (src/PCISPHSolver.cpp:365)
-// with p = pacc = 0 (:83-120).
 
 // ================================================================ DFSPH
 
