@@ -2652,11 +2652,12 @@ __global__ __launch_bounds__(kPartBlock<Q>) void k_df_vel(const DevScene* __rest
 // test.  MODE 0/1: predictDensities (src/DFSPHSolver.cpp:238-309),
 //   rho*_i = max(rho_i + dt (sum_j m (v_i - v_j).gradW_ij + v_i.gb_i), rho0),
 //   kappa_i = (rho*_i - rho0) alpha_i / (dt^2 rho_i)   (:346)
-// MODE 2/3: computeDivergenceError (:408-492),
+// MODE 3: computeDivergenceError (:408-492),
 //   e_i = sum_j m (v_i - v_j).gradW_ij + v_i.gb_i, 0 below 20 nonzero-gradient
 //   neighbors, else max(e_i, 0);  kappa_v_i = e_i alpha_i / (dt rho_i) (:531)
-// MODE 0/2 is the call before the loop: the loop's error starts at 0
-// (:326, :511); 1/3 is the call at the end of an iteration.  Loop test
+// MODE 0 is the call before the density loop, whose error starts at 0 (:326;
+// before the divergence loop, :511, the list build forms the error); 1 and 3
+// are the calls at the end of an iteration.  Loop test
 // (:327, :512; the divergence loop is bounded by maxIterations):
 //   continue while (err > eta (eta_V/dt) or it < minIt) and it < maxIt.
 template <int MODE, int Q>
